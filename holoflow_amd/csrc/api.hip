@@ -563,6 +563,7 @@ hfx_status hfx_moments_group(hfx_plan *const *plans, const uint16_t *const *ring
   mom.shift = (p0->d.flags & HFX_FLAG_FFTSHIFT) ? 1 : 0;
   auto set_windows = [&](hfx::PassArgs &a, bool mid) {
     a.nwin = n;
+    a.grouped = 1;
     for (int w = 0; w < n; ++w) {
       a.win[w].in = plans[w]->planes_blk;
       a.win[w].out = mid ? plans[w]->planes_blk : nullptr;

@@ -227,14 +227,14 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
   constexpr int E = F::E;
   constexpr int GB = row_group<W>();
   __shared__ float2 scr[GB * F::SCR];  // one padded row per plane of the current group
-  __shared__ float2 twl[F::TW];
+  __shared__ __align__(16) float2 twl[F::TW];
   extern __shared__ float4 wmat[];     // operand matrix of the MFMA loop
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   dft_stage_matrix<NBT, MODE>(wmat, a.wm_hi, a.wm_lo, a.r.T, tid, NT);
-  F::build_twiddles(twl, a.tw, tid, NT);
+  F::stage_twiddles(twl, a.tw, tid, NT);
   __syncthreads();
 
   const Band b = pinned_band(a);
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   constexpr int E = F::E;
   constexpr int GB = row_group<W>();
   __shared__ float2 scr[GB * F::SCR];  // one padded row per plane
-  __shared__ float2 twl[F::TW];
+  __shared__ __align__(16) float2 twl[F::TW];
   extern __shared__ float4 wmat[];     // operand matrix of the MFMA loop
 
   // one 16-bin tile (NBT == 2: up to 16 bins as 32 interleaved cos/-sin rows): the folded
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
                          tid, NT);
   else
     dft_stage_matrix<NBT, MODE>(wmat, a.wm_hi, a.wm_lo, a.r.T, tid, NT);
-  F::build_twiddles(twl, a.tw, tid, NT);
+  F::stage_twiddles(twl, a.tw, tid, NT);
   __syncthreads();
 
   const long long plane_elems = (long long)a.H * W;

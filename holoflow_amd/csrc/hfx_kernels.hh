@@ -66,7 +66,7 @@ bool dft_front_pipelined(int W, int nbc, int T, int n_planes, int precision);
 int launch_time_dft_row(const DftLaunch &L, int H, int blk_c, int n_planes, const float2 *tw,
                         hipStream_t st);
 
-// ---- 2-D FFT passes (fft2d.hip)
+// ---- 2-D FFT passes (wpass.hip)
 enum InMode { IN_NAT_C = 0, IN_NAT_R = 1, IN_BLK = 2 };
 enum OutMode { OUT_BLK = 0, OUT_NAT_C = 1, OUT_NAT_MAG = 2, OUT_MOMENTS = 3, OUT_NAT_RE = 4 };
 
@@ -106,9 +106,11 @@ struct PassArgs {
   int out_mode;
   const float2 *post_lx, *post_ly;  // lens applied to the output or null
   MomentArgs mom;
-  const float2 *tw;         // FFT twiddles for the transform length
-  const float2 *tw2;        // second twiddle table unused by single-axis passes
-  int nwin;                 // > 1: grouped launch, window blockIdx.z takes win[blockIdx.z]
+  const float2 *tw;         // pass-major FFT twiddles for the transform length
+  int nwin;                 // windows of the launch (blockIdx.z; 0 and 1: one)
+  // windows of one plan: byte strides of in and out, element stride of the moment images
+  long long win_in, win_out, win_mom;
+  int grouped;              // windows of several plans: window blockIdx.z takes win[blockIdx.z]
   PassWin win[HFX_MAX_WIN];
 };
 
@@ -117,10 +119,8 @@ int launch_col_pass(const PassArgs &a, hipStream_t st);
 bool row_pass_supported(int W);
 bool col_pass_supported(int H, int blk_c);
 int pick_blk_c(int W, int H);
-// wave-level FFT passes (wpass.hip) for lengths 256, 512, 768, 1024, 2048
+// lengths of one transform per wave (256, 512, 768, 1024, 2048): those that grouped launches take
 bool wave_pass_supported(int n);
-int launch_wave_row_pass(const PassArgs &a, hipStream_t st);
-int launch_wave_col_pass(const PassArgs &a, hipStream_t st);
 
 // ---- small ops (ops.hip)
 int launch_fftshift(const void *in, void *out, int elem_size, int ndim, const long long *shape,

@@ -2,19 +2,22 @@
 // the GPU and rounded once to FP32 (or FP16/BF16 hi/lo pairs for the MFMA operands),
 // because the propagation phases reach 1e6 rad where one FP32 ulp is ~0.1 rad.
 #include "hfx_kernels.hh"
+#include "wfft.hh"
 
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
 namespace hfx {
 
-// tw[m] = exp(-2*pi*i*m/N), m in [0, N).
+// Pass-major FFT twiddles exp(-2*pi*i*m/n) (fft_twiddle_index); entries past the passes' n - E
+// are 1 and unused.
 __global__ void k_fft_twiddles(float2 *tw, int n) {
-  int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n) return;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int m = fft_twiddle_index(n, i);
   double s, c;
   sincospi(2.0 * (double)m / (double)n, &s, &c);
-  tw[m] = make_float2((float)c, (float)(-s));
+  tw[i] = make_float2((float)c, (float)(-s));
 }
 
 void launch_fft_twiddles(float2 *tw, int n, hipStream_t st) {

@@ -1,8 +1,9 @@
-// Wave-level FFT engine: one 64-lane wavefront owns a whole transform of length
-// N = 64 * E (E in {4, 8, 12, 16, 32}), E elements per lane.
+// Wave-level FFT engine: L lanes of a 64-lane wavefront own a whole transform of length
+// N = L * E, E elements per lane.  L = 64 from 256 points on (one transform per wave); shorter
+// transforms share a wave, 64 / L side by side, each in its own scratch region.
 //
-// Convention: on entry lane l holds x[l + 64*m] in v[m]; on return it holds X[l + 64*m].
-// Consecutive lanes therefore read and write consecutive indices (coalesced global
+// Convention: on entry lane l of a transform holds x[l + L*m] in v[m]; on return it holds
+// X[l + L*m].  Consecutive lanes therefore read and write consecutive indices (coalesced global
 // access), and the data never leaves the wave:
 //
 //   pass 1 : radix-E DFT entirely in registers (butterfly j = lane, Stockham NS = 1)
@@ -10,15 +11,19 @@
 //            last pass leaving its results in registers in the natural layout.
 //
 // For N = 1024 this is radix 16 (registers) -> radix 16 -> radix 4: two LDS round trips
-// and no workgroup barrier, against five barrier-separated radix-4 LDS passes in a
-// workgroup-wide Stockham.  Within a wave, LDS instructions complete in issue order, so
+// and no workgroup barrier.  Within a wave, LDS instructions complete in issue order, so
 // a write followed by a read of another lane's element needs only a compiler barrier.
+//
+// Lanes per transform below 256 points: as few passes as registers allow (64 = 8 * 8,
+// 128 = 8 * 8 * 2, 96 = 12 * 4 * 2, 48 = 12 * 4, 32 = 8 * 4).  These sizes are bound by latency
+// (the chain of LDS round trips), not by bandwidth.
 //
 // The scratch is padded by one element per 16 (pad(i) = i + i/16; one per 32 at E = 32), which
 // makes the stride-E writes of pass 1 and the stride-NS accesses of the later passes free of
 // bank conflicts (at E = 32 the stride of 34 elements that one per 16 gives would put lanes l
-// and l + 16 on the same banks in pass 1; 33 spreads 32 lanes of 8-byte writes over all 64).  Pass twiddles come from an FP64-generated table tw[m] = exp(-2 pi i m/N);
-// the small in-register DFTs use the exact constants cos/sin(2 pi m/32) and (2 pi m/12).
+// and l + 16 on the same banks in pass 1; 33 spreads 32 lanes of 8-byte writes over all 64).
+// Pass twiddles come from an FP64-generated pass-major table (fft_twiddle_index); the small
+// in-register DFTs use the exact constants cos/sin(2 pi m/32) and (2 pi m/12).
 #pragma once
 
 #include "hfx_device.hh"
@@ -153,15 +158,39 @@ __host__ __device__ constexpr int wave_pass_radix(int rem, int E) {
   return r;
 }
 
+// Transform lengths of the passes, and the lanes that share one transform of length n.
+#define HFX_FFT_SIZES(X) \
+  X(2) X(4) X(8) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(256) X(512) X(768) X(1024) X(2048)
+__host__ __device__ constexpr int fft_lanes(int n) {
+  return n >= 256 ? 64 : n == 128 ? 16 : n == 96 || n == 64 ? 8 : n == 48 || n == 32 || n == 16 ? 4 : n == 24 || n == 8 ? 2 : 1;
+}
+
+// Pass-major twiddle table of an n-point transform: the pass with stride NS and radix R owns
+// (R-1)*NS entries W_{NS*R}^{r*k} at [r-1][k], so the lanes of a wave (consecutive k) read
+// consecutive entries; over all passes n - E entries.  Exponent m (of exp(-2 pi i m / n)) of
+// entry i.
+__host__ __device__ constexpr int fft_twiddle_index(int n, int i) {
+  const int E = n / fft_lanes(n);
+  for (int s = E; s < n;) {
+    const int r = wave_pass_radix(n / s, E), cnt = (r - 1) * s;
+    if (i < cnt) return (i / s + 1) * (i % s) * (n / (s * r));
+    i -= cnt;
+    s *= r;
+  }
+  return 0;
+}
+
 template <int N> struct WaveFft {
-  static_assert(N % 64 == 0, "wave FFT length must be a multiple of 64");
-  static constexpr int E = N / 64;
+  static constexpr int L = fft_lanes(N);
+  static constexpr int P = 64 / L;  // transforms per wave
+  static constexpr int E = N / L;
+  static_assert(N % L == 0, "lanes must divide the transform length");
   static constexpr int PSH = E >= 32 ? 5 : 4;  // one pad element per 2^PSH
-  static constexpr int SCR = N + (N >> PSH);    // padded scratch elements per transform
-  // Pass twiddles are stored pass-major: the pass with stride NS and radix R owns
-  // (R-1)*NS entries W_{NS*R}^{r*k} at [r-1][k], so the lanes of a wave (consecutive k)
-  // read consecutive entries.  Over all passes this is N - E entries.
-  static constexpr int TW = N - E;
+  // padded scratch elements per transform (side-by-side transforms are skewed by one more, which
+  // spreads them over the banks)
+  static constexpr int SCR = N + (N >> PSH) + (P > 1 ? 1 : 0);
+  static constexpr int TW = N - E;             // entries of the pass-major twiddle table
+  static constexpr int TWL = TW > 0 ? TW : 1;  // elements of its LDS copy
 
   __device__ __forceinline__ static int pad(int i) { return i + (i >> PSH); }
 
@@ -176,17 +205,11 @@ template <int N> struct WaveFft {
     return off;
   }
 
-  // Builds the pass-major table from an N-entry table t[m] = exp(-2 pi i m / N).
-  __device__ static void build_twiddles(float2 *dst, const float2 *t, int tid, int nthreads) {
-    for (int s = E; s < N;) {
-      const int r = wave_pass_radix(N / s, E);
-      const int off = tw_offset(s);
-      for (int i = tid; i < (r - 1) * s; i += nthreads) {
-        const int rr = i / s + 1, k = i % s;
-        dst[off + i] = t[rr * k * (N / (s * r))];
-      }
-      s *= r;
-    }
+  // Copies the pass-major table (16-byte aligned on both sides, TW even) into LDS.
+  __device__ __forceinline__ static void stage_twiddles(float2 *dst, const float2 *t, int tid, int nthreads) {
+    static_assert(TW % 2 == 0, "twiddles are copied in pairs");
+    for (int i = tid; i < TW / 2; i += nthreads)
+      reinterpret_cast<float4 *>(dst)[i] = reinterpret_cast<const float4 *>(t)[i];
   }
 
   template <int NS, int S>
@@ -194,7 +217,7 @@ template <int N> struct WaveFft {
     constexpr int R = wave_pass_radix(N / NS, E);
     static_assert(R >= 2, "bad factorisation");
     constexpr int NB = N / R;
-    constexpr int PER = NB / 64;  // butterflies per lane
+    constexpr int PER = NB / L;  // butterflies per lane
     constexpr bool LAST = NS * R == N;
     constexpr int TOFF = tw_offset(NS);
     float2 u[PER][R];
@@ -202,14 +225,14 @@ template <int N> struct WaveFft {
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
-      for (int r = 0; r < R; ++r) u[q][r] = scr[pad(lane + 64 * q + r * NB)];
+      for (int r = 0; r < R; ++r) u[q][r] = scr[pad(lane + L * q + r * NB)];
     // all twiddle reads issued together with the data reads, so their latencies overlap
     // instead of one LDS round trip per pair; the empty asm keeps the compiler from sinking
     // each read down to its use
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
-      for (int r = 1; r < R; ++r) w[q][r] = tw[TOFF + (r - 1) * NS + (lane + 64 * q) % NS];
+      for (int r = 1; r < R; ++r) w[q][r] = tw[TOFF + (r - 1) * NS + (lane + L * q) % NS];
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
@@ -224,7 +247,7 @@ template <int N> struct WaveFft {
       RegDft<R, S>::run(u[q]);
     }
     if constexpr (LAST) {
-      // outputs j + r*NS with NS = N/R: lane holds X[lane + 64*(q + r*E/R)]
+      // outputs j + r*NS with NS = N/R: lane holds X[lane + L*(q + r*E/R)]
 #pragma unroll
       for (int q = 0; q < PER; ++q)
 #pragma unroll
@@ -232,7 +255,7 @@ template <int N> struct WaveFft {
     } else {
 #pragma unroll
       for (int q = 0; q < PER; ++q) {
-        const int j = lane + 64 * q;
+        const int j = lane + L * q;
         const int base = (j / NS) * NS * R + j % NS;
 #pragma unroll
         for (int r = 0; r < R; ++r) scr[pad(base + r * NS)] = u[q][r];
@@ -242,8 +265,9 @@ template <int N> struct WaveFft {
     }
   }
 
-  // Transforms v in place (see the convention above); scr: SCR wave-private LDS elements;
-  // tw: the TW-entry pass-major table from build_twiddles; inv: kernel exp(+...), unscaled.
+  // Transforms v in place (see the convention above); scr: the transform's SCR wave-private LDS
+  // elements; tw: the pass-major table in LDS; lane: 0 .. L-1 within the transform; INV: kernel
+  // exp(+...), unscaled.
   template <bool INV>
   __device__ __forceinline__ static void run(float2 (&v)[E], float2 *scr, const float2 *tw, int lane) {
     stage_in<INV>(v, scr, lane);
@@ -254,22 +278,19 @@ template <int N> struct WaveFft {
   // stage_out runs the remaining passes and leaves X in o.
   template <bool INV> __device__ __forceinline__ static void stage_in(float2 (&v)[E], float2 *scr, int lane) {
     constexpr int S = INV ? 1 : -1;
-    RegDft<E, S>::run(v);  // pass 1: butterfly j = lane over x[lane + 64 r]
+    RegDft<E, S>::run(v);  // pass 1: butterfly j = lane over x[lane + L r]
 #pragma unroll
     for (int r = 0; r < E; ++r) scr[pad(lane * E + r)] = v[r];
     __builtin_amdgcn_wave_barrier();
   }
   template <bool INV>
   __device__ __forceinline__ static void stage_out(float2 (&o)[E], float2 *scr, const float2 *tw, int lane) {
-    pass<E, INV ? 1 : -1>(o, scr, tw, lane);
-  }
-  // run-time direction (a wave-uniform branch between the two instantiations)
-  __device__ __forceinline__ static void run(float2 (&v)[E], float2 *scr, const float2 *tw, int lane,
-                                             bool inv) {
-    if (inv)
-      run<true>(v, scr, tw, lane);
-    else
-      run<false>(v, scr, tw, lane);
+    if constexpr (N == E) {  // one lane holds the whole transform: pass 1 was all of it
+#pragma unroll
+      for (int r = 0; r < E; ++r) o[r] = scr[pad(r)];
+    } else {
+      pass<E, INV ? 1 : -1>(o, scr, tw, lane);
+    }
   }
 };
 
