@@ -112,7 +112,7 @@ struct hfx_plan {
   float2 *lx = nullptr, *ly = nullptr;
   float2 *tf = nullptr;
   float *wf = nullptr, *wf2 = nullptr;
-  int nwin = 1;              // windows per front launch in hfx_moments_batch
+  int nwin = 1;              // windows per launch in hfx_moments_batch
   int lanes = 1;             // streams hfx_moments_batch alternates over (1 or 2)
   hipStream_t aux = nullptr; // second lane's stream (default priority, non-blocking)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -164,9 +164,8 @@ hfx_plan::~hfx_plan() {
 
 static hfx_status spectral_setup(SpectralFilter &f, int64_t batch, int H, int W, hipStream_t st,
                                  float2 *borrowed_ws = nullptr);
-static hfx_status spectral_run(const SpectralFilter &f, const void *in, bool in_real, void *out, bool out_real,
-                               hipStream_t st);
-static hfx_status window_back_moments(hfx_plan *p, float2 *planes, float *out, hipStream_t st);
+static hfx_status spectral_run(const SpectralFilter &f, int planes, const void *in, bool in_real, void *out,
+                               bool out_real, hipStream_t st);
 
 extern "C" {
 
@@ -192,6 +191,13 @@ void hfx_plan_desc_init(hfx_plan_desc *d) {
   d->weight_fs_hz = 37e3;
 }
 
+// Planes of the windows that hfx_moments_batch puts into one launch, per lane.  A lone small window
+// leaves most of the chip idle and pays every kernel's fill and drain (32 windows of 128 x 128,
+// T = 32, ASM: 444 us one by one, 52 us together).  Measured with 16 / 32 / 64 / 128 MiB: 16 windows
+// of 512 x 512, T = 32: 467 / 349 / 314 / 299 us; 12 of 256 x 1024, T = 64: 422 / 420 / 344 / 331;
+// 64 takes most of it with half the memory, and two lanes of it fit the last-level cache.
+constexpr long long kBatchPlaneBytes = 64LL << 20;
+
 static hfx_status gen_prop_tables(hfx_plan *p, hipStream_t st) {
   const hfx_plan_desc &d = p->d;
   if (d.prop == HFX_PROP_FRESNEL) {
@@ -205,7 +211,7 @@ static hfx_status gen_prop_tables(hfx_plan *p, hipStream_t st) {
   return HFX_OK;
 }
 
-hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_plan **out) {
+static hfx_status plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_plan **out, bool one_window) {
   if (!dp || !out) return fail(HFX_E_INVALID, "null argument");
   *out = nullptr;
   const hfx_plan_desc &d = *dp;
@@ -274,20 +280,27 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
   p->fused_row = !p->filter2d && p->OH == p->H && p->OW == p->W && hfx::dft_row_supported(p->W, p->nbc, d.window);
   if (d.batch_windows > 1 && p->fused_row &&
       hfx::dft_front_pipelined(p->W, p->nbc, d.window, p->n_planes, d.precision))
-    p->nwin = std::min<int>(d.batch_windows, hfx::HFX_MAX_WIN);
+    p->nwin = std::min<int>(d.batch_windows, 4);
+  // Windows per launch the library chooses: as many as keep the group's planes within
+  // kBatchPlaneBytes.
+  const long long window_bytes = (long long)p->n_planes * std::max(p->npix, p->onpix) * (long long)sizeof(float2);
+  if (one_window)
+    p->nwin = 1;
+  else
+    p->nwin = std::max(p->nwin, (int)std::min<long long>(kBatchPlaneBytes / window_bytes, hfx::HFX_MAX_WIN));
   // batch lanes: a second stream (and plane workspaces) lets one window's kernels overlap the
   // neighbouring window's (measured +15 % at 1024^2, T = 64, in FP32 and the 16-bit modes);
   // the Flatfield's scratch images and Filter2D's tables are shared, so those keep one lane.
   if (d.batch_lanes < 0 || d.batch_lanes > 2) return fail(HFX_E_INVALID, "batch_lanes must be 0, 1 or 2");
-  p->lanes = d.batch_lanes != 1 && !p->filter2d && !d.flatfield_enabled ? 2 : 1;
-  // natural-layout planes, one set per lane: only the stand-alone time DFT needs them
-  HFX_TRY(A.alloc(&p->planes_nat, p->fused_row ? 1 : (size_t)p->lanes * p->n_planes * p->npix));
+  p->lanes = d.batch_lanes != 1 && !one_window && !p->filter2d && !d.flatfield_enabled ? 2 : 1;
+  // natural-layout planes per window of a launch and lane: only the stand-alone time DFT needs them
+  HFX_TRY(A.alloc(&p->planes_nat, p->fused_row ? 1 : (size_t)p->lanes * p->nwin * p->n_planes * p->npix));
   if (p->lanes == 2) {
     HFX_TRY_HIP(hipStreamCreateWithFlags(&p->aux, hipStreamNonBlocking));
     HFX_TRY_HIP(hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming));
     HFX_TRY_HIP(hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming));
   }
-  // one blocked plane workspace per window of a front launch, per lane
+  // one blocked plane workspace per window of a launch, per lane
   HFX_TRY(A.alloc(&p->planes_blk, (size_t)p->lanes * p->nwin * p->n_planes * p->onpix));
   HFX_TRY(A.alloc(&p->tw_w, p->OW));
   HFX_TRY(A.alloc(&p->tw_h, p->OH));
@@ -315,7 +328,7 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
                                (int)d.s_outer, 1, p->f2d.blk_c, st);
   }
   if (d.flatfield_enabled) {
-    HFX_TRY(A.alloc(&p->mom_tmp, (size_t)p->n_out * p->onpix));
+    HFX_TRY(A.alloc(&p->mom_tmp, (size_t)p->nwin * p->n_out * p->onpix));
     HFX_TRY(hfx_flatfield_create(p->n_out, p->OH, p->OW, d.flatfield_sigma_y, d.flatfield_sigma_x, stream, &p->ff,
                                  nullptr));
   }
@@ -328,6 +341,18 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
   *out = guard.release();
   return HFX_OK;
 }
+
+hfx_status hfx_plan_create(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out) {
+  return plan_create(d, stream, out, false);
+}
+
+}  // extern "C"
+namespace hfx {
+hfx_status plan_create_one_window(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out) {
+  return plan_create(d, stream, out, true);
+}
+}  // namespace hfx
+extern "C" {
 
 hfx_status hfx_plan_destroy(hfx_plan *p) {
   delete p;
@@ -419,26 +444,43 @@ static hfx::PassArgs base_pass(int H, int W, int planes, int blk_c) {
   return a;
 }
 
-// Front of the schedule: the window's band planes, row-transformed, in the plan's blocked
-// workspace (one fused kernel when the frame width allows, else time DFT + row pass).
-// planes: the blocked workspace (default the plan's first); lane: the natural-layout planes'
-// set of the stand-alone time DFT
-static hfx_status window_front(hfx_plan *p, const uint16_t *ring, int64_t ring_frames, int64_t first,
-                               hipStream_t st, float2 *planes = nullptr, int lane = 0) {
-  if (!planes) planes = p->planes_blk;
+// A run of consecutive windows of one plan's stream, computed together.
+struct Windows {
+  const uint16_t *ring;
+  int64_t ring_frames, first;  // first frame of window 0, in [0, ring_frames)
+  int64_t step = 0;            // frames from one window to the next
+  int n = 1;                   // windows, at most the plan's nwin
+  float *out = nullptr;
+  int64_t out_stride = 0;      // floats from one window's images to the next
+  int lane = 0;                // which of the plan's plane workspaces
+};
+
+static float2 *blocked_planes(const hfx_plan *p, int lane) {
+  return p->planes_blk + (long long)lane * p->nwin * p->n_planes * p->onpix;
+}
+
+// Front of the schedule: the windows' band planes, row-transformed, in the plan's blocked
+// workspace (one fused kernel when the frame width allows, else time DFT + row pass).  Planes of
+// consecutive windows are consecutive.
+static hfx_status windows_front(hfx_plan *p, const Windows &ws, hipStream_t st) {
+  float2 *planes = blocked_planes(p, ws.lane);
+  float2 *nat = p->planes_nat + (long long)ws.lane * p->nwin * p->n_planes * p->npix;
+  hfx::DftLaunch L = dft_launch(p, ws.ring, ws.ring_frames, ws.first, p->fused_row ? planes : nat);
+  L.nwin = ws.n;
+  for (int w = 0; w < ws.n; ++w) L.firsts[w] = (ws.first + w * ws.step) % ws.ring_frames;
+  L.planes_stride = (long long)p->n_planes * (p->fused_row ? p->onpix : p->npix);
   if (p->fused_row) {
-    hfx::DftLaunch L = dft_launch(p, ring, ring_frames, first, planes);
     if (hfx::launch_time_dft_row(L, p->OH, p->blk_c, p->n_planes, p->tw_w, st) != 0)
       return fail(HFX_E_HIP, "fused time-DFT/row-FFT launch failed");
     return HFX_OK;
   }
-  float2 *nat = p->planes_nat + (long long)lane * p->n_planes * p->npix;
-  HFX_TRY(run_dft(p, ring, ring_frames, first, nat, st));
+  const int rc = hfx::launch_time_dft(L, st);
+  if (rc != 0) return fail(HFX_E_HIP, "time DFT launch failed (" + std::to_string(rc) + ")");
   // Filter2D in place on the natural planes, through the blocked workspace (one lane)
-  if (p->filter2d) HFX_TRY(spectral_run(p->f2d, nat, false, nat, false, st));
+  if (p->filter2d) HFX_TRY(spectral_run(p->f2d, ws.n * p->n_planes, nat, false, nat, false, st));
   // row pass: natural planes (lens already applied for Fresnel, or here after Filter2D)
   // -> blocked spectrum rows
-  hfx::PassArgs r = base_pass(p->OH, p->OW, p->n_planes, p->blk_c);
+  hfx::PassArgs r = base_pass(p->OH, p->OW, ws.n * p->n_planes, p->blk_c);
   if (p->filter2d) {
     r.pre_lx = p->lx;
     r.pre_ly = p->ly;
@@ -457,32 +499,37 @@ static hfx_status window_front(hfx_plan *p, const uint16_t *ring, int64_t ring_f
 }
 
 // Back of the schedule: column pass (Fresnel: with |.| and the moment reduction; ASM: with
-// the transfer function, then the inverse row pass with the reduction) into `out`.
-static hfx_status window_back(hfx_plan *p, float *out, hipStream_t st, float2 *planes = nullptr) {
-  HFX_TRY(window_back_moments(p, planes ? planes : p->planes_blk, p->ff ? p->mom_tmp : out, st));
-  if (p->ff) return hfx_flatfield_execute(p->ff, p->mom_tmp, out, reinterpret_cast<hfx_stream_t>(st));
-  return HFX_OK;
-}
-
-static hfx_status window_back_moments(hfx_plan *p, float2 *planes, float *out, hipStream_t st) {
+// the transfer function, then the inverse row pass with the reduction) into the windows' images.
+static hfx_status windows_back(hfx_plan *p, const Windows &ws, hipStream_t st) {
   const long long on = p->onpix;
+  float2 *planes = blocked_planes(p, ws.lane);
+  // Flatfield reads the images from scratch, one window's after the other's
+  float *mom_out = p->ff ? p->mom_tmp : ws.out;
   hfx::MomentArgs mom{};
-  for (int i = 0; i < p->n_out; ++i) mom.out[i] = out + i * on;
+  for (int i = 0; i < p->n_out; ++i) mom.out[i] = mom_out + i * on;
   mom.f = p->wf;
   mom.f2 = p->wf2;
   mom.split = p->d.split_bin > 0 ? p->d.split_bin - p->d.bin_begin : 0;
   mom.power2 = (p->d.flags & HFX_FLAG_POWER2) ? 1 : 0;
   mom.shift = (p->d.flags & HFX_FLAG_FFTSHIFT) ? 1 : 0;
+  // the moment passes take the window as a grid dimension
+  auto moments = [&](hfx::PassArgs &a) {
+    a.out_mode = hfx::OUT_MOMENTS;
+    a.mom = mom;
+    a.nwin = ws.n;
+    a.win_in = (long long)p->n_planes * on * (long long)sizeof(float2);
+    a.win_mom = p->ff ? p->n_out * on : ws.out_stride;
+  };
 
   hfx::PassArgs c = base_pass(p->OH, p->OW, p->n_planes, p->blk_c);
   c.in = planes;
   c.in_mode = hfx::IN_BLK;
   c.tw = p->tw_h;
   if (p->d.prop == HFX_PROP_FRESNEL) {
-    c.out_mode = hfx::OUT_MOMENTS;
-    c.mom = mom;
+    moments(c);
     if (hfx::launch_col_pass(c, st) != 0) return fail(HFX_E_HIP, "column pass launch failed");
   } else {
+    c.planes = ws.n * p->n_planes;
     c.mid_tf = p->tf;
     c.out = planes;
     c.out_mode = hfx::OUT_BLK;
@@ -491,18 +538,23 @@ static hfx_status window_back_moments(hfx_plan *p, float2 *planes, float *out, h
     r2.in = planes;
     r2.in_mode = hfx::IN_BLK;
     r2.inv = 1;
-    r2.out_mode = hfx::OUT_MOMENTS;
-    r2.mom = mom;
     r2.tw = p->tw_w;
+    moments(r2);
     if (hfx::launch_row_pass(r2, st) != 0) return fail(HFX_E_HIP, "inverse row pass launch failed");
   }
+  if (p->ff)
+    for (int w = 0; w < ws.n; ++w)
+      HFX_TRY(hfx_flatfield_execute(p->ff, p->mom_tmp + w * p->n_out * on, ws.out + w * ws.out_stride,
+                                    reinterpret_cast<hfx_stream_t>(st)));
   return HFX_OK;
 }
 
 static hfx_status window_moments(hfx_plan *p, const uint16_t *ring, int64_t ring_frames,
                                  int64_t first, float *out, hipStream_t st) {
-  HFX_TRY(window_front(p, ring, ring_frames, first, st));
-  return window_back(p, out, st);
+  Windows ws{ring, ring_frames, first};
+  ws.out = out;
+  HFX_TRY(windows_front(p, ws, st));
+  return windows_back(p, ws, st);
 }
 
 // A group of plans whose windows can share one front launch and one launch per back pass:
@@ -521,7 +573,7 @@ static bool group_compatible(const hfx_plan *a, const hfx_plan *b) {
 hfx_status hfx_moments_group(hfx_plan *const *plans, const uint16_t *const *rings, const int64_t *ring_frames,
                              const int64_t *first_frames, float *const *outs, int32_t n, hfx_stream_t stream) {
   if (!plans || !rings || !ring_frames || !first_frames || !outs) return fail(HFX_E_INVALID, "null argument");
-  static_assert(HFX_GROUP_MAX <= hfx::HFX_MAX_WIN, "grouped launches carry at most HFX_MAX_WIN windows");
+  static_assert(HFX_GROUP_MAX <= hfx::HFX_MAX_GROUP, "grouped launches carry at most HFX_MAX_GROUP windows");
   if (n < 1 || n > HFX_GROUP_MAX)
     return fail(HFX_E_INVALID, "a group holds 1 to " + std::to_string(HFX_GROUP_MAX) + " windows");
   hfx_plan *p0 = plans[0];
@@ -605,11 +657,13 @@ hfx_status hfx_plan_run_stage(hfx_plan *p, int32_t stage, const uint16_t *ring, 
   if (!p) return fail(HFX_E_INVALID, "null plan");
   if (stage == 0) {
     HFX_TRY(check_ring(p, ring, ring_frames, first_frame));
-    return window_front(p, ring, ring_frames, first_frame, S(stream));
+    return windows_front(p, Windows{ring, ring_frames, first_frame}, S(stream));
   }
   if (stage == 1) {
     if (!out) return fail(HFX_E_INVALID, "null output");
-    return window_back(p, out, S(stream));
+    Windows ws{};
+    ws.out = out;
+    return windows_back(p, ws, S(stream));
   }
   return fail(HFX_E_INVALID, "stage must be 0 (front) or 1 (back)");
 }
@@ -628,38 +682,27 @@ hfx_status hfx_moments_batch(hfx_plan *p, const uint16_t *ring, int64_t ring_fra
   if (!out || n_windows < 0) return fail(HFX_E_INVALID, "invalid output");
   if (out_stride < (int64_t)p->n_out * p->onpix) return fail(HFX_E_INVALID, "out_stride too small");
   hipStream_t st = S(stream);
-  auto frame_of = [&](int w) { return (first_frame + (int64_t)w * p->d.stride) % ring_frames; };
-  const long long pstride = (long long)p->n_planes * p->onpix;  // one window's planes
-  // groups of nwin windows (one front launch each) alternate over the lanes; lane 1 runs on
-  // the plan's own stream, forked from and joined back into the caller's stream
-  const bool two = p->lanes == 2 && n_windows > p->nwin;
+  // groups of up to nwin windows (one launch per kernel each) alternate over the lanes; lane 1
+  // runs on the plan's own stream, forked from and joined back into the caller's stream.  The
+  // windows are spread evenly over the groups.
+  const int groups = (int)(((int64_t)n_windows + p->nwin - 1) / p->nwin);
+  const bool two = p->lanes == 2 && groups > 1;
   if (two) {
     HFX_TRY_HIP(hipEventRecord(p->ev_fork, st));
     HFX_TRY_HIP(hipStreamWaitEvent(p->aux, p->ev_fork, 0));
   }
   hfx_status rc = HFX_OK;
-  int g = 0;
-  for (int w = 0; w < n_windows && rc == HFX_OK; w += p->nwin, ++g) {
-    const int lane = two ? (g & 1) : 0;
-    hipStream_t ls = lane ? p->aux : st;
-    float2 *ws = p->planes_blk + (long long)lane * p->nwin * pstride;
-    if (p->nwin > 1) {
-      // nwin windows per front launch (the pipelined kernel runs on across their rows), then
-      // the back of each window from its own plane workspace
-      const int k = std::min(p->nwin, n_windows - w);
-      hfx::DftLaunch L = dft_launch(p, ring, ring_frames, frame_of(w), ws);
-      L.nwin = k;
-      for (int j = 0; j < k; ++j) L.firsts[j] = frame_of(w + j);
-      L.planes_stride = pstride;
-      if (hfx::launch_time_dft_row(L, p->OH, p->blk_c, p->n_planes, p->tw_w, ls) != 0) {
-        rc = fail(HFX_E_HIP, "multi-window front launch failed");
-        break;
-      }
-      for (int j = 0; j < k && rc == HFX_OK; ++j) rc = window_back(p, out + (w + j) * out_stride, ls, ws + j * pstride);
-    } else {
-      rc = window_front(p, ring, ring_frames, frame_of(w), ls, ws, lane);
-      if (rc == HFX_OK) rc = window_back(p, out + w * out_stride, ls, ws);
-    }
+  for (int g = 0; g < groups && rc == HFX_OK; ++g) {
+    const int w0 = (int)((int64_t)n_windows * g / groups), w1 = (int)((int64_t)n_windows * (g + 1) / groups);
+    Windows ws{ring, ring_frames, (first_frame + (int64_t)w0 * p->d.stride) % ring_frames};
+    ws.step = p->d.stride;
+    ws.n = w1 - w0;
+    ws.out = out + w0 * out_stride;
+    ws.out_stride = out_stride;
+    ws.lane = two ? (g & 1) : 0;
+    hipStream_t ls = ws.lane ? p->aux : st;
+    rc = windows_front(p, ws, ls);
+    if (rc == HFX_OK) rc = windows_back(p, ws, ls);
   }
   if (two) {  // join even after a failed launch, so the caller's stream orders after lane 1
     const hipError_t e1 = hipEventRecord(p->ev_join, p->aux);
@@ -870,9 +913,9 @@ static hfx_status spectral_setup(SpectralFilter &f, int64_t batch, int H, int W,
   return HFX_OK;
 }
 
-static hfx_status spectral_run(const SpectralFilter &f, const void *in, bool in_real, void *out, bool out_real,
-                               hipStream_t st) {
-  const int B = (int)f.batch;
+static hfx_status spectral_run(const SpectralFilter &f, int planes, const void *in, bool in_real, void *out,
+                               bool out_real, hipStream_t st) {
+  const int B = planes;
   hfx::PassArgs r = base_pass(f.H, f.W, B, f.blk_c);
   r.in = in;
   r.in_mode = in_real ? hfx::IN_NAT_R : hfx::IN_NAT_C;
@@ -946,7 +989,7 @@ hfx_status hfx_filter2d_create(int64_t batch, int32_t height, int32_t width, int
 
 hfx_status hfx_filter2d_execute(hfx_filter2d *f, const void *in, void *out, hfx_stream_t stream) {
   if (!f || !in || !out) return fail(HFX_E_INVALID, "null argument");
-  return spectral_run(f->sf, in, f->in_real != 0, out, f->in_real != 0, S(stream));
+  return spectral_run(f->sf, (int)f->sf.batch, in, f->in_real != 0, out, f->in_real != 0, S(stream));
 }
 
 hfx_status hfx_filter2d_destroy(hfx_filter2d *f) {
@@ -999,7 +1042,7 @@ hfx_status hfx_flatfield_execute(hfx_flatfield *f, const float *in, float *out, 
   if (!f || !in || !out) return fail(HFX_E_INVALID, "null argument");
   if (in == out) return fail(HFX_E_INVALID, "flatfield output must not alias its input");
   hipStream_t st = S(stream);
-  if (f->use_fft) return spectral_run(f->sf, in, true, out, true, st);
+  if (f->use_fft) return spectral_run(f->sf, (int)f->sf.batch, in, true, out, true, st);
   if (hfx::launch_flatfield_spatial(in, out, f->tmp, f->batch, f->H, f->W, f->kx, f->rx, f->ky, f->ry, st) != 0)
     return fail(HFX_E_HIP, "flatfield launch failed");
   return HFX_OK;

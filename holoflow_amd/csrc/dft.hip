@@ -31,14 +31,14 @@ struct DftArgs {
   DftRing r;
   int W;
   int kb, nb, nbc, both;
-  float2 *planes;          // k_dft: natural [planes][npix]; k_dft_row: blocked
-  const float2 *lx, *ly;   // Fresnel lens vectors or null
+  const float2 *lx, *ly;   // k_dft, k_dft_row: Fresnel lens vectors or null
   const void *wm_hi, *wm_lo;
-  // k_dft_row only
+  // fused kernels only
   int H, blk_c, n_planes;
   const float2 *tw;        // W-point FFT twiddles
-  // k_front only: the windows of one launch (one plan's consecutive windows, or one window
-  // each of a group of plans of one shape): ring, ring length, first frame, planes, lens
+  // the windows of one launch (one plan's consecutive windows, or for k_front one window each of
+  // a group of plans of one shape): ring, ring length, first frame, planes (k_dft: natural
+  // [planes][npix]; the fused kernels: blocked), lens
   int nwin;
   long long firsts[HFX_MAX_WIN];
   const uint16_t *rings[HFX_MAX_WIN];
@@ -83,7 +83,7 @@ __device__ __forceinline__ void dft_bin_values(const Band &b, const f4 (&acc)[4]
 // ----------------------------------------------------------------------- stand-alone
 // Band bin `bin` of the 4 pixels from p0 into its natural-layout plane (and the conjugate
 // plane of the two-sided path), times the lens when there is one.
-__device__ __forceinline__ void dft_store_bin(const DftArgs &a, const Band &b, long long p0, int bin,
+__device__ __forceinline__ void dft_store_bin(float2 *planes, long long npix, const Band &b, long long p0, int bin,
                                               const float2 (&v)[4], const float2 (&L)[4], bool lens) {
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
@@ -103,33 +103,46 @@ __device__ __forceinline__ void dft_store_bin(const DftArgs &a, const Band &b, l
       float2 c = side ? make_float2(v[t].x, -v[t].y) : v[t];
       o[t] = lens ? cmul(c, L[t]) : c;
     }
-    float4 *dst = reinterpret_cast<float4 *>(a.planes + (long long)q * a.r.npix + p0);
+    float4 *dst = reinterpret_cast<float4 *>(planes + (long long)q * npix + p0);
     dst[0] = make_float4(o[0].x, o[0].y, o[1].x, o[1].y);
     dst[1] = make_float4(o[2].x, o[2].y, o[3].x, o[3].y);
   }
 }
 
+// Ring of window w of the launch (windows of one plan share it up to the first frame).
+__device__ __forceinline__ DftRing window_ring(const DftArgs &a, int w) {
+  DftRing r = a.r;
+  r.ring = a.rings[w];
+  r.ring_frames = a.ring_frames_w[w];
+  r.first = a.firsts[w];
+  return r;
+}
+
 // Persistent: a block stages the operand matrix once (tens of KB, and index arithmetic per
-// element) and then walks groups of four 64-pixel tiles blockIdx, blockIdx + grid, ...
+// element) and then walks groups of four 64-pixel tiles blockIdx, blockIdx + grid, ... of all
+// windows of the launch, window-major.
 template <int NBT, int MODE>
 __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
   extern __shared__ float4 lds_dyn[];
   dft_stage_matrix<NBT, MODE>(lds_dyn, a.wm_hi, a.wm_lo, a.r.T, threadIdx.x, 256);
   __syncthreads();
   const Band b = pinned_band(a);
-  const long long tiles = (a.r.npix + 63) / 64;
+  const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
   const bool lens = a.lx != nullptr;
-  for (long long t0 = (long long)blockIdx.x * 4; t0 < tiles; t0 += (long long)gridDim.x * 4) {
+  for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
+    const unsigned w = it / quads;
+    const DftRing r = window_ring(a, w);
+    float2 *planes = a.planes_w[w];
     // an opaque per-tile copy of the lane index keeps the lane-derived LDS and load addresses of
     // the MFMA loop from being hoisted out of the tile loop (where they would hold registers)
     int lane;
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(threadIdx.x & 63));
     // tiles past the end load clamped pixels (dft_px) and store nothing
-    const long long p0w = (t0 + (threadIdx.x >> 6)) * 64;
+    const long long p0w = ((long long)(it - w * quads) * 4 + (threadIdx.x >> 6)) * 64;
     uint2 pre[1][dft_pre_steps<MODE>()];
-    dft_prefetch<MODE, 1>(a.r, p0w, lane, pre);
+    dft_prefetch<MODE, 1>(r, p0w, lane, pre);
     f4 acc1[1][NBT][4];
-    dft_tile<NBT, MODE, 1>(a.r, lds_dyn, p0w, lane, pre, acc1);
+    dft_tile<NBT, MODE, 1>(r, lds_dyn, p0w, lane, pre, acc1);
     auto &acc = acc1[0];
 
     const long long p0 = p0w + 4 * (lane & 15);
@@ -149,7 +162,7 @@ __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
         if (bin >= b.nbc) continue;
         float2 v[4];
         dft_bin_values(b, acc[bt], h, bin, v);
-        dft_store_bin(a, b, p0, bin, v, L, lens);
+        dft_store_bin(planes, a.r.npix, b, p0, bin, v, L, lens);
       }
     }
   }
@@ -171,15 +184,18 @@ __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs 
   __syncthreads();
   const Band b = pinned_band(a);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long long tiles = (a.r.npix + 63) / 64;
+  const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
   const bool lens = a.lx != nullptr;
-  for (long long t0 = (long long)blockIdx.x * 4; t0 < tiles; t0 += (long long)gridDim.x * 4) {
+  for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
+    const unsigned w = it / quads;
+    const DftRing r = window_ring(a, w);
+    float2 *planes = a.planes_w[w];
     int lane;  // opaque per tile, as in k_dft
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(threadIdx.x & 63));
     // tiles past the end load clamped pixels (dft_px) and store nothing
-    const long long p0w = (t0 + wave) * 64;
+    const long long p0w = ((long long)(it - w * quads) * 4 + wave) * 64;
     f4 ac[NBF][4], as[NBF][4];
-    dft_fold_tile<NBF>(a.r, lf, p0w, lane, ac, as);
+    dft_fold_tile<NBF>(r, lf, p0w, lane, ac, as);
 
     const long long p0 = p0w + 4 * (lane & 15);
     if (p0 >= a.r.npix) continue;
@@ -200,7 +216,7 @@ __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs 
         float2 v[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) v[t] = make_float2(ac[f][t][rr] + dc, as[f][t][rr]);
-        dft_store_bin(a, b, p0, bin, v, L, lens);
+        dft_store_bin(planes, a.r.npix, b, p0, bin, v, L, lens);
       }
     }
   }
@@ -241,17 +257,29 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
   const long long plane_elems = (long long)a.H * W;
   const bool lens = a.lx != nullptr;
   const int G = gridDim.x;
-  int y = xcd_tile(blockIdx.x, G);
+  // rows of all windows of the launch, window-major (MULTI has no registers for the window's
+  // pointers: 217 -> 296 us at 1024^2; its launcher runs one window at a time)
+  const int rows = MULTI ? a.H : a.H * a.nwin;
+  int row = xcd_tile(blockIdx.x, G);
   uint2 pre[TPW][dft_pre_steps<MODE>()];
-  if (y < a.H) dft_prefetch<MODE, TPW>(a.r, (long long)y * W + wave * 64 * TPW, lane, pre);
+  auto prefetch = [&](int i, int ln) {
+    if constexpr (MULTI) {
+      dft_prefetch<MODE, TPW>(a.r, (long long)i * W + wave * 64 * TPW, ln, pre);
+    } else {
+      const int w = i / a.H;
+      dft_prefetch<MODE, TPW>(window_ring(a, w), (long long)(i - w * a.H) * W + wave * 64 * TPW, ln, pre);
+    }
+  };
+  if (row < rows) prefetch(row, lane);
 
-  for (; y < a.H; y += G) {
+  for (; row < rows; row += G) {
+    const int win = MULTI ? 0 : row / a.H, y = row - win * a.H;
     // An opaque per-row copy of the lane index keeps the many loop-invariant LDS
     // addresses of the scatter and the transforms out of registers across rows.
     int lane;
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
     f4 acc[TPW][NBT][4];
-    dft_tile<NBT, MODE, TPW>(a.r, wmat, (long long)y * W + wave * 64 * TPW, lane, pre, acc);
+    dft_tile<NBT, MODE, TPW>(MULTI ? a.r : window_ring(a, win), wmat, (long long)y * W + wave * 64 * TPW, lane, pre, acc);
     // lens factors of the lane's pixels (1 without a lens: the product with (1, 0) is exact,
     // and cheaper than a select)
     auto lens_factors = [&](int i, float2 (&L)[4]) {
@@ -273,7 +301,7 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
       for (int i = 0; i < TPW; ++i) lens_factors(i, Ls[i]);
     }
     // the next row's first frames load while this row is scattered and transformed
-    if (y + G < a.H) dft_prefetch<MODE, TPW>(a.r, (long long)(y + G) * W + wave * 64 * TPW, lane, pre);
+    if (row + G < rows) prefetch(row + G, lane);
 
     // scatter planes [q0, q0+GB) from the MFMA registers into padded LDS rows
     auto scatter = [&](int q0) {
@@ -328,7 +356,7 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = ws[F::pad(lane + 64 * m)];
         F::template run<false>(v, ws, twl, lane);
-        float2 *dst = a.planes + (long long)q * plane_elems + row_off;
+        float2 *dst = a.planes_w[win] + (long long)q * plane_elems + row_off;
 #pragma unroll
         for (int m = 0; m < E; ++m) dst[(long long)m * 64 * a.H] = v[m];
       }
@@ -406,23 +434,16 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   const bool lens = a.lx_w[0] != nullptr;
   const int G = gridDim.x;
   const int y0 = xcd_tile(blockIdx.x, G);
-  const int nrw = y0 < a.H ? (a.H - 1 - y0) / G + 1 : 0;  // rows of one window
-  const int nr = nrw * a.nwin;                             // rows of all windows, window-major
+  const int rows = a.H * a.nwin;                           // rows of all windows, window-major
+  const int nr = y0 < rows ? (rows - 1 - y0) / G + 1 : 0;  // of them this block's
 
   f4 acc[TPW][NBT][4];        // interleaved rows (!FOLD)
   f4 fre[TPW][4], fim[TPW][4];  // Re and Im of bins 4 g + r (FOLD)
   std::conditional_t<FOLD, DftStreamFold<TPW, T, 4>, DftStream<NBT, TPW, T, front_ring(T)>> stream;
   auto px0 = [&](int y) { return (long long)y * W + rw * 64 * TPW; };
-  auto row_y = [&](int i) { return y0 + (nrw ? i % nrw : 0) * G; };
-  auto win_of = [&](int i) { return nrw ? i / nrw : 0; };
-  auto ring_of = [&](int i) {
-    const int w = win_of(i);
-    DftRing r = a.r;
-    r.ring = a.rings[w];
-    r.ring_frames = a.ring_frames_w[w];
-    r.first = a.firsts[w];
-    return r;
-  };
+  auto win_of = [&](int i) { return (y0 + i * G) / a.H; };
+  auto row_y = [&](int i) { return (y0 + i * G) % a.H; };
+  auto ring_of = [&](int i) { return window_ring(a, win_of(i)); };
 
   // producers: the band spectra of row i for their 128 pixels
   auto dft_row = [&](int i, int lane) {
@@ -529,7 +550,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   if (producer) {
     const int lane0 = tid & 63;
     if (nr > 0) {
-      stream.start(ring_of(0), px0(y0), lane0);
+      stream.start(ring_of(0), px0(row_y(0)), lane0);
       dft_row(0, lane0);
       scatter(0, lane0);
     }
@@ -569,7 +590,6 @@ static DftArgs make_args(const DftLaunch &L) {
   a.nb = L.nb;
   a.nbc = L.nbc;
   a.both = L.both;
-  a.planes = L.planes;
   a.lx = L.lx;
   a.ly = L.ly;
   switch (L.precision) {
@@ -580,7 +600,7 @@ static DftArgs make_args(const DftLaunch &L) {
   a.wm_lo = L.wm_f16lo;
   a.nwin = L.nwin > 0 ? L.nwin : 1;
   for (int w = 0; w < HFX_MAX_WIN; ++w) {
-    const bool own = w < a.nwin && L.rings[w] != nullptr;  // a window of another plan of the group
+    const bool own = w < a.nwin && w < HFX_MAX_GROUP && L.rings[w] != nullptr;  // a window of another plan of the group
     a.firsts[w] = w == 0 ? L.first : w < a.nwin ? L.firsts[w] : L.first;
     a.rings[w] = own ? L.rings[w] : L.ring;
     a.ring_frames_w[w] = own ? L.ring_frames_w[w] : L.ring_frames;
@@ -602,10 +622,12 @@ static unsigned persistent_grid(const void *kernel, size_t lds, long long items)
   return (unsigned)(items < g ? (items > 0 ? items : 1) : g);
 }
 
+// groups of four 64-pixel tiles over all windows of a stand-alone launch
+static long long dft_quads(const DftArgs &a) { return (a.r.npix + 255) / 256 * a.nwin; }
+
 template <int NBT, int MODE> static int launch_plain(const DftArgs &a, hipStream_t st) {
-  const long long waves = (a.r.npix + 63) / 64;
   const size_t lds = dft_matrix_lds_bytes(NBT, MODE, a.r.T);
-  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft<NBT, MODE>), lds, (waves + 3) / 4);
+  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft<NBT, MODE>), lds, dft_quads(a));
   hipLaunchKernelGGL((k_dft<NBT, MODE>), dim3(grid), dim3(256), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -621,14 +643,14 @@ template <int NBT> static int launch_plain_mode(const DftArgs &a, int mode, hipS
 }
 
 template <int NBF> static int launch_fold(const DftArgs &a, hipStream_t st) {
-  const long long waves = (a.r.npix + 63) / 64;
   const size_t lds = dft_fold_lds_bytes(NBF, a.r.T);
-  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF>), lds, (waves + 3) / 4);
+  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF>), lds, dft_quads(a));
   hipLaunchKernelGGL((k_dft_fold<NBF>), dim3(grid), dim3(256), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_time_dft(const DftLaunch &L, hipStream_t st) {
+  if (L.nwin > HFX_MAX_WIN) return -6;
   const DftArgs a = make_args(L);
   // FP32 with more than one 16-row tile of interleaved rows: the folded contraction
   if (L.precision == 0 && L.T % 32 == 0 && L.nbc > 8 && L.nbc <= 64) {
@@ -664,12 +686,13 @@ bool dft_front_pipelined(int W, int nbc, int T, int n_planes, int precision) {
 
 template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipStream_t st) {
   const size_t lds = dft_matrix_lds_bytes(NBT, MODE, a.r.T);
-  // persistent grid: one workgroup per CU (the LDS footprint allows no more), each
-  // walking rows blockIdx, blockIdx + grid, ...
+  // persistent grid: one workgroup per CU (the LDS footprint allows no more), each walking rows
+  // blockIdx, blockIdx + grid, ... of the launch's windows
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const unsigned grid = (unsigned)(a.H < cus ? a.H : cus);
+  const long long rows = (long long)a.H * a.nwin;
+  const unsigned grid = (unsigned)(rows < cus ? rows : cus);
   const int T = a.r.T;
   if (MODE == 0 && a.n_planes <= row_group<W>() && (T == 32 || T == 64 || T == 128)) {
     if (T == 32)
@@ -678,10 +701,17 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
       hipLaunchKernelGGL((k_front<W, NBT, 0, 64>), dim3(grid), dim3(front_threads<W>()), lds, st, a);
     else
       hipLaunchKernelGGL((k_front<W, NBT, 0, 128>), dim3(grid), dim3(front_threads<W>()), lds, st, a);
-  } else if (a.n_planes <= row_group<W>())
+  } else if (a.n_planes <= row_group<W>()) {
     hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, false>), dim3(grid), dim3(row_threads<W>()), lds, st, a);
-  else
-    hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, true>), dim3(grid), dim3(row_threads<W>()), lds, st, a);
+  } else {
+    for (int w = 0; w < a.nwin; ++w) {  // one window per launch
+      DftArgs one = a;
+      one.r.first = a.firsts[w];
+      one.planes_w[0] = a.planes_w[w];
+      hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, true>), dim3((unsigned)(a.H < cus ? a.H : cus)), dim3(row_threads<W>()),
+                         lds, st, one);
+    }
+  }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -704,8 +734,9 @@ template <int W> static int launch_row_w(const DftArgs &a, int nbt, int mode, hi
 int launch_time_dft_row(const DftLaunch &L, int H, int blk_c, int n_planes, const float2 *tw,
                         hipStream_t st) {
   if (!dft_row_supported(L.W, L.nbc, L.T)) return -2;
-  if (L.nwin > 1 && (L.nwin > HFX_MAX_WIN || !dft_front_pipelined(L.W, L.nbc, L.T, n_planes, L.precision)))
-    return -6;
+  if (L.nwin > HFX_MAX_WIN || (long long)H * (L.nwin > 1 ? L.nwin : 1) > INT32_MAX) return -6;
+  // windows of several plans: only k_front reads each window's own lens
+  if (L.nwin > 1 && L.rings[0] != nullptr && !dft_front_pipelined(L.W, L.nbc, L.T, n_planes, L.precision)) return -6;
   DftArgs a = make_args(L);
   a.H = H;
   a.blk_c = blk_c;

@@ -32,22 +32,24 @@ int launch_flatfield_spatial(const float *in, float *out, float *tmp, long long 
                              const float *kx, int rx, const float *ky, int ry, hipStream_t st);
 
 // ---- time DFT (dft.hip)
-constexpr int HFX_MAX_WIN = 4;  // windows per pipelined front launch (one plan, or a group of plans)
+constexpr int HFX_MAX_WIN = 32;   // windows of one plan per launch
+constexpr int HFX_MAX_GROUP = 4;  // windows of several plans per launch
 
 struct DftLaunch {
   const uint16_t *ring;
   long long ring_frames, first;
-  // pipelined front only: windows 1 .. nwin-1 start at firsts[w] and write their planes at
-  // planes + w * planes_stride (nwin = 1: just `first` and `planes`)
+  // windows 1 .. nwin-1 start at firsts[w] and write their planes at planes + w * planes_stride
+  // (nwin <= 1: just `first` and `planes`)
   int nwin;
   long long firsts[HFX_MAX_WIN];
   long long planes_stride;
-  // grouped launch (windows of several plans of one shape): per-window ring, ring length,
-  // planes and Fresnel lens; null rings[w] means ring / ring_frames / planes + w * stride / lx, ly
-  const uint16_t *rings[HFX_MAX_WIN];
-  long long ring_frames_w[HFX_MAX_WIN];
-  float2 *planes_w[HFX_MAX_WIN];
-  const float2 *lx_w[HFX_MAX_WIN], *ly_w[HFX_MAX_WIN];
+  // grouped launch (windows of several plans of one shape, pipelined front only): per-window
+  // ring, ring length, planes and Fresnel lens; null rings[w] means ring / ring_frames /
+  // planes + w * stride / lx, ly
+  const uint16_t *rings[HFX_MAX_GROUP];
+  long long ring_frames_w[HFX_MAX_GROUP];
+  float2 *planes_w[HFX_MAX_GROUP];
+  const float2 *lx_w[HFX_MAX_GROUP], *ly_w[HFX_MAX_GROUP];
   int T;
   long long npix;
   int W;
@@ -61,7 +63,7 @@ struct DftLaunch {
 int launch_time_dft(const DftLaunch &L, hipStream_t st);
 // Fused time DFT + forward row FFT into the column-blocked layout (L.planes is blocked).
 bool dft_row_supported(int W, int nbc, int T);
-// true when launch_time_dft_row runs the pipelined front kernel (and so accepts nwin > 1)
+// true when launch_time_dft_row runs the pipelined front kernel (and so accepts grouped windows)
 bool dft_front_pipelined(int W, int nbc, int T, int n_planes, int precision);
 int launch_time_dft_row(const DftLaunch &L, int H, int blk_c, int n_planes, const float2 *tw,
                         hipStream_t st);
@@ -111,7 +113,7 @@ struct PassArgs {
   // windows of one plan: byte strides of in and out, element stride of the moment images
   long long win_in, win_out, win_mom;
   int grouped;              // windows of several plans: window blockIdx.z takes win[blockIdx.z]
-  PassWin win[HFX_MAX_WIN];
+  PassWin win[HFX_MAX_GROUP];
 };
 
 int launch_row_pass(const PassArgs &a, hipStream_t st);

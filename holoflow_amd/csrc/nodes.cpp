@@ -38,6 +38,8 @@
 #include "holoflow/core/registry.hh"
 
 namespace hfx {
+// hfx_plan_create without the batch workspaces (api.hip): for plans that only run hfx_moments
+hfx_status plan_create_one_window(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out);
 void set_last_error(const std::string &msg);  // libhfx's thread-local last error (api.hip)
 }
 
@@ -1231,7 +1233,7 @@ class DopplerMomentsFactory : public ISyncTaskFactory {
     t->settings = j;
     t->idesc = in[0];
     const auto p = moments_desc(j, in[0]);
-    HFX_CHECK(hfx_plan_create(&p, hs(ctx.stream), &t->plan));
+    HFX_CHECK(hfx::plan_create_one_window(&p, hs(ctx.stream), &t->plan));
     return t;
   }
   std::unique_ptr<ISyncTask> update(std::unique_ptr<ISyncTask> old, std::span<const TDesc> in, const Json &j,
