@@ -565,73 +565,249 @@ __global__ void k_dft_axis(DftAxisArgs a) {
   a.out[t] = make_float2(sr * a.scale, si * a.scale);
 }
 
-// Band DFT along one axis, tiled: a block owns 256 consecutive inner indices of one outer
-// index, so every load of x[o, j, i0 .. i0+255] is one coalesced row; each thread keeps
-// DFT_KC bins' accumulators and walks j once per chunk of bins.  The twiddles
-// w[m] = exp(-2 pi i m / n) are built in LDS (FP64 sincospi, rounded once); the phase index
-// (k j) mod n advances by k per sample (bins past the band advance by 0 and are not stored).
-// DT: 1 U16, 2 F32, 3 CF32 (compile-time, so real inputs carry no imaginary terms).
-constexpr int DFT_KC = 16, DFT_TILE = 256, DFT_MAXN = 4096;
+// Band DFT along the middle axis on the matrix cores, n <= DFT_MAXN.  A wave owns 64 columns (an
+// outer and an inner index; four adjacent ones per lane), and the symmetry of the kernel is folded
+// as in the fused path's time DFT: with s = x_p + x_{n-p}, d = x_p - x_{n-p},
+//   X_k = x_0 [+ (-1)^k x_{n/2}] + sum_{p=1}^{(n-1)/2} (s cos(2 pi k p / n) - i d sin(2 pi k p / n)),
+// so 16 bins and 16 columns take 2 ((n-1)/2)/4 + 1 FP32 MFMAs for real input, twice that for
+// complex.  Step st covers the pairs p = 4 st + g + 1 (g = lane >> 4, the MFMA's K index).  The
+// operands cos, -sin come from an LDS table of the n roots (FP64 sincospi, rounded once) through a
+// running index k p mod n, one 8-byte read per 16 bins and step for four (complex: eight) MFMAs per
+// operand, so any n and any bin range work without an operand matrix.
+//
+// Bound by memory: F32 [64][1024^2] -> 33 bins (three 16-bin tiles) moves 545 MB.  The kernel it
+// replaces (direct sums on the VALU, 16 bins per pass over the input) took 570 us there.
+//
+// Lanes whose pair or column does not exist get zero samples, not zero weights, so that an
+// infinity elsewhere in the column is not turned into a NaN.
+//
+// DT: 1 U16, 2 F32, 3 CF32.  VEC: the four columns of a lane are adjacent in memory and aligned.
+constexpr int DFT_MAXN = 4096;
+typedef float f4v __attribute__((ext_vector_type(4)));
 
-template <int DT>
-__global__ __launch_bounds__(DFT_TILE) void k_dft_axis_tiled(DftAxisArgs a, long long tiles) {
+template <int DT, bool VEC> struct DftColumns {
+  static constexpr int NF = DT == 3 ? 8 : 4;  // floats of four samples
+  const char *base[VEC ? 1 : 4];
+  long long step;  // bytes from sample j to j + 1 of a column
+  // first column c (of outer * inner)
+  __device__ __forceinline__ void init(const DftAxisArgs &a, long long c, long long cols) {
+    constexpr int esz = DT == 1 ? 2 : DT == 2 ? 4 : 8;
+    step = a.inner * esz;
+#pragma unroll
+    for (int t = 0; t < (VEC ? 1 : 4); ++t) {
+      const long long cc = c + t < cols ? c + t : cols - 1;  // past the end: the last column, not stored
+      const long long o = cc / a.inner, i = cc - o * a.inner;
+      base[t] = reinterpret_cast<const char *>(a.in) + (o * a.n * a.inner + i) * esz;
+    }
+  }
+  // the raw samples j of the four columns
+  struct Raw {
+    uint4 q[VEC && DT == 3 ? 2 : 1];
+    unsigned w[VEC ? 1 : NF];
+  };
+  __device__ __forceinline__ void load(Raw &r, int j) const {
+    const long long off = j * step;
+    if constexpr (VEC) {
+      if constexpr (DT == 1) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(base[0] + off);
+        r.q[0].x = v.x;
+        r.q[0].y = v.y;
+      } else {
+        r.q[0] = *reinterpret_cast<const uint4 *>(base[0] + off);
+        if constexpr (DT == 3) r.q[1] = *reinterpret_cast<const uint4 *>(base[0] + off + 16);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (DT == 1) {
+          r.w[t] = *reinterpret_cast<const uint16_t *>(base[t] + off);
+        } else if constexpr (DT == 2) {
+          r.w[t] = *reinterpret_cast<const unsigned *>(base[t] + off);
+        } else {
+          const uint2 v = *reinterpret_cast<const uint2 *>(base[t] + off);
+          r.w[2 * t] = v.x;
+          r.w[2 * t + 1] = v.y;
+        }
+      }
+    }
+  }
+  // samples as floats (complex: re, im per column)
+  __device__ __forceinline__ static void unpack(const Raw &r, float (&x)[NF]) {
+    if constexpr (VEC && DT == 1) {
+      x[0] = (float)(r.q[0].x & 0xffffu);
+      x[1] = (float)(r.q[0].x >> 16);
+      x[2] = (float)(r.q[0].y & 0xffffu);
+      x[3] = (float)(r.q[0].y >> 16);
+    } else if constexpr (VEC) {
+#pragma unroll
+      for (int h = 0; h < NF / 4; ++h) {
+        x[4 * h] = __uint_as_float(r.q[h].x);
+        x[4 * h + 1] = __uint_as_float(r.q[h].y);
+        x[4 * h + 2] = __uint_as_float(r.q[h].z);
+        x[4 * h + 3] = __uint_as_float(r.q[h].w);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NF; ++t) x[t] = DT == 1 ? (float)r.w[t] : __uint_as_float(r.w[t]);
+    }
+  }
+};
+
+// NBF: 16-bin tiles from bin k0 on that a wave holds at once (the input is read once per launch)
+template <int DT, bool VEC, int NBF>
+__global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0, long long cols) {
   extern __shared__ float2 tw[];
-  for (int m = threadIdx.x; m < a.n; m += DFT_TILE) {
+  for (int m = threadIdx.x; m < a.n; m += 256) {
     double s, c;
     sincospi(2.0 * (double)m / (double)a.n, &s, &c);
     tw[m] = make_float2((float)c, (float)(-s));
   }
   __syncthreads();
-  const long long o = blockIdx.x / tiles;
-  const long long i = (blockIdx.x % tiles) * DFT_TILE + threadIdx.x;
-  if (i >= a.inner) return;
-  const long long nk = a.ke - a.kb;
-  const long long base = o * (long long)a.n * a.inner + i;
-  for (int k0 = a.kb; k0 < a.ke; k0 += DFT_KC) {
-    float2 acc[DFT_KC];
-    int m[DFT_KC], step[DFT_KC];
+  using X = DftColumns<DT, VEC>;
+  constexpr int NF = X::NF;
+  constexpr int K = DT == 3 ? 2 : 4;  // pair steps in flight
+  const int n = a.n, pairs = (n - 1) / 2, steps = (pairs + 3) / 4;
+  const int lane = threadIdx.x & 63, g = lane >> 4, rw = lane & 15;
+  const long long tiles = (cols + 63) / 64;
+  for (long long it = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); it < tiles; it += (long long)gridDim.x * 4) {
+    const long long c0 = it * 64 + 4 * rw;
+    X x;
+    x.init(a, c0 < cols ? c0 : cols - 1, cols);
+    f4v re[NBF][4], im[NBF][4];
+    int idx[NBF], inc[NBF];  // k p mod n of this lane's bin and pair, and its advance by four pairs
 #pragma unroll
-    for (int c = 0; c < DFT_KC; ++c) {
-      acc[c] = make_float2(0.f, 0.f);
-      m[c] = 0;
-      step[c] = k0 + c < a.ke ? k0 + c : 0;
+    for (int f = 0; f < NBF; ++f) {
+      const long long k = k0 + 16 * f + rw;
+      idx[f] = (int)(k * (g + 1) % n);
+      inc[f] = (int)(4 * k % n);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) re[f][t] = im[f][t] = f4v{0.f, 0.f, 0.f, 0.f};
     }
-#pragma unroll 2
-    for (int j = 0; j < a.n; ++j) {
-      const long long src = base + (long long)j * a.inner;
-      float xr, xi = 0.f;
-      if constexpr (DT == 1) {
-        xr = (float)reinterpret_cast<const uint16_t *>(a.in)[src];
-      } else if constexpr (DT == 2) {
-        xr = reinterpret_cast<const float *>(a.in)[src];
-      } else {
-        const float2 v = reinterpret_cast<const float2 *>(a.in)[src];
-        xr = v.x;
-        xi = v.y;
+    typename X::Raw r[K][2], xe;
+    auto load = [&](int st, int slot) {
+      const int p = min(4 * st + g + 1, max(pairs, 1));
+      x.load(r[slot][0], n > 1 ? p : 0);
+      x.load(r[slot][1], n - p);
+    };
+    x.load(xe, g == 0 ? 0 : n / 2);
+#pragma unroll
+    for (int j = 0; j < K; ++j) load(j, j);
+    auto step = [&](int st, int slot, bool refill) {
+      float x1[NF], x2[NF];
+      X::unpack(r[slot][0], x1);
+      X::unpack(r[slot][1], x2);
+      if (refill) load(st + K, slot);
+      const bool in = 4 * st + g < pairs;
+      float sm[NF], df[NF];
+#pragma unroll
+      for (int t = 0; t < NF; ++t) {
+        sm[t] = in ? x1[t] + x2[t] : 0.f;
+        df[t] = in ? x1[t] - x2[t] : 0.f;
       }
-      float2 w[DFT_KC];
 #pragma unroll
-      for (int c = 0; c < DFT_KC; ++c) w[c] = tw[m[c]];
+      for (int f = 0; f < NBF; ++f) {
+        const float2 w = tw[idx[f]];
+        idx[f] += inc[f];
+        idx[f] = idx[f] >= n ? idx[f] - n : idx[f];
 #pragma unroll
-      for (int c = 0; c < DFT_KC; ++c) {
-        if constexpr (DT == 3) {
-          acc[c].x += xr * w[c].x - xi * w[c].y;
-          acc[c].y += xr * w[c].y + xi * w[c].x;
-        } else {
-          acc[c].x += xr * w[c].x;
-          acc[c].y += xr * w[c].y;
+        for (int t = 0; t < 4; ++t) {
+          if constexpr (DT == 3) {
+            re[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, sm[2 * t], re[f][t], 0, 0, 0);
+            im[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, sm[2 * t + 1], im[f][t], 0, 0, 0);
+          } else {
+            re[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, sm[t], re[f][t], 0, 0, 0);
+            im[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, df[t], im[f][t], 0, 0, 0);
+          }
         }
-        m[c] += step[c];
-        m[c] = m[c] >= a.n ? m[c] - a.n : m[c];
+        if constexpr (DT == 3) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            re[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, -df[2 * t + 1], re[f][t], 0, 0, 0);
+            im[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, df[2 * t], im[f][t], 0, 0, 0);
+          }
+        }
       }
+    };
+    int st = 0;
+    for (; st + K < steps; st += K) {
+#pragma unroll
+      for (int j = 0; j < K; ++j) step(st + j, j, true);
     }
 #pragma unroll
-    for (int c = 0; c < DFT_KC; ++c) {
-      if (k0 + c < a.ke) {
-        const long long k = k0 + c - a.kb;
-        a.out[(o * nk + k) * a.inner + i] = make_float2(acc[c].x * a.scale, acc[c].y * a.scale);
+    for (int j = 0; j < K; ++j) step(st + j, j, false);  // steps past the last pair add zeros
+    // x_0 (g = 0, weight 1) and, for even n, x_{n/2} (g = 1, weight (-1)^k)
+    float xv[NF];
+    X::unpack(xe, xv);
+    const bool in = g == 0 || (g == 1 && n % 2 == 0);
+#pragma unroll
+    for (int t = 0; t < NF; ++t) xv[t] = in ? xv[t] : 0.f;
+#pragma unroll
+    for (int f = 0; f < NBF; ++f) {
+      const float w = g == 1 && ((k0 + 16 * f + rw) & 1) ? -1.f : 1.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (DT == 3) {
+          re[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, xv[2 * t], re[f][t], 0, 0, 0);
+          im[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, xv[2 * t + 1], im[f][t], 0, 0, 0);
+        } else {
+          re[f][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, xv[t], re[f][t], 0, 0, 0);
+        }
       }
     }
+    // lane holds bins 16 f + 4 g + r of its four columns
+    const long long nk = a.ke - a.kb;
+    if (c0 >= cols) continue;
+#pragma unroll
+    for (int f = 0; f < NBF; ++f) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 16 * f + 4 * g + q;
+        if (k >= a.ke) continue;
+        float2 v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = make_float2(re[f][t][q] * a.scale, im[f][t][q] * a.scale);
+        if constexpr (VEC) {
+          const long long o = c0 / a.inner, i = c0 - o * a.inner;
+          float4 *dst = reinterpret_cast<float4 *>(a.out + (o * nk + (k - a.kb)) * a.inner + i);
+          dst[0] = make_float4(v[0].x, v[0].y, v[1].x, v[1].y);
+          dst[1] = make_float4(v[2].x, v[2].y, v[3].x, v[3].y);
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            if (c0 + t < cols) {
+              const long long o = (c0 + t) / a.inner, i = c0 + t - o * a.inner;
+              a.out[(o * nk + (k - a.kb)) * a.inner + i] = v[t];
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int DT, bool VEC, int NBF> static void launch_axis_nbf(const DftAxisArgs &a, int k0, long long cols, hipStream_t st) {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  // persistent: the blocks that are resident at once (their registers allow four, three and two per
+  // CU for one, two and three 16-bin tiles) walk the tiles
+  const long long quads = (cols + 255) / 256, most = (long long)cus * (NBF == 1 ? 4 : NBF == 2 ? 3 : 2);
+  const unsigned grid = (unsigned)(quads < most ? quads : most);
+  hipLaunchKernelGGL((k_dft_axis_mfma<DT, VEC, NBF>), dim3(grid), dim3(256), (size_t)a.n * sizeof(float2), st, a, k0, cols);
+}
+
+template <int DT, bool VEC> static void launch_axis(const DftAxisArgs &a, long long cols, hipStream_t st) {
+  // the bins in as few passes over the input as the registers allow (three 16-bin tiles; two where
+  // a lane keeps four addresses), evenly filled
+  constexpr int MOST = VEC ? 3 : 2;
+  const int tiles = (a.ke - a.kb + 15) / 16, passes = (tiles + MOST - 1) / MOST, nbf = (tiles + passes - 1) / passes;
+  for (int k0 = a.kb; k0 < a.ke; k0 += 16 * nbf) {
+    if (nbf == 1)
+      launch_axis_nbf<DT, VEC, 1>(a, k0, cols, st);
+    else if (nbf == 2)
+      launch_axis_nbf<DT, VEC, 2>(a, k0, cols, st);
+    else
+      launch_axis_nbf<DT, VEC, MOST>(a, k0, cols, st);
   }
 }
 
@@ -640,17 +816,15 @@ int launch_dft_axis(const void *in, int dtype, long long outer, int n, long long
   DftAxisArgs a{in, dtype, outer, inner, n, kb, ke, scale, out};
   long long total = outer * (long long)(ke - kb) * inner;
   if (total == 0) return 0;
-  const long long tiles = (inner + DFT_TILE - 1) / DFT_TILE;
-  if (n <= DFT_MAXN && outer * tiles < (1LL << 31) && kb >= 0 && ke <= n) {
-    // the phase counters reach at most (k0 + c) + n - 1 < 2 n before their wrap
-    const dim3 grid((unsigned)(outer * tiles)), block(DFT_TILE);
-    const size_t lds = (size_t)n * sizeof(float2);
-    if (dtype == 1)
-      hipLaunchKernelGGL(k_dft_axis_tiled<1>, grid, block, lds, st, a, tiles);
-    else if (dtype == 2)
-      hipLaunchKernelGGL(k_dft_axis_tiled<2>, grid, block, lds, st, a, tiles);
-    else
-      hipLaunchKernelGGL(k_dft_axis_tiled<3>, grid, block, lds, st, a, tiles);
+  if (n <= DFT_MAXN) {
+    const long long cols = outer * inner;
+    const uintptr_t align = reinterpret_cast<uintptr_t>(in) % (dtype == 1 ? 8 : 16) + reinterpret_cast<uintptr_t>(out) % 16;
+    const bool vec = inner % 4 == 0 && align == 0;  // four adjacent columns share an outer index
+    switch (dtype) {
+      case 1: vec ? launch_axis<1, true>(a, cols, st) : launch_axis<1, false>(a, cols, st); break;
+      case 2: vec ? launch_axis<2, true>(a, cols, st) : launch_axis<2, false>(a, cols, st); break;
+      default: vec ? launch_axis<3, true>(a, cols, st) : launch_axis<3, false>(a, cols, st); break;
+    }
   } else {
     hipLaunchKernelGGL(k_dft_axis, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a);
   }
