@@ -36,15 +36,19 @@ struct DftArgs {
   // fused kernels only
   int H, blk_c, n_planes;
   const float2 *tw;        // W-point FFT twiddles
-  // the windows of one launch (one plan's consecutive windows, or for k_front one window each of
-  // a group of plans of one shape): ring, ring length, first frame, planes (k_dft: natural
-  // [planes][npix]; the fused kernels: blocked), lens
-  int nwin;
-  long long firsts[HFX_MAX_WIN];
-  const uint16_t *rings[HFX_MAX_WIN];
-  long long ring_frames_w[HFX_MAX_WIN];
-  float2 *planes_w[HFX_MAX_WIN];
-  const float2 *lx_w[HFX_MAX_WIN], *ly_w[HFX_MAX_WIN];
+  // the windows of one launch: one plan's consecutive windows (first frames, planes at a stride),
+  // or for k_front one window each of a group of plans of one shape (the group's tables).  The
+  // fields of the common case come first and the tables last: kernel arguments lie in host memory,
+  // and each further line of them that a kernel reads is another round trip (a table entry per
+  // pointer cost a 64 x 64 window's time DFT 0.7 us)
+  int nwin, grouped;
+  float2 *planes;          // k_dft: natural [planes][npix]; the fused kernels: blocked
+  long long planes_stride; // elements from one window's planes to the next
+  int firsts[HFX_MAX_WIN];
+  const uint16_t *rings[HFX_MAX_GROUP];
+  long long ring_frames_w[HFX_MAX_GROUP];
+  float2 *planes_w[HFX_MAX_GROUP];
+  const float2 *lx_w[HFX_MAX_GROUP], *ly_w[HFX_MAX_GROUP];
 };
 
 // a wave-uniform value kept in a scalar register from here on (an opaque copy the compiler
@@ -109,12 +113,21 @@ __device__ __forceinline__ void dft_store_bin(float2 *planes, long long npix, co
   }
 }
 
+// Window of item i where each window has `per` items (no division in the first window, which is all
+// of a single-window launch: the integer division is some forty dependent instructions).
+__device__ __forceinline__ int window_of(unsigned i, unsigned per) {
+  if (i < per) return 0;
+  return (int)(i / per);
+}
+
 // Ring of window w of the launch (windows of one plan share it up to the first frame).
-__device__ __forceinline__ DftRing window_ring(const DftArgs &a, int w) {
+template <bool GROUPS = false> __device__ __forceinline__ DftRing window_ring(const DftArgs &a, int w) {
   DftRing r = a.r;
-  r.ring = a.rings[w];
-  r.ring_frames = a.ring_frames_w[w];
-  r.first = a.firsts[w];
+  if (GROUPS && a.grouped) {
+    r.ring = a.rings[w];
+    r.ring_frames = a.ring_frames_w[w];
+  }
+  if (w != 0) r.first = a.firsts[w];  // (window 0's is in the struct's first lines)
   return r;
 }
 
@@ -130,9 +143,9 @@ __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
   const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
   const bool lens = a.lx != nullptr;
   for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
-    const unsigned w = it / quads;
+    const unsigned w = window_of(it, quads);
     const DftRing r = window_ring(a, w);
-    float2 *planes = a.planes_w[w];
+    float2 *planes = a.planes + w * a.planes_stride;
     // an opaque per-tile copy of the lane index keeps the lane-derived LDS and load addresses of
     // the MFMA loop from being hoisted out of the tile loop (where they would hold registers)
     int lane;
@@ -187,9 +200,9 @@ __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs 
   const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
   const bool lens = a.lx != nullptr;
   for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
-    const unsigned w = it / quads;
+    const unsigned w = window_of(it, quads);
     const DftRing r = window_ring(a, w);
-    float2 *planes = a.planes_w[w];
+    float2 *planes = a.planes + w * a.planes_stride;
     int lane;  // opaque per tile, as in k_dft
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(threadIdx.x & 63));
     // tiles past the end load clamped pixels (dft_px) and store nothing
@@ -266,14 +279,14 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
     if constexpr (MULTI) {
       dft_prefetch<MODE, TPW>(a.r, (long long)i * W + wave * 64 * TPW, ln, pre);
     } else {
-      const int w = i / a.H;
+      const int w = window_of(i, a.H);
       dft_prefetch<MODE, TPW>(window_ring(a, w), (long long)(i - w * a.H) * W + wave * 64 * TPW, ln, pre);
     }
   };
   if (row < rows) prefetch(row, lane);
 
   for (; row < rows; row += G) {
-    const int win = MULTI ? 0 : row / a.H, y = row - win * a.H;
+    const int win = MULTI ? 0 : window_of(row, a.H), y = row - win * a.H;
     // An opaque per-row copy of the lane index keeps the many loop-invariant LDS
     // addresses of the scatter and the transforms out of registers across rows.
     int lane;
@@ -356,7 +369,7 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = ws[F::pad(lane + 64 * m)];
         F::template run<false>(v, ws, twl, lane);
-        float2 *dst = a.planes_w[win] + (long long)q * plane_elems + row_off;
+        float2 *dst = a.planes + win * a.planes_stride + (long long)q * plane_elems + row_off;
 #pragma unroll
         for (int m = 0; m < E; ++m) dst[(long long)m * 64 * a.H] = v[m];
       }
@@ -431,7 +444,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   __syncthreads();
 
   const long long plane_elems = (long long)a.H * W;
-  const bool lens = a.lx_w[0] != nullptr;
+  const bool lens = a.lx != nullptr;
   const int G = gridDim.x;
   const int y0 = xcd_tile(blockIdx.x, G);
   const int rows = a.H * a.nwin;                           // rows of all windows, window-major
@@ -441,9 +454,9 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   f4 fre[TPW][4], fim[TPW][4];  // Re and Im of bins 4 g + r (FOLD)
   std::conditional_t<FOLD, DftStreamFold<TPW, T, 4>, DftStream<NBT, TPW, T, front_ring(T)>> stream;
   auto px0 = [&](int y) { return (long long)y * W + rw * 64 * TPW; };
-  auto win_of = [&](int i) { return (y0 + i * G) / a.H; };
-  auto row_y = [&](int i) { return (y0 + i * G) % a.H; };
-  auto ring_of = [&](int i) { return window_ring(a, win_of(i)); };
+  auto win_of = [&](int i) { return window_of(y0 + i * G, a.H); };
+  auto row_y = [&](int i) { return y0 + i * G - win_of(i) * a.H; };
+  auto ring_of = [&](int i) { return window_ring<true>(a, win_of(i)); };
 
   // producers: the band spectra of row i for their 128 pixels
   auto dft_row = [&](int i, int lane) {
@@ -461,7 +474,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   // producers: MFMA registers of row i -> padded LDS rows (its window's lens for Fresnel)
   auto scatter = [&](int i, int lane) {
     const int y = row_y(i);
-    const float2 *lxw = a.lx_w[win_of(i)], *lyw = a.ly_w[win_of(i)];
+    const float2 *lxw = a.grouped ? a.lx_w[win_of(i)] : a.lx, *lyw = a.grouped ? a.ly_w[win_of(i)] : a.ly;
     // band bin `bin` of 4 pixels from x0 into the LDS plane rows (and its conjugate plane on
     // the two-sided path), lens applied.  The product's rounding is pinned (cmul_rn): the
     // first row is scattered by the copy of this code before the row loop, the others by the
@@ -530,7 +543,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
   // consumers: one wave per plane row: forward row FFT, then the column-blocked store
   auto transform = [&](int i, int lane) {
     const int y = row_y(i);
-    float2 *planes = a.planes_w[win_of(i)];
+    float2 *planes = a.grouped ? a.planes_w[win_of(i)] : a.planes + win_of(i) * a.planes_stride;
     const long long row_off = blk_lane_offset(lane, a.H, a.blk_c) + (long long)y * a.blk_c;
     for (int q = rw; q < a.n_planes; q += front_cw<W>()) {
       float2 *ws = scr + q * F::SCR;
@@ -599,14 +612,16 @@ static DftArgs make_args(const DftLaunch &L) {
   }
   a.wm_lo = L.wm_f16lo;
   a.nwin = L.nwin > 0 ? L.nwin : 1;
-  for (int w = 0; w < HFX_MAX_WIN; ++w) {
-    const bool own = w < a.nwin && w < HFX_MAX_GROUP && L.rings[w] != nullptr;  // a window of another plan of the group
-    a.firsts[w] = w == 0 ? L.first : w < a.nwin ? L.firsts[w] : L.first;
-    a.rings[w] = own ? L.rings[w] : L.ring;
-    a.ring_frames_w[w] = own ? L.ring_frames_w[w] : L.ring_frames;
-    a.planes_w[w] = own ? L.planes_w[w] : L.planes + (w < a.nwin ? w : 0) * L.planes_stride;
-    a.lx_w[w] = own ? L.lx_w[w] : L.lx;
-    a.ly_w[w] = own ? L.ly_w[w] : L.ly;
+  a.planes = L.planes;
+  a.planes_stride = L.planes_stride;
+  for (int w = 0; w < a.nwin && w < HFX_MAX_WIN; ++w) a.firsts[w] = (int)(w == 0 ? L.first : L.firsts[w]);
+  a.grouped = a.nwin > 1 && L.rings[0] != nullptr;
+  for (int w = 0; a.grouped && w < a.nwin && w < HFX_MAX_GROUP; ++w) {
+    a.rings[w] = L.rings[w];
+    a.ring_frames_w[w] = L.ring_frames_w[w];
+    a.planes_w[w] = L.planes_w[w];
+    a.lx_w[w] = L.lx_w[w];
+    a.ly_w[w] = L.ly_w[w];
   }
   return a;
 }
@@ -707,7 +722,7 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
     for (int w = 0; w < a.nwin; ++w) {  // one window per launch
       DftArgs one = a;
       one.r.first = a.firsts[w];
-      one.planes_w[0] = a.planes_w[w];
+      one.planes = a.planes + w * a.planes_stride;
       hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, true>), dim3((unsigned)(a.H < cus ? a.H : cus)), dim3(row_threads<W>()),
                          lds, st, one);
     }
@@ -735,8 +750,10 @@ int launch_time_dft_row(const DftLaunch &L, int H, int blk_c, int n_planes, cons
                         hipStream_t st) {
   if (!dft_row_supported(L.W, L.nbc, L.T)) return -2;
   if (L.nwin > HFX_MAX_WIN || (long long)H * (L.nwin > 1 ? L.nwin : 1) > INT32_MAX) return -6;
-  // windows of several plans: only k_front reads each window's own lens
-  if (L.nwin > 1 && L.rings[0] != nullptr && !dft_front_pipelined(L.W, L.nbc, L.T, n_planes, L.precision)) return -6;
+  // windows of several plans: only k_front reads their tables
+  if (L.nwin > 1 && L.rings[0] != nullptr &&
+      (L.nwin > HFX_MAX_GROUP || !dft_front_pipelined(L.W, L.nbc, L.T, n_planes, L.precision)))
+    return -6;
   DftArgs a = make_args(L);
   a.H = H;
   a.blk_c = blk_c;
