@@ -1075,18 +1075,7 @@ hfx_status hfx_weighted_mean(const void *in, int32_t in_complex, int64_t planes,
   if (planes <= 0 || npix <= 0) return fail(HFX_E_INVALID, "reduction has zero elements");
   const int power2 = (flags & HFX_REDUCE_POWER2) ? 1 : 0;
   const int absval = (flags & HFX_REDUCE_ABS) ? 1 : 0;
-  float *outs[3] = {out, nullptr, nullptr};
-  int rc;
-  if (weights) {
-    // out = mean_k(w_k * m_k): the weighted sum is the reducer's second output; its first
-    // (unweighted) output is written to the same buffer first and then overwritten.
-    outs[1] = out;
-    rc = hfx::launch_moments_reduce(in, in_complex, planes, npix, weights, weights, outs, 2, power2,
-                                    absval, S(stream));
-  } else {
-    rc = hfx::launch_moments_reduce(in, in_complex, planes, npix, nullptr, nullptr, outs, 1, power2,
-                                    absval, S(stream));
-  }
+  const int rc = hfx::launch_weighted_mean(in, in_complex, planes, npix, weights, out, power2, absval, S(stream));
   if (rc != 0) return fail(HFX_E_HIP, "reduce launch failed");
   return HFX_OK;
 }
@@ -1150,7 +1139,8 @@ hfx_status hfx_fftshift(const void *in, void *out, int32_t elem_size, int32_t nd
 hfx_status hfx_convert_u16(const uint16_t *in, void *out, int64_t n, int32_t to_complex,
                            hfx_stream_t stream) {
   if ((!in || !out) && n > 0) return fail(HFX_E_INVALID, "null argument");
-  if (hfx::launch_convert_u16(in, out, n, to_complex, S(stream)) != 0)
+  if (hfx::launch_convert(in, HFX_DTYPE_U16, out, to_complex ? HFX_DTYPE_CF32 : HFX_DTYPE_F32, HFX_CONV_REAL, n, nullptr,
+                          S(stream)) != 0)
     return fail(HFX_E_HIP, "conversion launch failed");
   return HFX_OK;
 }
