@@ -68,12 +68,13 @@ template <int E, bool BAND> struct Moments {
 // Sums of the S plane subsets of a block, added in subset order: thread t (of the 64 * waves
 // threads that hold one subset) of subset `sub` gets the elements m = sub, sub + S, ... of its
 // position, so the additions and the stores after them are spread over all waves.  Two of the
-// sums fit the transforms' scratch at a time.
-template <int E, int S, int NACC>
-__device__ __forceinline__ void fold_subsets(const float (&s)[NACC][E], float *red, int sub, int t, int nt,
+// sums fit the transforms' scratch at a time.  tr: the thread whose pixels this one reads back (t,
+// or with TR another mapping that suits the stores better).
+template <int E, int S, int NACC, bool TR = false>
+__device__ __forceinline__ void fold_subsets(const float (&s)[NACC][E], float *red, int sub, int t, int tr, int nt,
                                              float (&val)[NACC][(E + S - 1) / S]) {
   constexpr int IT = (E + S - 1) / S;
-  if constexpr (S == 1) {
+  if constexpr (S == 1 && !TR) {
 #pragma unroll
     for (int k = 0; k < NACC; ++k)
 #pragma unroll
@@ -94,9 +95,9 @@ __device__ __forceinline__ void fold_subsets(const float (&s)[NACC][E], float *r
           const int m = sub + it * S;
           float x = 0.f;
           if (m < E) {
-            x = red[((k - k0) * S * E + m) * nt + t];
+            x = red[((k - k0) * S * E + m) * nt + tr];
 #pragma unroll
-            for (int j = 1; j < S; ++j) x += red[(((k - k0) * S + j) * E + m) * nt + t];
+            for (int j = 1; j < S; ++j) x += red[(((k - k0) * S + j) * E + m) * nt + tr];
           }
           val[k][it] = x;
         }
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(wrow_threads(N, KIND)) void k_wrow(PassArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // an unused last refill lands first
     constexpr int IT = (E + S - 1) / S, NACC = Moments<E, BAND>::NACC;
     float val[NACC][IT];
-    fold_subsets<E, S, NACC>(acc.s, reinterpret_cast<float *>(scr), sub, rw * 64 + lane, 64 * RW, val);
+    fold_subsets<E, S, NACC>(acc.s, reinterpret_cast<float *>(scr), sub, rw * 64 + lane, rw * 64 + lane, 64 * RW, val);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
       const int m = sub + it * S;
@@ -310,7 +311,9 @@ __global__ __launch_bounds__(wrow_threads(N, KIND)) void k_wrow(PassArgs a) {
 constexpr int wcol_subsets(int n, int kind) {
   return !is_mom(kind) || n >= 2048 ? 1 : n >= 256 ? (kind == BLK_TO_MOM5 ? 2 : 3) : 8;
 }
-constexpr int wcol_waves(int n, int kind) { return n < 256 ? 1 : n >= 1024 && !is_mom(kind) ? 8 : 4; }
+constexpr int wcol_waves(int n, int kind) {
+  return n < 256 ? 1 : kind == BLK_TO_NAT || (n >= 1024 && !is_mom(kind)) ? 8 : 4;
+}
 constexpr int wcol_threads(int n, int kind) { return 64 * wcol_waves(n, kind) * wcol_subsets(n, kind); }
 
 template <int N, int KIND, bool G = false>
@@ -394,11 +397,25 @@ __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
     }
     constexpr int IT = (E + S - 1) / S, NACC = Moments<E, BAND>::NACC;
     float val[NACC][IT];
-    fold_subsets<E, S, NACC>(acc.s, reinterpret_cast<float *>(scr), sub, wc * 64 + lane, 64 * WC, val);
+    // One column per wave: the fold hands four neighbouring columns of a row to four neighbouring
+    // lanes.  A store then touches 16 cache lines instead of 64, which had bound the pass as much
+    // as its transforms (15 planes of 1024^2: 43.5 -> 32.5 us; 10 of 2048 x 1024: 90 -> 71 us).
+    // Column c's lanes are rotated by 16 c so that the reads hit all banks.
+    constexpr bool TR = P == 1;
+    static_assert(!TR || WC == 4, "the fold pairs four columns");
+    int ln;  // opaque: keeps the fold's addresses out of registers during the transforms
+    asm volatile("v_mov_b32 %0, %1" : "=v"(ln) : "v"(threadIdx.x & 63));
+    const int rt = wc * 64 + ln, rc = rt % 4, rl = rt / 4;
+    const int t = wc * 64 + (TR ? (ln + 16 * wc) % 64 : ln);
+    fold_subsets<E, S, NACC, TR>(acc.s, reinterpret_cast<float *>(scr), sub, t, TR ? rc * 64 + (rl + 16 * rc) % 64 : t,
+                                 64 * WC, val);
+    const int sx = TR ? bt * 4 + rc : x, sl = TR ? rl : l;
+    if (sx < a.W) {
 #pragma unroll
-    for (int it = 0; it < IT; ++it) {
-      const int m = sub + it * S;
-      if (m < E && active) store_moment<NACC, IT>(a, pw, l + L * m, x, val, it);
+      for (int it = 0; it < IT; ++it) {
+        const int m = sub + it * S;
+        if (m < E) store_moment<NACC, IT>(a, pw, sl + L * m, sx, val, it);
+      }
     }
   } else {
     F::template run<false>(v, ws, twl, l);
@@ -412,21 +429,57 @@ __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
 #pragma unroll
       for (int m = 0; m < E; ++m) dst[coff + m * col_step] = v[m];
     } else {
-      if (!active) return;
-      const long long o = q0 * plane_elems + (long long)l * a.W + x, ostep = (long long)L * a.W;
-      if (a.out_mode == OUT_NAT_MAG) {
-        float *dst = reinterpret_cast<float *>(pw.out) + o;
+      const bool mag = a.out_mode == OUT_NAT_MAG;
+      if (!mag && a.post_lx) {
+        const float2 lx = a.post_lx[xl];
 #pragma unroll
-        for (int m = 0; m < E; ++m) dst[m * ostep] = sqrtf(v[m].x * v[m].x + v[m].y * v[m].y);
-      } else {
-        float2 *dst = reinterpret_cast<float2 *>(pw.out) + o;
-        if (a.post_lx) {
-          const float2 lx = a.post_lx[x];
+        for (int m = 0; m < E; ++m) v[m] = cmul(v[m], cmul(lx, a.post_ly[l + L * m]));
+      }
+      if constexpr (P == 1) {
+        // a wave's column lies one element per row in the natural layout: the block's eight columns
+        // go through the scratch, so that eight lanes store eight neighbours of one row (64
+        // single elements per store touched 64 cache lines: 15 planes of 1024^2, |X|, 95 us; 48
+        // here).  Row y of column c sits rotated by R c within the column's region: the regions are
+        // a multiple of all banks apart.
+        constexpr int CB = WC, R = 64 / CB;
+        auto rot = [](int y, int c, int r) { return y + r * c < N ? y + r * c : y + r * c - N; };
+        const int tx0 = bt * CB;
+        __builtin_amdgcn_wave_barrier();
+        if (mag) {
+          float *reg = reinterpret_cast<float *>(ws);
 #pragma unroll
-          for (int m = 0; m < E; ++m) v[m] = cmul(v[m], cmul(lx, a.post_ly[l + L * m]));
+          for (int m = 0; m < E; ++m) reg[rot(l + L * m, wc, R)] = sqrtf(v[m].x * v[m].x + v[m].y * v[m].y);
+        } else {
+#pragma unroll
+          for (int m = 0; m < E; ++m) ws[rot(l + L * m, wc, R / 2)] = v[m];
         }
+        __syncthreads();
+        const int c = tid % CB, y0 = tid / CB;
+        if (tx0 + c >= a.W) return;
+        const long long o = q0 * plane_elems + (long long)y0 * a.W + tx0 + c, ostep = (long long)(64 * WC / CB) * a.W;
+        if (mag) {
+          float *dst = reinterpret_cast<float *>(pw.out) + o;
+          const float *reg = reinterpret_cast<const float *>(scr + c * F::SCR);
 #pragma unroll
-        for (int m = 0; m < E; ++m) dst[m * ostep] = v[m];
+          for (int m = 0; m < E; ++m) dst[m * ostep] = reg[rot(y0 + 64 * m, c, R)];
+        } else {
+          float2 *dst = reinterpret_cast<float2 *>(pw.out) + o;
+          const float2 *reg = scr + c * F::SCR;
+#pragma unroll
+          for (int m = 0; m < E; ++m) dst[m * ostep] = reg[rot(y0 + 64 * m, c, R / 2)];
+        }
+      } else {
+        if (!active) return;
+        const long long o = q0 * plane_elems + (long long)l * a.W + x, ostep = (long long)L * a.W;
+        if (mag) {
+          float *dst = reinterpret_cast<float *>(pw.out) + o;
+#pragma unroll
+          for (int m = 0; m < E; ++m) dst[m * ostep] = sqrtf(v[m].x * v[m].x + v[m].y * v[m].y);
+        } else {
+          float2 *dst = reinterpret_cast<float2 *>(pw.out) + o;
+#pragma unroll
+          for (int m = 0; m < E; ++m) dst[m * ostep] = v[m];
+        }
       }
     }
   }
