@@ -180,6 +180,17 @@ __host__ __device__ constexpr int fft_twiddle_index(int n, int i) {
   return 0;
 }
 
+// One 8-byte LDS access.  Volatile, so that accesses at constant offsets are not paired into
+// ds_read2_b64 / ds_write2_b64: a pair keeps the LDS unit busy about a third longer than two single
+// accesses (2048-row column pass: 133 M against 100 M LDS cycles, waits on LDS twice as long).
+typedef float lds_f2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) volatile lds_f2 lds_vf2;
+__device__ __forceinline__ float2 lds_get(const float2 *p) {
+  const lds_f2 v = *(const lds_vf2 *)p;
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void lds_put(float2 *p, float2 x) { *(lds_vf2 *)p = lds_f2{x.x, x.y}; }
+
 template <int N> struct WaveFft {
   static constexpr int L = fft_lanes(N);
   static constexpr int P = 64 / L;  // transforms per wave
@@ -192,7 +203,13 @@ template <int N> struct WaveFft {
   static constexpr int TW = N - E;             // entries of the pass-major twiddle table
   static constexpr int TWL = TW > 0 ? TW : 1;  // elements of its LDS copy
 
-  __device__ __forceinline__ static int pad(int i) { return i + (i >> PSH); }
+  __device__ __forceinline__ static unsigned pad(unsigned i) { return i + (i >> PSH); }
+  // pad(i + c) == pad(i) + padc(c) when adding c to i carries nothing past the pad granule 2^PSH
+  // out of i's low bits: c a multiple of it, or i's low bits below a granule fraction that c is a
+  // multiple of.  With the offsets split off this way, an exchange has one address register and
+  // immediate offsets (the padded index recomputed per element had been 210 of the 690 VALU
+  // instructions of a 1024-point row).
+  static constexpr int padc(int c) { return c + (c >> PSH); }
 
   // offset of the table of the pass that starts at stride NS
   static constexpr int tw_offset(int ns) {
@@ -222,17 +239,29 @@ template <int N> struct WaveFft {
     constexpr int TOFF = tw_offset(NS);
     float2 u[PER][R];
     float2 w[PER][R];  // w[q][0] unused
+    constexpr int GR = 1 << PSH;
+    const unsigned ul = (unsigned)lane;
+    if constexpr (NB % GR == 0 && (L % GR == 0 || PER == 1)) {
+      const float2 *src = scr + pad(ul);
 #pragma unroll
-    for (int q = 0; q < PER; ++q)
+      for (int q = 0; q < PER; ++q)
 #pragma unroll
-      for (int r = 0; r < R; ++r) u[q][r] = scr[pad(lane + L * q + r * NB)];
+        for (int r = 0; r < R; ++r) u[q][r] = lds_get(src + padc(L * q + r * NB));
+    } else {
+#pragma unroll
+      for (int q = 0; q < PER; ++q)
+#pragma unroll
+        for (int r = 0; r < R; ++r) u[q][r] = lds_get(scr + pad(ul + L * q + r * NB));
+    }
+    // (ul + L q) mod NS, the division left to the cases where neither of L, NS divides the other
+    auto mod_ns = [&](int q) { return L % NS == 0 ? ul % NS : NS % L == 0 ? ul + L * q % NS : (ul + L * q) % NS; };
     // all twiddle reads issued together with the data reads, so their latencies overlap
     // instead of one LDS round trip per pair; the empty asm keeps the compiler from sinking
     // each read down to its use
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
-      for (int r = 1; r < R; ++r) w[q][r] = tw[TOFF + (r - 1) * NS + (lane + L * q) % NS];
+      for (int r = 1; r < R; ++r) w[q][r] = lds_get(tw + TOFF + (r - 1) * NS + mod_ns(q));
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
@@ -253,12 +282,22 @@ template <int N> struct WaveFft {
 #pragma unroll
         for (int r = 0; r < R; ++r) v[q + r * (E / R)] = u[q][r];
     } else {
+// butterfly j = ul + L q writes (j / NS) NS R + j % NS + r NS
+      if constexpr ((L % NS == 0 || NS % L == 0) && (GR % NS == 0 || NS % GR == 0) && NS * R % GR == 0 &&
+                    (L * R % GR == 0 || PER == 1)) {
+        float2 *dst = scr + pad(L % NS == 0 ? ul / NS * (NS * R) + ul % NS : ul);
 #pragma unroll
-      for (int q = 0; q < PER; ++q) {
-        const int j = lane + L * q;
-        const int base = (j / NS) * NS * R + j % NS;
+        for (int q = 0; q < PER; ++q)
 #pragma unroll
-        for (int r = 0; r < R; ++r) scr[pad(base + r * NS)] = u[q][r];
+          for (int r = 0; r < R; ++r)
+            lds_put(dst + padc((L % NS == 0 ? L * q * R : L * q / NS * (NS * R) + L * q % NS) + r * NS), u[q][r]);
+      } else {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+          const unsigned j = ul + L * q, base = j / NS * (NS * R) + j % NS;
+#pragma unroll
+          for (int r = 0; r < R; ++r) lds_put(scr + pad(base + r * NS), u[q][r]);
+        }
       }
       __builtin_amdgcn_wave_barrier();
       pass<NS * R, S>(v, scr, tw, lane);
@@ -279,15 +318,23 @@ template <int N> struct WaveFft {
   template <bool INV> __device__ __forceinline__ static void stage_in(float2 (&v)[E], float2 *scr, int lane) {
     constexpr int S = INV ? 1 : -1;
     RegDft<E, S>::run(v);  // pass 1: butterfly j = lane over x[lane + L r]
+    __builtin_assume(lane >= 0 && lane < L);
+    if constexpr ((1 << PSH) % E == 0) {
+      float2 *dst = scr + pad((unsigned)lane * E);
 #pragma unroll
-    for (int r = 0; r < E; ++r) scr[pad(lane * E + r)] = v[r];
+      for (int r = 0; r < E; ++r) lds_put(dst + r, v[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < E; ++r) lds_put(scr + pad((unsigned)lane * E + r), v[r]);
+    }
     __builtin_amdgcn_wave_barrier();
   }
   template <bool INV>
   __device__ __forceinline__ static void stage_out(float2 (&o)[E], float2 *scr, const float2 *tw, int lane) {
+    __builtin_assume(lane >= 0 && lane < L);
     if constexpr (N == E) {  // one lane holds the whole transform: pass 1 was all of it
 #pragma unroll
-      for (int r = 0; r < E; ++r) o[r] = scr[pad(r)];
+      for (int r = 0; r < E; ++r) o[r] = lds_get(scr + pad(r));
     } else {
       pass<E, INV ? 1 : -1>(o, scr, tw, lane);
     }

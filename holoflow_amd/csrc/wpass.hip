@@ -418,17 +418,26 @@ __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
       }
     }
   } else {
-    F::template run<false>(v, ws, twl, l);
     if constexpr (KIND == BLK_MID) {
-      asm volatile("" ::: "memory");  // keep the table loads after the forward transform
+      // the table tile loads once pass 1 has moved the column into the scratch, so its latency
+      // overlaps the remaining passes (held together by the empty asm: the compiler else sinks
+      // each load to its product)
+      F::template stage_in<false>(v, ws, l);
+      float2 tf[E];
 #pragma unroll
-      for (int m = 0; m < E; ++m) v[m] = cmul(v[m], pw.mid_tf[coff + m * col_step]);
+      for (int m = 0; m < E; ++m) tf[m] = pw.mid_tf[coff + m * col_step];
+      F::template stage_out<false>(v, ws, twl, l);
+#pragma unroll
+      for (int m = 0; m < E; ++m) asm volatile("" : "+v"(tf[m].x), "+v"(tf[m].y));
+#pragma unroll
+      for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tf[m]);
       F::template run<true>(v, ws, twl, l);
       if (!active) return;
       float2 *dst = reinterpret_cast<float2 *>(pw.out) + q0 * plane_elems;
 #pragma unroll
       for (int m = 0; m < E; ++m) dst[coff + m * col_step] = v[m];
     } else {
+      F::template run<false>(v, ws, twl, l);
       const bool mag = a.out_mode == OUT_NAT_MAG;
       if (!mag && a.post_lx) {
         const float2 lx = a.post_lx[xl];
