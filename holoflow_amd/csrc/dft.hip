@@ -352,7 +352,7 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
                 float2 c = side ? make_float2(v[t].x, -v[t].y) : v[t];
-                dst[F::pad(x0 + t)] = cmul(c, L[t]);
+                dst[F::pad(x0) + t] = cmul(c, L[t]);  // x0 is a multiple of four
               }
             }
           }
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
         float2 *ws = scr + (q - q0) * F::SCR;
         float2 v[E];
 #pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = ws[F::pad(lane + 64 * m)];
+        for (int m = 0; m < E; ++m) v[m] = lds_get(ws + F::pad(lane) + F::padc(64 * m));
         F::template run<false>(v, ws, twl, lane);
         float2 *dst = a.planes + win * a.planes_stride + (long long)q * plane_elems + row_off;
 #pragma unroll
@@ -395,33 +395,30 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
 // ----------------------------------------------------------------------- pipelined front
 // Same result as k_dft_row for a single LDS group of planes (up to FP32 rounding where the
 // DFT is folded), with the waves split by role: W/128 producer waves (8 at W = 1024) run the
-// MFMA time DFT of the block's next row into registers while four consumer waves run the row
+// MFMA time DFT of the block's next row into registers while the consumer waves run the row
 // FFTs of the current row's planes out of LDS and store them; then the producers scatter the
 // next row into LDS.  HBM loads and MFMAs of one row overlap the LDS/VALU work and the stores
 // of the previous one.
 // Producers own 128 pixels each (two 64-pixel MFMA tiles) and stream their frame loads
 // through a register ring that runs on across rows: DftStream (interleaved cos/-sin rows, up
 // to 8 bins) or DftStreamFold (9..16 bins, real-input symmetry folded).  FP32 only, for T in
-// {32, 64, 128}.  HFX_FRONT_CW / HFX_FRONT_RING override the consumer-wave count and the ring
-// depth at compile time (tuning builds; the defaults are the measured best).
+// {32, 64, 128}.
+// Consumer waves: a block has at most twelve waves where a producer holds the folded DFT's sums
+// (three per SIMD, 168 registers; a thirteenth spills: 1024^2 batch 1690 -> 1980 us), so four, six
+// and eight at 1024, 768 and 512; up to 8 bins, eight at 512 (four windows of 512^2, T = 32: 92 ->
+// 87 us) and four beyond, where eight measured 3-5 % slower.
 template <int W> constexpr int front_pw() { return W / 128; }
-#ifndef HFX_FRONT_CW
-#define HFX_FRONT_CW 4
-#endif
-template <int W> constexpr int front_cw() { return HFX_FRONT_CW; }
-template <int W> constexpr int front_threads() { return (front_pw<W>() + front_cw<W>()) * 64; }
-#ifndef HFX_FRONT_RING
-#define HFX_FRONT_RING 8
-#endif
-constexpr int front_ring(int T) { return T / 4 < HFX_FRONT_RING ? T / 4 : HFX_FRONT_RING; }
+template <int W, bool FOLD> constexpr int front_cw() { return W == 512 ? 8 : FOLD ? 12 - front_pw<W>() : 4; }
+template <int W, int NBT> constexpr int front_threads() { return (front_pw<W>() + front_cw<W, NBT == 2>()) * 64; }
+constexpr int front_ring(int T) { return T / 4 < 8 ? T / 4 : 8; }
 
 template <int W, int NBT, int MODE, int T>
-__global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
+__global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) {
   static_assert(MODE == 0, "the pipelined front kernel runs the FP32 time DFT");
   using F = WaveFft<W>;
   constexpr int TPW = 2;
   constexpr int NPW = front_pw<W>();
-  constexpr int NT = front_threads<W>();
+  constexpr int NT = (front_threads<W, NBT>());
   constexpr int E = F::E;
   constexpr int GB = row_group<W>();
   __shared__ float2 scr[GB * F::SCR];  // one padded row per plane
@@ -497,7 +494,7 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           float2 c = side ? make_float2(v[t].x, -v[t].y) : v[t];
-          dst[F::pad(x0 + t)] = cmul_rn(c, L[t]);
+          dst[F::pad(x0) + t] = cmul_rn(c, L[t]);  // x0 is a multiple of four
         }
       }
     };
@@ -545,11 +542,11 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
     const int y = row_y(i);
     float2 *planes = a.grouped ? a.planes_w[win_of(i)] : a.planes + win_of(i) * a.planes_stride;
     const long long row_off = blk_lane_offset(lane, a.H, a.blk_c) + (long long)y * a.blk_c;
-    for (int q = rw; q < a.n_planes; q += front_cw<W>()) {
+    for (int q = rw; q < a.n_planes; q += front_cw<W, FOLD>()) {
       float2 *ws = scr + q * F::SCR;
       float2 v[E];
 #pragma unroll
-      for (int m = 0; m < E; ++m) v[m] = ws[F::pad(lane + 64 * m)];
+      for (int m = 0; m < E; ++m) v[m] = lds_get(ws + F::pad(lane) + F::padc(64 * m));
       F::template run<false>(v, ws, twl, lane);
       float2 *dst = planes + (long long)q * plane_elems + row_off;
 #pragma unroll
@@ -578,6 +575,9 @@ __global__ __launch_bounds__(front_threads<W>()) void k_front(DftArgs a) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last row's unused refills land first
   } else {
+    // the row FFTs are the longer half of a row at 9..16 bins: their waves issue first (front alone
+    // 84.6 -> 75.5 us at 1024^2, 15 planes; at up to 8 bins it measured 3 % slower)
+    if constexpr (FOLD) __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       // opaque per-row lane index: keeps loop-invariant LDS addresses out of registers
@@ -711,11 +711,11 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
   const int T = a.r.T;
   if (MODE == 0 && a.n_planes <= row_group<W>() && (T == 32 || T == 64 || T == 128)) {
     if (T == 32)
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 32>), dim3(grid), dim3(front_threads<W>()), lds, st, a);
+      hipLaunchKernelGGL((k_front<W, NBT, 0, 32>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
     else if (T == 64)
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 64>), dim3(grid), dim3(front_threads<W>()), lds, st, a);
+      hipLaunchKernelGGL((k_front<W, NBT, 0, 64>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
     else
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 128>), dim3(grid), dim3(front_threads<W>()), lds, st, a);
+      hipLaunchKernelGGL((k_front<W, NBT, 0, 128>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
   } else if (a.n_planes <= row_group<W>()) {
     hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, false>), dim3(grid), dim3(row_threads<W>()), lds, st, a);
   } else {
