@@ -13,7 +13,7 @@
 //                    the result once, column-blocked, for the column pass.  The next row's
 //                    first frames are loaded while the current row is transformed.  The
 //                    band planes never make an HBM round trip in natural layout.
-//   k_front        : the FP32 form of k_dft_row with the waves split into producers (DFT)
+//   k_front        : the FP32 form of k_dft_row (T = 32, 64, 128) with the waves split into producers (DFT)
 //                    and consumers (row FFTs) that overlap across rows (the main path).
 //
 // Plane q of the output: q < nb -> bin kb+q; q >= nb (two-sided path) -> conj of computed
@@ -412,7 +412,10 @@ template <int W, bool FOLD> constexpr int front_cw() { return W == 512 ? 8 : FOL
 template <int W, int NBT> constexpr int front_threads() { return (front_pw<W>() + front_cw<W, NBT == 2>()) * 64; }
 constexpr int front_ring(int T) { return T / 4 < 8 ? T / 4 : 8; }
 
-template <int W, int NBT, int MODE, int T>
+// MULTI: the planes take several LDS groups (two-sided bands).  The producers keep a row's spectra
+// and scatter one group after the other, each as soon as the consumers are done with the previous
+// one; the next row's DFT overlaps the last group's row FFTs.
+template <int W, int NBT, int MODE, int T, bool MULTI = false>
 __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) {
   static_assert(MODE == 0, "the pipelined front kernel runs the FP32 time DFT");
   using F = WaveFft<W>;
@@ -446,6 +449,9 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
   const int y0 = xcd_tile(blockIdx.x, G);
   const int rows = a.H * a.nwin;                           // rows of all windows, window-major
   const int nr = y0 < rows ? (rows - 1 - y0) / G + 1 : 0;  // of them this block's
+  // LDS groups of planes, evenly filled
+  const int ng = MULTI ? (a.n_planes + GB - 1) / GB : 1;
+  const int gp = MULTI ? (a.n_planes + ng - 1) / ng : a.n_planes;
 
   f4 acc[TPW][NBT][4];        // interleaved rows (!FOLD)
   f4 fre[TPW][4], fim[TPW][4];  // Re and Im of bins 4 g + r (FOLD)
@@ -469,7 +475,7 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
   };
   const Band b = pinned_band(a);
   // producers: MFMA registers of row i -> padded LDS rows (its window's lens for Fresnel)
-  auto scatter = [&](int i, int lane) {
+  auto scatter = [&](int i, int q0, int lane) {  // group of planes from q0
     const int y = row_y(i);
     const float2 *lxw = a.grouped ? a.lx_w[win_of(i)] : a.lx, *lyw = a.grouped ? a.ly_w[win_of(i)] : a.ly;
     // band bin `bin` of 4 pixels from x0 into the LDS plane rows (and its conjugate plane on
@@ -490,7 +496,8 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
           if (j < 0 || j >= b.nb) continue;
           q = b.nb + j;
         }
-        float2 *dst = scr + q * F::SCR;
+        if (MULTI && (q < q0 || q >= q0 + gp)) continue;
+        float2 *dst = scr + (q - q0) * F::SCR;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           float2 c = side ? make_float2(v[t].x, -v[t].y) : v[t];
@@ -538,12 +545,13 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
   };
 
   // consumers: one wave per plane row: forward row FFT, then the column-blocked store
-  auto transform = [&](int i, int lane) {
+  auto transform = [&](int i, int q0, int lane) {
     const int y = row_y(i);
     float2 *planes = a.grouped ? a.planes_w[win_of(i)] : a.planes + win_of(i) * a.planes_stride;
     const long long row_off = blk_lane_offset(lane, a.H, a.blk_c) + (long long)y * a.blk_c;
-    for (int q = rw; q < a.n_planes; q += front_cw<W, FOLD>()) {
-      float2 *ws = scr + q * F::SCR;
+    const int q1 = MULTI ? min(q0 + gp, a.n_planes) : a.n_planes;
+    for (int q = q0 + rw; q < q1; q += front_cw<W, FOLD>()) {
+      float2 *ws = scr + (q - q0) * F::SCR;
       float2 v[E];
 #pragma unroll
       for (int m = 0; m < E; ++m) v[m] = lds_get(ws + F::pad(lane) + F::padc(64 * m));
@@ -555,22 +563,29 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
   };
 
   // The two roles run separate loops (wave-uniform branch) that meet at the same number of
-  // workgroup barriers: 1 + 2 per row.  Keeping them apart keeps the producers' MFMA
+  // workgroup barriers: 1 + 2 per row and group.  Keeping them apart keeps the producers' MFMA
   // accumulators out of the consumers' register allocation.
   if (producer) {
     const int lane0 = tid & 63;
     if (nr > 0) {
       stream.start(ring_of(0), px0(row_y(0)), lane0);
       dft_row(0, lane0);
-      scatter(0, lane0);
+      scatter(0, 0, lane0);
     }
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       int lane;
       asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
+      if constexpr (MULTI) {
+        for (int g = 1; g < ng; ++g) {
+          __syncthreads();  // consumers are done with row i's planes below group g
+          scatter(i, g * gp, lane);
+          __syncthreads();
+        }
+      }
       if (i + 1 < nr) dft_row(i + 1, lane);
       __syncthreads();  // consumers are done with row i's planes
-      if (i + 1 < nr) scatter(i + 1, lane);
+      if (i + 1 < nr) scatter(i + 1, 0, lane);
       __syncthreads();  // row i + 1's planes are in LDS
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last row's unused refills land first
@@ -580,12 +595,14 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
     if constexpr (FOLD) __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
-      // opaque per-row lane index: keeps loop-invariant LDS addresses out of registers
-      int lane;
-      asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
-      transform(i, lane);
-      __syncthreads();
-      __syncthreads();
+      for (int g = 0; g < ng; ++g) {
+        // opaque lane index: keeps loop-invariant LDS addresses out of registers
+        int lane;
+        asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
+        transform(i, g * gp, lane);
+        __syncthreads();
+        __syncthreads();
+      }
     }
   }
 }
@@ -709,13 +726,24 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
   const long long rows = (long long)a.H * a.nwin;
   const unsigned grid = (unsigned)(rows < cus ? rows : cus);
   const int T = a.r.T;
-  if (MODE == 0 && a.n_planes <= row_group<W>() && (T == 32 || T == 64 || T == 128)) {
+  // several groups need more than 8 computed bins at every width (two-sided, 16 planes or more)
+  constexpr bool CAN_MULTI = NBT == 2 && W > 512;
+  const bool multi = a.n_planes > row_group<W>();
+  if (MODE == 0 && (CAN_MULTI || !multi) && (T == 32 || T == 64 || T == 128)) {
+    const dim3 g(grid), b((front_threads<W, NBT>()));
+    auto go = [&](auto t) {
+      constexpr int TT = decltype(t)::value;
+      if (multi)
+        hipLaunchKernelGGL((k_front<W, NBT, 0, TT, CAN_MULTI>), g, b, lds, st, a);
+      else
+        hipLaunchKernelGGL((k_front<W, NBT, 0, TT>), g, b, lds, st, a);
+    };
     if (T == 32)
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 32>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
+      go(std::integral_constant<int, 32>{});
     else if (T == 64)
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 64>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
+      go(std::integral_constant<int, 64>{});
     else
-      hipLaunchKernelGGL((k_front<W, NBT, 0, 128>), dim3(grid), dim3((front_threads<W, NBT>())), lds, st, a);
+      go(std::integral_constant<int, 128>{});
   } else if (a.n_planes <= row_group<W>()) {
     hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, false>), dim3(grid), dim3(row_threads<W>()), lds, st, a);
   } else {
