@@ -8,6 +8,8 @@
 //                Fresnel); BLK_TO_MOM5 also makes the two band-split M0 images
 //   BLK_MID    : column-blocked -> forward, times the transfer function, inverse ->
 //                column-blocked in place                                      (column pass)
+//   BLK_LENS   : column-blocked -> inverse, times the Fresnel lens, forward -> column-blocked in
+//                place (row pass between Filter2D's spectrum and the propagation's)
 //   BLK_TO_NAT : column-blocked -> transform -> natural complex (optionally times the
 //                output lens), natural |X| or natural real part
 //
@@ -32,12 +34,12 @@ namespace hfx {
 
 namespace {
 
-enum Kind { NAT_TO_BLK = 0, BLK_TO_MOM = 1, BLK_MID = 2, BLK_TO_NAT = 3, BLK_TO_MOM5 = 4 };
+enum Kind { NAT_TO_BLK = 0, BLK_TO_MOM = 1, BLK_MID = 2, BLK_TO_NAT = 3, BLK_TO_MOM5 = 4, BLK_LENS = 5 };
 constexpr bool is_mom(int k) { return k == BLK_TO_MOM || k == BLK_TO_MOM5; }
 // Transform direction each kind is compiled for: the row pass out of natural data is
 // forward (it feeds the column pass), the row passes that read the blocked spectrum back
 // (angular spectrum) are inverse, and every column pass is forward (BLK_MID runs forward,
-// transfer function, inverse).  The launchers reject a PassArgs::inv that disagrees.
+// transfer function, inverse; BLK_LENS starts inverse).  The launchers reject a PassArgs::inv that disagrees.
 constexpr bool row_inv(int k) { return k != NAT_TO_BLK; }
 
 // Running sums of one lane's E pixels: a, f a, f^2 a; with a band split, sum 0 holds the planes
@@ -283,8 +285,14 @@ __global__ __launch_bounds__(wrow_threads(N, KIND)) void k_wrow(PassArgs a) {
     F::template stage_in<row_inv(KIND)>(v, ws, l);
     float2 o[E];
     F::template stage_out<row_inv(KIND)>(o, ws, twl, l);
+    if constexpr (KIND == BLK_LENS) {
+      const float2 ly = a.pre_ly[yl];
+#pragma unroll
+      for (int m = 0; m < E; ++m) o[m] = cmul(o[m], cmul(a.pre_lx[l + L * m], ly));
+      F::template run<false>(o, ws, twl, l);
+    }
     if (!active) return;
-    if constexpr (KIND == NAT_TO_BLK) {
+    if constexpr (KIND == NAT_TO_BLK || KIND == BLK_LENS) {
       float2 *dst = reinterpret_cast<float2 *>(pw.out) + q0 * plane_elems;
 #pragma unroll
       for (int m = 0; m < E; ++m) dst[blk(m)] = o[m];
@@ -567,6 +575,7 @@ int launch_row_pass(const PassArgs &a, hipStream_t st) {
   }
   if (a.out_mode == OUT_MOMENTS)
     return a.mom.split > 0 ? wrow_dispatch<BLK_TO_MOM5>(a, st) : wrow_dispatch<BLK_TO_MOM>(a, st);
+  if (a.out_mode == OUT_BLK && a.pre_lx) return wrow_dispatch<BLK_LENS>(a, st);
   if ((a.out_mode == OUT_NAT_C && !a.post_lx) || a.out_mode == OUT_NAT_RE) return wrow_dispatch<BLK_TO_NAT>(a, st);
   return -4;
 }
