@@ -4,7 +4,7 @@
 //                    (optionally times the Fresnel lens; negative-band conjugate planes for
 //                    the two-sided FFT path).  Used for the per-stage entry point and for
 //                    widths the fused kernels do not cover.
-//   k_dft_fold     : the same for FP32 with 9..64 bins and T % 32 == 0, with the real-input
+//   k_dft_fold     : the same for FP32 with 9..64 bins, with the real-input
 //                    symmetry folded into the contraction (about half the MFMAs).
 //   k_dft_row      : fused time DFT + forward row FFT.  A persistent workgroup walks a
 //                    set of image rows; for each row its waves (64 or 128 pixels each) keep
@@ -182,8 +182,8 @@ __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
 }
 
 // FP32 stand-alone time DFT with the real-input symmetry folded (dft_fold_tile): NBF tiles of
-// 16 bins per wave (all of the band's tiles: every frame sample is loaded by one wave only),
-// T % 32 == 0.  Same outputs as k_dft<NBT, 0> up to FP32 rounding, with 2 (T/8) + 1 MFMAs per
+// 16 bins per wave (all of the band's tiles: every frame sample is loaded by one wave only).
+// Same outputs as k_dft<NBT, 0> up to FP32 rounding, with 2 (T/8) + 1 MFMAs per
 // 16 bins and 16 pixels instead of T/2.
 // Persistent like k_dft.  The second launch bound (resident blocks per CU) makes the compiler
 // keep the accumulators in ordinary registers instead of splitting them off into accumulation
@@ -684,8 +684,11 @@ template <int NBF> static int launch_fold(const DftArgs &a, hipStream_t st) {
 int launch_time_dft(const DftLaunch &L, hipStream_t st) {
   if (L.nwin > HFX_MAX_WIN) return -6;
   const DftArgs a = make_args(L);
-  // FP32 with more than one 16-row tile of interleaved rows: the folded contraction
-  if (L.precision == 0 && L.T % 32 == 0 && L.nbc > 8 && L.nbc <= 64) {
+  // FP32 with more than one 16-row tile of interleaved rows: the folded contraction.  Its last batch
+  // of steps may be cut short, so any T % 4 == 0 runs (512 x 768, T = 48, 12 bins: 29.6 us with k_dft,
+  // 20.5 folded); longer windows that are no multiple of 32 stay on k_dft, whose larger operand
+  // matrix sets the window lengths that such a band accepts.
+  if (L.precision == 0 && (L.T % 32 == 0 || L.T <= 256) && L.nbc > 8 && L.nbc <= 64) {
     switch ((L.nbc + 15) / 16) {
       case 1: return launch_fold<1>(a, st);
       case 2: return launch_fold<2>(a, st);

@@ -342,6 +342,10 @@ template <int NBT, int TPW, int T, int K> struct DftStream {
   }
 };
 
+// Pitch of the folded operand matrix: 4 beyond a multiple of 16 floats, so that the 16 rows x 4
+// K-slots of one step hit 64 distinct banks (T/2 + 4 where 32 divides T).
+__host__ __device__ constexpr int fold_pitch(int T) { return (T / 2 + 15) / 16 * 16 + 4; }
+
 // FP32 time DFT of one 16-bin tile with the real-input symmetry folded in (T even):
 //   Re X_k = x_0 + (-1)^k x_{T/2} + sum_{p=1}^{T/2-1} (x_p + x_{T-p}) cos(2 pi k p / T)
 //   Im X_k =                      - sum_{p=1}^{T/2-1} (x_p - x_{T-p}) sin(2 pi k p / T)
@@ -357,7 +361,7 @@ template <int NBT, int TPW, int T, int K> struct DftStream {
 // the next row as in DftStream.
 template <int TPW, int T, int K> struct DftStreamFold {
   static constexpr int STEPS = T / 8;
-  static constexpr int PC = T / 2 + 4;  // pitch: 16 rows x 4 K-slots hit 64 distinct banks
+  static constexpr int PC = fold_pitch(T);
   static_assert(STEPS % K == 0, "ring depth must divide the steps of a row");
   uint2 ring[K][TPW][2];
 
@@ -436,12 +440,13 @@ template <int TPW, int T, int K> struct DftStreamFold {
 };
 
 // Runtime-T form of the folded FP32 time DFT (see DftStreamFold) for NBF 16-bin tiles and one
-// 64-pixel tile per wave (stand-alone time DFT): steps of four frame pairs in batches of K,
-// T % (8 K) == 0.  Operand matrix from stage_fold_matrix_rt (NBF tiles) with pitch T/2 + 4.
+// 64-pixel tile per wave (stand-alone time DFT), T % 4 == 0: steps of four frame pairs in batches
+// of K, the last batch cut where the steps end.  Operand matrix from stage_fold_matrix_rt (NBF
+// tiles).
 template <int NBF, int K = 4>
 __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds, long long p0w, int lane,
                                               f4 (&ac)[NBF][4], f4 (&as)[NBF][4]) {
-  const int T = r.T, steps = T / 8, PC = T / 2 + 4;
+  const int T = r.T, steps = (T / 2 + 2) / 4, PC = fold_pitch(T);  // ceil((T/2 - 1) / 4) steps
   const float *lc = lds, *ls = lds + 16 * NBF * PC, *lx = lds + 32 * NBF * PC;
   const int g = lane >> 4, rw = lane & 15;
   const long long p0 = dft_px(r, p0w, lane, 0);
@@ -455,7 +460,7 @@ __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds
   const uint2 xe = dft_load4(r, ring_frame(r, g == 0 ? 0 : T / 2), p0);  // x_0, x_{T/2}
   uint2 ring[K][2];
   auto load = [&](int st, int k) {
-    const int p = 4 * st + g + 1;
+    const int p = min(4 * st + g + 1, T / 2);  // pairs past the last one: any frame, zero weights or no step
     ring[k][0] = dft_load4(r, ring_frame(r, p), p0);
     ring[k][1] = dft_load4(r, ring_frame(r, T - p), p0);
   };
@@ -495,7 +500,8 @@ __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds
     for (int k = 0; k < K; ++k) step(s0 + k, k, std::true_type{});
   }
 #pragma unroll
-  for (int k = 0; k < K; ++k) step(s0 + k, k, std::false_type{});
+  for (int k = 0; k < K; ++k)
+    if (s0 + k < steps) step(s0 + k, k, std::false_type{});
   float x[4];
   unpack4(xe, x);
 #pragma unroll
@@ -509,10 +515,10 @@ __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds
 // Operand matrix of the folded DFT (DftStreamFold, dft_fold_tile) from the interleaved rows
 // wm[2b][n] = cos, wm[2b+1][n] = -sin (b < nbc): for nbf tiles of 16 bins, a cos block
 // C[b][p-1] and a sin block S[b][p-1] for the pairs p = 1 .. T/2-1 (zero beyond and for bins
-// >= nbc), pitch T/2 + 4, then X[b] = (cos 0, cos(pi k), 0, 0) for x_0, x_{T/2}.
+// >= nbc), pitch fold_pitch(T), then X[b] = (cos 0, cos(pi k), 0, 0) for x_0, x_{T/2}.
 __device__ __forceinline__ void stage_fold_matrix_rt(float *l, const float *wm, int T, int nbf, int nbc, int tid,
                                                      int nthreads) {
-  const int PC = T / 2 + 4, rows = 16 * nbf;
+  const int PC = fold_pitch(T), rows = 16 * nbf;
   for (int i = tid; i < rows * PC; i += nthreads) {
     const int b = i / PC, j = i % PC;
     const bool in = b < nbc && j < T / 2 - 1;
@@ -528,7 +534,7 @@ __device__ __forceinline__ void stage_fold_matrix_rt(float *l, const float *wm, 
 }
 
 __host__ __device__ constexpr size_t dft_fold_lds_bytes(int nbf, int T) {
-  return (size_t)nbf * (32 * (T / 2 + 4) + 64) * 4;
+  return (size_t)nbf * (32 * fold_pitch(T) + 64) * 4;
 }
 
 }  // namespace hfx
