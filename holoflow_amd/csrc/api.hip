@@ -563,6 +563,8 @@ static hfx_status windows_back(hfx_plan *p, const Windows &ws, hipStream_t st) {
   } else {
     c.planes = ws.n * p->n_planes;
     c.mid_tf = p->tf;
+    c.row0 = (p->OH - p->H) / 2;
+    c.row1 = c.row0 + p->H;
     c.out = planes;
     c.out_mode = hfx::OUT_BLK;
     if (hfx::launch_col_pass(c, st) != 0) return fail(HFX_E_HIP, "column pass launch failed");
@@ -898,6 +900,8 @@ hfx_status hfx_asm_execute(hfx_asm *a, const void *in, void *out, hfx_stream_t s
   r.tw = a->tw_w;
   if (hfx::launch_row_pass(r, st) != 0) return fail(HFX_E_HIP, "row pass launch failed");
   hfx::PassArgs c = base_pass(a->OH, a->OW, B, a->blk_c);
+  c.row0 = r.off_y;
+  c.row1 = r.off_y + r.in_h;
   c.in = a->ws;
   c.in_mode = hfx::IN_BLK;
   c.mid_tf = a->tf;

@@ -99,7 +99,9 @@ struct PassArgs {
   const void *in;
   int in_mode;
   int in_h, in_w;           // input plane dims (== H, W unless zero-padded)
-  int off_y, off_x;         // centred padding offsets
+  int off_y, off_x;         // centred padding offsets; a row pass writes the input's rows only
+  int row0, row1;           // column pass with mid_tf: rows written by that row pass, the others
+                            // taken as zeros (row1 == 0: all rows)
   const float2 *pre_lx, *pre_ly;  // lens applied to the input (row pass) or null
   // column pass: multiply by a blocked table between forward and inverse column FFTs
   const float2 *mid_tf;
