@@ -190,6 +190,8 @@ __device__ __forceinline__ float2 lds_get(const float2 *p) {
   return make_float2(v.x, v.y);
 }
 __device__ __forceinline__ void lds_put(float2 *p, float2 x) { *(lds_vf2 *)p = lds_f2{x.x, x.y}; }
+typedef volatile __attribute__((address_space(3))) float lds_vf1;
+__device__ __forceinline__ void lds_put(float *p, float x) { *(lds_vf1 *)p = x; }
 
 template <int N> struct WaveFft {
   static constexpr int L = fft_lanes(N);

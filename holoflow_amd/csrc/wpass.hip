@@ -42,6 +42,11 @@ constexpr bool is_mom(int k) { return k == BLK_TO_MOM || k == BLK_TO_MOM5; }
 // transfer function, inverse; BLK_LENS starts inverse).  The launchers reject a PassArgs::inv that disagrees.
 constexpr bool row_inv(int k) { return k != NAT_TO_BLK; }
 
+__device__ __forceinline__ float magnitude(float2 v, bool power2) {
+  const float a = sq_mag(v);
+  return power2 ? a : mag_sqrt(a);
+}
+
 // Running sums of one lane's E pixels: a, f a, f^2 a; with a band split, sum 0 holds the planes
 // below the split and sum 3 those from it on (M0 is their sum).
 template <int E, bool BAND> struct Moments {
@@ -57,13 +62,12 @@ template <int E, bool BAND> struct Moments {
   // (wave-uniform scalar loads) so that their latency is not paid after the transform
   template <bool HI> __device__ __forceinline__ void add(const float2 (&v)[E], float f, float f2, bool power2) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) {
-      float a = sq_mag(v[m]);
-      if (!power2) a = mag_sqrt(a);
-      s[HI ? 3 : 0][m] += a;
-      s[1][m] += __fmul_rn(f, a);
-      s[2][m] += __fmul_rn(f2, a);
-    }
+    for (int m = 0; m < E; ++m) add_mag<HI>(m, magnitude(v[m], power2), f, f2);
+  }
+  template <bool HI> __device__ __forceinline__ void add_mag(int m, float a, float f, float f2) {
+    s[HI ? 3 : 0][m] += a;
+    s[1][m] += __fmul_rn(f, a);
+    s[2][m] += __fmul_rn(f2, a);
   }
 };
 
@@ -165,15 +169,33 @@ __device__ __forceinline__ void store_moment(const PassArgs &a, const PassWin &p
 // leave no register room.  Short transforms take one wave per block, so that a small image still
 // reaches many CUs.
 //
-// Plane subsets of the moment kinds (S): below 256 points eight waves take one subset each (a
-// 64 x 64 window's moment pass: 14.7 -> 4.6 us against one wave for all planes).  From 256 points
-// on one wave sums all planes of its row, the next plane's row loading meanwhile: splitting them
-// over two to four waves makes a lone 512 x 512 window's pass faster (10.5 -> 8.6 us) and that of
-// four windows slower (17.6 -> 19.5 us), and the split may not depend on the launch, since a
-// window's result does not.
-constexpr int wrow_subsets(int n, int kind) { return is_mom(kind) && n < 256 ? 8 : 1; }
-constexpr int wrow_waves(int n, int kind) { return n < 256 ? 1 : n >= (is_mom(kind) ? 4096 : 1024) ? 8 : 4; }
-constexpr int wrow_threads(int n, int kind) { return 64 * wrow_waves(n, kind) * wrow_subsets(n, kind); }
+// Planes over waves in the moment kinds (S waves per row).  Below 256 points eight waves sum one
+// subset of the planes each, folded at the end (a 64 x 64 window's moment pass: 14.7 -> 4.6 us
+// against one wave for all planes).  From 256 points on the sums run over the planes in order,
+// so that they do not depend on the launch: either one wave does all planes of its row, or, with
+// SPLIT, S waves transform S planes at a time, hand their magnitudes over through LDS, and each
+// adds up its share of the row's elements.  That takes one row per block up to 1024 points (the
+// waves of a row wait for each other only, and a few hundred rows still reach every CU), and
+// eight waves per block at 2048, where a block fills the CU.
+//
+// Launches of fewer than 1024 rows split: one wave per row leaves most SIMDs empty there, from
+// 1024 on it does not and the exchange only costs.  Inverse row pass with the column pass before
+// it, one wave per row -> split: 512 x 512, 7 planes 26.3 -> 23.3 us; 512 x 768, 12 planes 47.4 ->
+// 37.5; 512 x 1024, 15 planes 66.2 -> 56.0; 768 x 1024, 12 planes 70.1 -> 68.3; 512 x 2048, 12 planes
+// 109 -> 98.5; 1024 x 1024, 15 planes 101.6 -> 104.3; 2048 x 2048, 52 planes 1673 -> 1735.
+constexpr bool wrow_splits(long long rows) { return rows < 1024; }
+constexpr int wrow_subsets(int n, int kind, bool split) {
+  if (!is_mom(kind)) return 1;
+  return n < 256 ? 8 : !split ? 1 : n >= 2048 && kind == BLK_TO_MOM ? 2 : 4;
+}
+constexpr int wrow_waves(int n, int kind, bool split) {
+  if (n < 256) return 1;
+  if (!is_mom(kind)) return n >= 1024 ? 8 : 4;
+  return !split ? 4 : n >= 2048 ? 8 / wrow_subsets(n, kind, true) : 1;
+}
+constexpr int wrow_threads(int n, int kind, bool split) {
+  return 64 * wrow_waves(n, kind, split) * wrow_subsets(n, kind, split);
+}
 
 // IN (NAT_TO_BLK only): 1 = the input is a complex plane of the output's size with no lens, so a
 // row loads from one base address with no per-element bounds checks or index products; 2 = the
@@ -181,11 +203,11 @@ constexpr int wrow_threads(int n, int kind) { return 64 * wrow_waves(n, kind) * 
 // input plane are not computed: the column pass takes them as zeros (k_wcol, PADDED).  512 x 768
 // padded to 768 x 1024, 12 planes: row pass 28.6 -> 20.8 us against transforming all rows through the
 // general load, column pass 47.7 -> 44.0.
-template <int N, int KIND, bool G = false, int IN = 0>
-__global__ __launch_bounds__(wrow_threads(N, KIND)) void k_wrow(PassArgs a) {
+template <int N, int KIND, bool G = false, int IN = 0, bool SPLIT = false>
+__global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs a) {
   using F = WaveFft<N>;
   constexpr int E = F::E, L = F::L, P = F::P;
-  constexpr int RW = wrow_waves(N, KIND), S = wrow_subsets(N, KIND);
+  constexpr int RW = wrow_waves(N, KIND, SPLIT), S = wrow_subsets(N, KIND, SPLIT);
   __shared__ __align__(16) float2 scr[RW * S * P * F::SCR];
   __shared__ __align__(16) float2 twl[F::TWL];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -260,7 +282,52 @@ __global__ __launch_bounds__(wrow_threads(N, KIND)) void k_wrow(PassArgs a) {
   __syncthreads();
   if constexpr (N >= 2048) load(v, q0);
 
-  if constexpr (is_mom(KIND)) {
+  if constexpr (is_mom(KIND) && SPLIT) {
+    static_assert(P == 1 && E % S == 0, "a wave's share of the elements");
+    constexpr bool BAND = KIND == BLK_TO_MOM5;
+    constexpr int ES = E / S, NACC = Moments<ES, BAND>::NACC;
+    Moments<ES, BAND> acc;
+    acc.zero();
+    // the magnitudes of a wave's plane, in its own scratch
+    float *own = reinterpret_cast<float *>(ws);
+    const float *mine = reinterpret_cast<const float *>(scr + rw * F::SCR) + sub * ES * L + l;
+    for (int qb = 0; qb < a.planes; qb += S) {
+      float f[S], f2[S];
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        f[j] = a.mom.f[min(qb + j, a.planes - 1)];
+        f2[j] = a.mom.f2[min(qb + j, a.planes - 1)];
+      }
+      F::template stage_in<row_inv(KIND)>(v, ws, l);
+      load(v, min(qb + sub + S, a.planes - 1));  // as below; past the last plane: unused
+      float2 o[E];
+      F::template stage_out<row_inv(KIND)>(o, ws, twl, l);
+      float mag[E];
+#pragma unroll
+      for (int m = 0; m < E; ++m) mag[m] = magnitude(o[m], a.mom.power2);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int m = 0; m < E; ++m) lds_put(own + l + L * m, mag[m]);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        if (qb + j >= a.planes) break;
+        const float *from = mine + j * RW * F::SCR * 2;
+        if (BAND && qb + j >= a.mom.split) {
+#pragma unroll
+          for (int m = 0; m < ES; ++m) acc.template add_mag<BAND>(m, from[L * m], f[j], f2[j]);
+        } else {
+#pragma unroll
+          for (int m = 0; m < ES; ++m) acc.template add_mag<false>(m, from[L * m], f[j], f2[j]);
+        }
+      }
+      __syncthreads();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // an unused last refill lands first
+    if (!active) return;
+#pragma unroll
+    for (int m = 0; m < ES; ++m) store_moment<NACC, ES>(a, pw, y, l + L * (sub * ES + m), acc.s, m);
+  } else if constexpr (is_mom(KIND)) {
     constexpr bool BAND = KIND == BLK_TO_MOM5;
     Moments<E, BAND> acc;
     acc.zero();
@@ -548,13 +615,22 @@ bool col_pass_supported(int H, int blk_c) { return row_pass_supported(H) && blk_
 
 template <int N, int KIND> static int launch_wrow_n(const PassArgs &a, hipStream_t st) {
   if ((a.inv != 0) != row_inv(KIND)) return -5;
-  constexpr int rows = wrow_waves(N, KIND) * WaveFft<N>::P;
+  constexpr bool CAN_SPLIT = is_mom(KIND) && N >= 256;
   const int h = KIND == NAT_TO_BLK ? a.in_h : a.H;
-  const dim3 grid((unsigned)((h + rows - 1) / rows), is_mom(KIND) ? 1u : (unsigned)a.planes,
-                  (unsigned)(a.nwin > 1 ? a.nwin : 1));
-  const dim3 block(wrow_threads(N, KIND));
-  if (a.grouped) {
-    hipLaunchKernelGGL((k_wrow<N, KIND, is_mom(KIND)>), grid, block, 0, st, a);
+  const unsigned nz = (unsigned)(a.nwin > 1 ? a.nwin : 1);
+  const bool split = CAN_SPLIT && wrow_splits((long long)a.H * nz);
+  const int rows = (split ? wrow_waves(N, KIND, CAN_SPLIT) : wrow_waves(N, KIND, false)) * WaveFft<N>::P;
+  const dim3 grid((unsigned)((h + rows - 1) / rows), is_mom(KIND) ? 1u : (unsigned)a.planes, nz);
+  const dim3 block(split ? wrow_threads(N, KIND, CAN_SPLIT) : wrow_threads(N, KIND, false));
+  if constexpr (is_mom(KIND)) {
+    if (a.grouped && split)
+      hipLaunchKernelGGL((k_wrow<N, KIND, true, 0, CAN_SPLIT>), grid, block, 0, st, a);
+    else if (a.grouped)
+      hipLaunchKernelGGL((k_wrow<N, KIND, true>), grid, block, 0, st, a);
+    else if (split)
+      hipLaunchKernelGGL((k_wrow<N, KIND, false, 0, CAN_SPLIT>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_wrow<N, KIND>), grid, block, 0, st, a);
   } else if constexpr (KIND == NAT_TO_BLK) {
     const bool cplx = a.in_mode == IN_NAT_C, full = a.in_h == a.H && a.in_w == a.W && a.off_x == 0 && a.off_y == 0;
     if (cplx && full && a.pre_lx == nullptr)
