@@ -332,6 +332,11 @@ __global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs 
     Moments<E, BAND> acc;
     acc.zero();
     int q = sub;
+    // Waves of a block load at the same time where a CU holds two blocks or more: four rows share
+    // every cache line of the blocked planes, and waves that drift apart over the planes fetch it
+    // more than once (2048 x 1024, 15 planes with the column pass before it: 224 -> 210 us; a CU with
+    // one block has nothing to run while its waves wait, 1024 x 1024: 102.5 -> 104.9)
+    const bool in_step = gridDim.x * gridDim.z >= 512;
     // (the band split as two loops: fewer sums are live at a time)
     auto run_planes = [&](int end, auto hi) {
       for (; q < end; q += S) {
@@ -340,6 +345,8 @@ __global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs 
         // the next plane's row is loaded once pass 1 has moved this one into the scratch, so its
         // latency overlaps the remaining passes; the load is unconditional (the last one reloads
         // the last plane, unused), which keeps it out of a branch
+        if constexpr (N >= 256 && N <= 1024)
+          if (in_step) __syncthreads();
         load(v, q + S < a.planes ? q + S : q);
         float2 o[E];
         F::template stage_out<row_inv(KIND)>(o, ws, twl, l);
@@ -404,8 +411,15 @@ constexpr int wcol_waves(int n, int kind) {
 }
 constexpr int wcol_threads(int n, int kind) { return 64 * wcol_waves(n, kind) * wcol_subsets(n, kind); }
 
+// LOOP (BLK_MID): 2048-row columns, where a block fills the CU, so that nothing else runs while it
+// starts, loads its first columns and drains: 256 blocks stay and walk the (tile, plane) items, each
+// loading its next column behind the inverse transform and the stores of this one.  The waves load
+// in step, since four columns share every cache line (without the barrier they drift apart and the
+// pass is slower than one item per block: 1.9 ms).  52 planes of 2048^2 with the moment pass behind
+// it: 1677 -> 1596 us.  At 1024 rows and below, where blocks share a CU, one item per block is
+// faster (28 planes of 1024^2 with the moment pass: 169 against 176).
 // PADDED (BLK_MID): only the rows [row0, row1) of the input were written; the others are zero.
-template <int N, int KIND, bool G = false, bool PADDED = false>
+template <int N, int KIND, bool G = false, bool PADDED = false, bool LOOP = false>
 __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
   using F = WaveFft<N>;
   constexpr int E = F::E, L = F::L, P = F::P;
@@ -429,8 +443,17 @@ __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
   // run plane-fastest (block = tile * planes + plane, in contiguous runs per XCD): the planes
   // of one tile are in flight together on one XCD and read the table tile from its L2,
   // instead of the whole table streaming from memory once per plane.
-  int bt, bp;
-  if constexpr (KIND == BLK_MID) {
+  int bt, bp, item = 0, item_end = 0;
+  if constexpr (LOOP) {
+    // one eighth of the items to each XCD, whose blocks walk it side by side
+    const long long items = (long long)((a.W + WC * P - 1) / (WC * P)) * a.planes;
+    const int xcd = blockIdx.x % 8;
+    item = (int)(items * xcd / 8) + blockIdx.x / 8;
+    item_end = (int)(items * (xcd + 1) / 8);
+    if (item >= item_end) return;
+    bt = item / a.planes;
+    bp = item - bt * a.planes;
+  } else if constexpr (KIND == BLK_MID) {
     const int b = xcd_tile(blockIdx.x, gridDim.x);
     bt = b / a.planes;
     bp = b - bt * a.planes;
@@ -476,7 +499,45 @@ __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
   __syncthreads();
   if constexpr (EARLY && N >= 2048) load(v, q0);
 
-  if constexpr (is_mom(KIND)) {
+  if constexpr (LOOP) {
+    static_assert(KIND == BLK_MID && P == 1 && !PADDED && !G, "full columns, one per wave");
+    const int nloc = gridDim.x / 8;
+    const float2 *in = reinterpret_cast<const float2 *>(pw.in);
+    float2 *out = reinterpret_cast<float2 *>(pw.out);
+    const long long lane_off = (long long)l * C;
+    // column bt * WC + wc of plane bp; C divides the tile's columns
+    long long co = coff, po = (long long)bp * plane_elems;
+    for (;;) {
+      F::template stage_in<false>(v, ws, l);
+      float2 tf[E];
+#pragma unroll
+      for (int m = 0; m < E; ++m) tf[m] = pw.mid_tf[co + m * col_step];
+      F::template stage_out<false>(v, ws, twl, l);
+#pragma unroll
+      for (int m = 0; m < E; ++m) asm volatile("" : "+v"(tf[m].x), "+v"(tf[m].y));
+#pragma unroll
+      for (int m = 0; m < E; ++m) v[m] = cmul(v[m], tf[m]);
+      F::template stage_in<true>(v, ws, l);
+      // the next item's column loads behind this one's inverse transform and its stores; the last
+      // one loads its own column again, unused
+      __syncthreads();  // the block's waves load in step
+      const bool more = item + nloc < item_end;
+      item += more ? nloc : 0;
+      const int nt = item / a.planes, np = item - nt * a.planes;
+      const int nx = min(nt * WC + wc, a.W - 1);
+      const long long nco = blk_lane_offset(nx, a.H, C) + lane_off, npo = (long long)np * plane_elems;
+#pragma unroll
+      for (int m = 0; m < E; ++m) v[m] = in[npo + nco + m * col_step];
+      float2 o[E];
+      F::template stage_out<true>(o, ws, twl, l);
+#pragma unroll
+      for (int m = 0; m < E; ++m) out[po + co + m * col_step] = o[m];
+      if (!more) break;
+      co = nco;
+      po = npo;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the unused last load lands first
+  } else if constexpr (is_mom(KIND)) {
     constexpr bool BAND = KIND == BLK_TO_MOM5;
     Moments<E, BAND> acc;
     acc.zero();
@@ -655,12 +716,16 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
   const dim3 grid(KIND == BLK_MID ? tiles * (unsigned)a.planes : tiles,
                   is_mom(KIND) || KIND == BLK_MID ? 1u : (unsigned)a.planes, (unsigned)(a.nwin > 1 ? a.nwin : 1));
   const dim3 block(wcol_threads(N, KIND));
+  constexpr bool CAN_LOOP = KIND == BLK_MID && N >= 2048;
+  constexpr unsigned MID_BLOCKS = 256;  // one per CU
   const bool padded = a.row1 > a.row0 && (a.row0 > 0 || a.row1 < a.H);
   if (padded && KIND != BLK_MID) return -4;
   if (a.grouped)
     hipLaunchKernelGGL((k_wcol<N, KIND, KIND != BLK_TO_NAT>), grid, block, 0, st, a);
   else if (padded)
     hipLaunchKernelGGL((k_wcol<N, KIND, false, KIND == BLK_MID>), grid, block, 0, st, a);
+  else if (CAN_LOOP && a.W % cols == 0 && a.nwin <= 1 && grid.x >= 4 * MID_BLOCKS)
+    hipLaunchKernelGGL((k_wcol<N, KIND, false, false, CAN_LOOP>), dim3(MID_BLOCKS), block, 0, st, a);
   else
     hipLaunchKernelGGL((k_wcol<N, KIND>), grid, block, 0, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
