@@ -178,12 +178,16 @@ __device__ __forceinline__ void store_moment(const PassArgs &a, const PassWin &p
 // waves of a row wait for each other only, and a few hundred rows still reach every CU), and
 // eight waves per block at 2048, where a block fills the CU.
 //
-// Launches of fewer than 1024 rows split: one wave per row leaves most SIMDs empty there, from
-// 1024 on it does not and the exchange only costs.  Inverse row pass with the column pass before
-// it, one wave per row -> split: 512 x 512, 7 planes 26.3 -> 23.3 us; 512 x 768, 12 planes 47.4 ->
-// 37.5; 512 x 1024, 15 planes 66.2 -> 56.0; 768 x 1024, 12 planes 70.1 -> 68.3; 512 x 2048, 12 planes
-// 109 -> 98.5; 1024 x 1024, 15 planes 101.6 -> 104.3; 2048 x 2048, 52 planes 1673 -> 1735.
-constexpr bool wrow_splits(long long rows) { return rows < 1024; }
+// Launches of few rows split: one wave per row leaves most SIMDs empty there.  The more rows, the
+// more planes it takes to win back the rounds that S planes do not fill; from 1024 rows on the
+// chip is full without it.  Row pass, one wave per row -> split: 256 x 512 with 1, 4, 16 planes 5.0 ->
+// 4.5, 7.6 -> 5.1, 18.8 -> 10.0 us; 512 x 1024 with 1, 3, 5, 16 planes 7.6 -> 7.9, 12.3 -> 9.6, 16.7 ->
+// 13.7, 37.4 -> 24.7; 768 x 768 with 5, 8, 16 planes 15.4 -> 16.2, 20.5 -> 17.6, 34.4 -> 28.2; 512 x 2048
+// with 2, 5, 16 planes 20.1 -> 16.0, 34.4 -> 31.6, 79.1 -> 65.1; 1024 x 1024 with 5, 16 planes 18.5 ->
+// 21.9, 39.6 -> 39.9.
+constexpr bool wrow_splits(long long rows, int planes) {
+  return rows <= 256 || (rows <= 512 && planes >= 3) || (rows < 1024 && planes >= 8);
+}
 constexpr int wrow_subsets(int n, int kind, bool split) {
   if (!is_mom(kind)) return 1;
   return n < 256 ? 8 : !split ? 1 : n >= 2048 && kind == BLK_TO_MOM ? 2 : 4;
@@ -679,7 +683,7 @@ template <int N, int KIND> static int launch_wrow_n(const PassArgs &a, hipStream
   constexpr bool CAN_SPLIT = is_mom(KIND) && N >= 256;
   const int h = KIND == NAT_TO_BLK ? a.in_h : a.H;
   const unsigned nz = (unsigned)(a.nwin > 1 ? a.nwin : 1);
-  const bool split = CAN_SPLIT && wrow_splits((long long)a.H * nz);
+  const bool split = CAN_SPLIT && wrow_splits((long long)a.H * nz, a.planes);
   const int rows = (split ? wrow_waves(N, KIND, CAN_SPLIT) : wrow_waves(N, KIND, false)) * WaveFft<N>::P;
   const dim3 grid((unsigned)((h + rows - 1) / rows), is_mom(KIND) ? 1u : (unsigned)a.planes, nz);
   const dim3 block(split ? wrow_threads(N, KIND, CAN_SPLIT) : wrow_threads(N, KIND, false));
