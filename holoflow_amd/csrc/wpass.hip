@@ -336,11 +336,6 @@ __global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs 
     Moments<E, BAND> acc;
     acc.zero();
     int q = sub;
-    // Waves of a block load at the same time where a CU holds two blocks or more: four rows share
-    // every cache line of the blocked planes, and waves that drift apart over the planes fetch it
-    // more than once (2048 x 1024, 15 planes with the column pass before it: 224 -> 210 us; a CU with
-    // one block has nothing to run while its waves wait, 1024 x 1024: 102.5 -> 104.9)
-    const bool in_step = gridDim.x * gridDim.z >= 512;
     // (the band split as two loops: fewer sums are live at a time)
     auto run_planes = [&](int end, auto hi) {
       for (; q < end; q += S) {
@@ -349,8 +344,6 @@ __global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs 
         // the next plane's row is loaded once pass 1 has moved this one into the scratch, so its
         // latency overlaps the remaining passes; the load is unconditional (the last one reloads
         // the last plane, unused), which keeps it out of a branch
-        if constexpr (N >= 256 && N <= 1024)
-          if (in_step) __syncthreads();
         load(v, q + S < a.planes ? q + S : q);
         float2 o[E];
         F::template stage_out<row_inv(KIND)>(o, ws, twl, l);

@@ -1,6 +1,6 @@
 """The 2048-row column pass of the angular spectrum over a persistent grid: fewer items than the
 rule asks for, the smallest launch that loops, items that do not divide evenly over the blocks, planes
-of several windows in one launch; and the moment rows in step (blocks of 512 and more per launch).
+of several windows in one launch.
 FP32 bar of the path: relative L2 <= 1e-5 against FP64."""
 import numpy as np
 import pytest
