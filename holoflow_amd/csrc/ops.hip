@@ -9,6 +9,8 @@
 
 #include "hfx_kernels.hh"
 
+#include "axis_columns.hh"
+
 namespace hfx {
 
 struct ShiftGeo {
@@ -761,18 +763,12 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 
 template <int DT, bool VEC> struct DftColumns {
   static constexpr int NF = DT == 3 ? 8 : 4;  // floats of four samples
-  const char *base[VEC ? 1 : 4];
-  long long step;  // bytes from sample j to j + 1 of a column
-  // first column c (of outer * inner)
-  __device__ __forceinline__ void init(const DftAxisArgs &a, long long c, long long cols) {
-    constexpr int esz = DT == 1 ? 2 : DT == 2 ? 4 : 8;
-    step = a.inner * esz;
-#pragma unroll
-    for (int t = 0; t < (VEC ? 1 : 4); ++t) {
-      const long long cc = c + t < cols ? c + t : cols - 1;  // past the end: the last column, not stored
-      const long long o = cc / a.inner, i = cc - o * a.inner;
-      base[t] = reinterpret_cast<const char *>(a.in) + (o * a.n * a.inner + i) * esz;
-    }
+  const char *in;
+  AxisColumns<DT == 1 ? 2 : DT == 2 ? 4 : 8, VEC> col;
+  // columns c0 .. c0 + 3 (of outer * inner)
+  __device__ __forceinline__ void init(const DftAxisArgs &a, long long c0, long long cols) {
+    in = reinterpret_cast<const char *>(a.in);
+    col.init(c0, cols, a.n, a.inner);
   }
   // the raw samples j of the four columns
   struct Raw {
@@ -780,25 +776,25 @@ template <int DT, bool VEC> struct DftColumns {
     unsigned w[VEC ? 1 : NF];
   };
   __device__ __forceinline__ void load(Raw &r, int j) const {
-    const long long off = j * step;
+    const long long off = j * col.step;
     if constexpr (VEC) {
       if constexpr (DT == 1) {
-        const uint2 v = *reinterpret_cast<const uint2 *>(base[0] + off);
+        const uint2 v = *reinterpret_cast<const uint2 *>(in + col.off[0] + off);
         r.q[0].x = v.x;
         r.q[0].y = v.y;
       } else {
-        r.q[0] = *reinterpret_cast<const uint4 *>(base[0] + off);
-        if constexpr (DT == 3) r.q[1] = *reinterpret_cast<const uint4 *>(base[0] + off + 16);
+        r.q[0] = *reinterpret_cast<const uint4 *>(in + col.off[0] + off);
+        if constexpr (DT == 3) r.q[1] = *reinterpret_cast<const uint4 *>(in + col.off[0] + off + 16);
       }
     } else {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         if constexpr (DT == 1) {
-          r.w[t] = *reinterpret_cast<const uint16_t *>(base[t] + off);
+          r.w[t] = *reinterpret_cast<const uint16_t *>(in + col.off[t] + off);
         } else if constexpr (DT == 2) {
-          r.w[t] = *reinterpret_cast<const unsigned *>(base[t] + off);
+          r.w[t] = *reinterpret_cast<const unsigned *>(in + col.off[t] + off);
         } else {
-          const uint2 v = *reinterpret_cast<const uint2 *>(base[t] + off);
+          const uint2 v = *reinterpret_cast<const uint2 *>(in + col.off[t] + off);
           r.w[2 * t] = v.x;
           r.w[2 * t + 1] = v.y;
         }
@@ -846,7 +842,7 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
   for (long long it = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); it < tiles; it += (long long)gridDim.x * 4) {
     const long long c0 = it * 64 + 4 * rw;
     X x;
-    x.init(a, c0 < cols ? c0 : cols - 1, cols);
+    x.init(a, c0, cols);
     f4v re[NBF][4], im[NBF][4];
     int idx[NBF], inc[NBF];  // k p mod n of this lane's bin and pair, and its advance by four pairs
 #pragma unroll
