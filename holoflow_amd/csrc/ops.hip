@@ -42,14 +42,17 @@ __global__ void k_fftshift(const uint8_t *in, uint8_t *out, int esz, ShiftGeo g)
 }
 
 // fftshift of [batch][rows][units] with units of U bytes (the largest of 16, 8, 4 that the row, its
-// half and both buffers are multiples of): no index division, one 16-byte copy per lane.  A
-// 1024 x 1024 F32 image: 5.7 us with one division per axis and element, 3.3 us here.
+// half and both buffers are multiples of): no index division, one 16-byte copy per lane.  A block's
+// lanes spread over units, rows and images as the sizes fill them.  1024 x 1024 F32: 5.7 us with one
+// division per axis and element, 3.3 us here; 262,140 rows of 8 F32: 7.7 and 3.6 (64
+// lanes along every row: 30); 65,535 images of 4 x 4: 5.9 and 3.0 (30).
 template <typename V>
-__global__ __launch_bounds__(256) void k_fftshift_rows(const V *__restrict__ in, V *__restrict__ out, int rows,
-                                                       int units, int row_shift, int unit_shift) {
-  const int u = blockIdx.x * 64 + threadIdx.x, r = blockIdx.y * 4 + threadIdx.y;
-  if (u >= units || r >= rows) return;
-  const long long base = (long long)blockIdx.z * rows * units;
+__global__ __launch_bounds__(256) void k_fftshift_rows(const V *__restrict__ in, V *__restrict__ out, int batch,
+                                                       int rows, int units, int row_shift, int unit_shift) {
+  const int u = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y * blockDim.y + threadIdx.y;
+  const int b = blockIdx.z * blockDim.z + threadIdx.z;
+  if (u >= units || r >= rows || b >= batch) return;
+  const long long base = (long long)b * rows * units;
   int sr = r + row_shift, su = u + unit_shift;
   if (sr >= rows) sr -= rows;
   if (su >= units) su -= units;
@@ -77,23 +80,26 @@ static bool launch_fftshift_rows(const void *in, void *out, int elem_size, int n
   const uintptr_t align = reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out) | (uintptr_t)wbytes | (uintptr_t)half;
   const int u = align % 16 == 0 ? 16 : align % 8 == 0 ? 8 : align % 4 == 0 ? 4 : 0;
   if (u == 0) return false;
-  if (rows == 1 && row_shift == 0 && batch > 1) {  // only rows: the batch takes their place
+  if (rows == 1) {  // only rows: the batch takes their place
     rows = batch;
     batch = 1;
   }
   const long long units = wbytes / u;
-  if (units >= (1LL << 31) || (rows + 3) / 4 > 65535 || batch > 65535) return false;
-  const dim3 grid((unsigned)((units + 63) / 64), (unsigned)((rows + 3) / 4), (unsigned)batch), block(64, 4);
+  // the lanes of a block: 64 along a row, fewer where it is shorter, then rows, then images
+  unsigned bx = 64, by = 4, bz = 1;
+  while (bx / 2 >= units) bx /= 2, by *= 2;
+  while (by / 2 >= rows) by /= 2, bz *= 2;
+  while (bz / 2 >= batch) bz /= 2, bx *= 2;
+  const long long gx = (units + bx - 1) / bx, gy = (rows + by - 1) / by, gz = (batch + bz - 1) / bz;
+  if (units >= (1LL << 31) || rows >= (1LL << 31) || batch >= (1LL << 31) || gy > 65535 || gz > 65535) return false;
+  const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz), block(bx, by, bz);
   const int us = (int)(half / u);
-  if (u == 16)
-    hipLaunchKernelGGL(k_fftshift_rows<uint4>, grid, block, 0, st, reinterpret_cast<const uint4 *>(in),
-                       reinterpret_cast<uint4 *>(out), (int)rows, (int)units, (int)row_shift, us);
-  else if (u == 8)
-    hipLaunchKernelGGL(k_fftshift_rows<uint2>, grid, block, 0, st, reinterpret_cast<const uint2 *>(in),
-                       reinterpret_cast<uint2 *>(out), (int)rows, (int)units, (int)row_shift, us);
-  else
-    hipLaunchKernelGGL(k_fftshift_rows<uint32_t>, grid, block, 0, st, reinterpret_cast<const uint32_t *>(in),
-                       reinterpret_cast<uint32_t *>(out), (int)rows, (int)units, (int)row_shift, us);
+  auto go = [&](auto v) {
+    using V = decltype(v);
+    hipLaunchKernelGGL(k_fftshift_rows<V>, grid, block, 0, st, reinterpret_cast<const V *>(in),
+                       reinterpret_cast<V *>(out), (int)batch, (int)rows, (int)units, (int)row_shift, us);
+  };
+  u == 16 ? go(uint4{}) : u == 8 ? go(uint2{}) : go(uint32_t{});
   return true;
 }
 
