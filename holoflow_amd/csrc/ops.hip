@@ -125,9 +125,9 @@ int launch_fftshift(const void *in, void *out, int elem_size, int ndim, const lo
 
 // Mean over the plane axis of m_k(p) = |x| (complex), x or |x| (real), or its square, weighted by
 // w_k when WEIGHTED; products rounded before the ascending sum.  V pixels per lane (16-byte
-// loads), planes in groups of eight whose loads are in flight together: three reductions of
+// loads), planes in groups of J whose loads are in flight together: three reductions of
 // [15][1024^2] F32, 63 MB each in the last-level cache, 15.8 -> 12.7 us each.
-template <bool CPLX, bool WEIGHTED, int V>
+template <bool CPLX, bool WEIGHTED, int V, int J>
 __global__ __launch_bounds__(256) void k_weighted_mean(const float *__restrict__ in, const float *__restrict__ w,
                                                        float *__restrict__ out, long long planes, long long npix,
                                                        int power2, int absval) {
@@ -159,19 +159,19 @@ __global__ __launch_bounds__(256) void k_weighted_mean(const float *__restrict__
   const float *src = in + p * C;
   const long long step = npix * C;
   long long k = 0;
-  for (; k + 8 <= planes; k += 8) {
-    vec x[8];
+  for (; k + J <= planes; k += J) {
+    vec x[J];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = *reinterpret_cast<const vec *>(src + (k + j) * step);
+    for (int j = 0; j < J; ++j) x[j] = *reinterpret_cast<const vec *>(src + (k + j) * step);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) add(x[j], k + j);
+    for (int j = 0; j < J; ++j) add(x[j], k + j);
   }
   if (k < planes) {  // the rest, with planes past the end loading the last one, unused
-    vec x[8];
+    vec x[J];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = *reinterpret_cast<const vec *>(src + (k + j < planes ? k + j : planes - 1) * step);
+    for (int j = 0; j < J; ++j) x[j] = *reinterpret_cast<const vec *>(src + (k + j < planes ? k + j : planes - 1) * step);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < J; ++j)
       if (k + j < planes) add(x[j], k + j);
   }
   const float n = (float)planes;
@@ -191,12 +191,20 @@ static void launch_mean(const float *in, const float *w, float *out, long long p
   constexpr int V = CPLX ? 2 : 4;
   // wide loads need aligned planes, and pay only when the wider lanes still fill the chip
   const uintptr_t align = reinterpret_cast<uintptr_t>(in) % 16 + reinterpret_cast<uintptr_t>(out) % (4 * V);
-  if (align == 0 && npix % V == 0 && npix / V >= 65536)
-    hipLaunchKernelGGL((k_weighted_mean<CPLX, WEIGHTED, V>), dim3((unsigned)((npix / V + 255) / 256)), dim3(256), 0, st,
-                       in, w, out, planes, npix, power2, absval);
-  else
-    hipLaunchKernelGGL((k_weighted_mean<CPLX, WEIGHTED, 1>), dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, st, in,
+  const bool wide = align == 0 && npix % V == 0 && npix / V >= 65536;
+  const dim3 block(256);
+  // Complex planes that stay in the 256 MiB last-level cache: two planes in flight per lane.  Eight
+  // walk eight planes at once, which the cache serves worse: [15][1024^2] 25.2 against 21.9 us,
+  // [30][1024^2] 46.9 and 39.7; beyond it, out of memory, eight are better ([52][2048^2] 321 and 336).
+  if (CPLX && wide && planes * npix * 8 <= (256LL << 20))
+    hipLaunchKernelGGL((k_weighted_mean<CPLX, WEIGHTED, V, CPLX ? 2 : 8>), dim3((unsigned)((npix / V + 255) / 256)), block, 0,
+                       st, in, w, out, planes, npix, power2, absval);
+  else if (wide)
+    hipLaunchKernelGGL((k_weighted_mean<CPLX, WEIGHTED, V, 8>), dim3((unsigned)((npix / V + 255) / 256)), block, 0, st, in,
                        w, out, planes, npix, power2, absval);
+  else
+    hipLaunchKernelGGL((k_weighted_mean<CPLX, WEIGHTED, 1, 8>), dim3((unsigned)((npix + 255) / 256)), block, 0, st, in, w,
+                       out, planes, npix, power2, absval);
 }
 
 int launch_weighted_mean(const void *in, int in_complex, long long planes, long long npix, const float *w, float *out,
