@@ -6,6 +6,7 @@
 //               multiply.cu:69-92 wired by graph_builder.cc:612-631)
 //   convert   : uint16 -> float32 or complex64 (x + 0i) (conversion.cu:156-202)
 #include <mutex>
+#include <type_traits>
 
 #include "hfx_kernels.hh"
 
@@ -232,6 +233,9 @@ __device__ __forceinline__ float conv_complex(float2 z, int strategy) {
   return strategy == 3 ? atan2f(z.y, z.x) : hypotf(z.x, z.y);
 }
 
+// elements that a lane of k_convert's wide form converts at once: 16 bytes on the wider side
+constexpr int convert_width(int in, int out) { return in == 3 || out == 3 ? 2 : 4; }
+
 template <int IN, int OUT> __device__ __forceinline__ void convert_one(const void *in, void *out, int strategy, long long i) {
   if constexpr (IN == 3) {  // CF32 -> F32: modulus (hypot) or argument (atan2)
     reinterpret_cast<float *>(out)[i] = conv_complex(reinterpret_cast<const float2 *>(in)[i], strategy);
@@ -242,83 +246,68 @@ template <int IN, int OUT> __device__ __forceinline__ void convert_one(const voi
   }
 }
 
-// Bound by memory.  VEC: four consecutive elements per lane and access (8-byte U16 loads, 16-byte
-// stores) and four such groups in flight; the [64][1024^2] U16 -> F32 conversion of a window:
-// 146 us with one element per lane, 61 us here (403 MB; the store side stays partly in the last-level cache).  Otherwise (buffers not aligned to
-// four elements) one element per lane.
-template <int IN, int OUT, bool VEC>
+// Bound by memory.  G > 0: V consecutive elements per lane and access and G such groups in flight,
+// 16 bytes of neighbouring lanes next to each other on the wider side; G = 0 (buffers not aligned to V
+// elements): one element per lane.  [64][1024^2] U16 -> F32 (403 MB): 149 us with one element per lane,
+// 66-69 here; 4 M U16 -> CF32: 8.5 and 7.0 (four elements per lane, whose two stores then take every
+// other 16 bytes: 9.9).
+template <int IN, int OUT, int G>
 __global__ __launch_bounds__(256) void k_convert(const void *__restrict__ in, void *__restrict__ out, int strategy,
                                                  long long n) {
-  if constexpr (!VEC) {
+  if constexpr (G == 0) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i < n) convert_one<IN, OUT>(in, out, strategy, i);
   } else {
-    constexpr int G = 4;
-    const long long i0 = (long long)blockIdx.x * (1024 * G) + 4 * threadIdx.x;
-    if (i0 + 1024 * (G - 1) + 3 < n) {
-      uint4 raw[G][IN == 3 ? 2 : 1];
+    constexpr int V = convert_width(IN, OUT), NI = IN == 3 ? 2 * V : V;  // elements and their 32-bit parts
+    typedef std::conditional_t<IN == 1, uint16_t, std::conditional_t<IN == 4, uint8_t, float>> E;
+    typedef E vin __attribute__((ext_vector_type(NI)));
+    typedef float vout __attribute__((ext_vector_type(OUT == 3 ? 2 * V : V)));
+    const long long i0 = (long long)blockIdx.x * (256 * V * G) + V * threadIdx.x;
+    if (i0 + 256 * V * (G - 1) + V <= n) {
+      vin raw[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) raw[g] = *reinterpret_cast<const vin *>(reinterpret_cast<const E *>(in) + (i0 + 256 * V * g) * (NI / V));
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const long long i = i0 + 1024 * g;
-        if constexpr (IN == 1) {
-          const uint2 v = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(in) + i);
-          raw[g][0].x = v.x;
-          raw[g][0].y = v.y;
-        } else if constexpr (IN == 4) {
-          raw[g][0].x = *reinterpret_cast<const unsigned *>(reinterpret_cast<const uint8_t *>(in) + i);
-        } else {
-          constexpr int C = IN == 3 ? 2 : 1;
+        vout y;
 #pragma unroll
-          for (int h = 0; h < C; ++h) raw[g][h] = reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(in) + C * i)[h];
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const long long i = i0 + 1024 * g;
-        float x[4];
-        if constexpr (IN == 1) {
-          x[0] = (float)(raw[g][0].x & 0xffffu);
-          x[1] = (float)(raw[g][0].x >> 16);
-          x[2] = (float)(raw[g][0].y & 0xffffu);
-          x[3] = (float)(raw[g][0].y >> 16);
-        } else if constexpr (IN == 4) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) x[t] = (float)((raw[g][0].x >> (8 * t)) & 0xffu);
-        } else if constexpr (IN == 2) {
-          x[0] = __uint_as_float(raw[g][0].x);
-          x[1] = __uint_as_float(raw[g][0].y);
-          x[2] = __uint_as_float(raw[g][0].z);
-          x[3] = __uint_as_float(raw[g][0].w);
-        } else {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            x[2 * h] = conv_complex(make_float2(__uint_as_float(raw[g][h].x), __uint_as_float(raw[g][h].y)), strategy);
-            x[2 * h + 1] = conv_complex(make_float2(__uint_as_float(raw[g][h].z), __uint_as_float(raw[g][h].w)), strategy);
+        for (int t = 0; t < V; ++t) {
+          if constexpr (IN == 3) {
+            y[t] = conv_complex(make_float2(raw[g][2 * t], raw[g][2 * t + 1]), strategy);
+          } else if constexpr (OUT == 3) {
+            y[2 * t] = (float)raw[g][t];
+            y[2 * t + 1] = 0.f;
+          } else {
+            y[t] = (float)raw[g][t];
           }
         }
-        if constexpr (OUT == 3) {
-          float4 *dst = reinterpret_cast<float4 *>(reinterpret_cast<float2 *>(out) + i);
-          dst[0] = make_float4(x[0], 0.f, x[1], 0.f);
-          dst[1] = make_float4(x[2], 0.f, x[3], 0.f);
-        } else {
-          *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + i) = make_float4(x[0], x[1], x[2], x[3]);
-        }
+        *reinterpret_cast<vout *>(reinterpret_cast<float *>(out) + (i0 + 256 * V * g) * (OUT == 3 ? 2 : 1)) = y;
       }
     } else {
       for (int g = 0; g < G; ++g)
-        for (int t = 0; t < 4; ++t)
-          if (i0 + 1024 * g + t < n) convert_one<IN, OUT>(in, out, strategy, i0 + 1024 * g + t);
+        for (int t = 0; t < V; ++t)
+          if (i0 + 256 * V * g + t < n) convert_one<IN, OUT>(in, out, strategy, i0 + 256 * V * g + t);
     }
   }
 }
 
 template <int IN, int OUT> static void launch_convert_pair(const void *in, void *out, int strategy, long long n, hipStream_t st) {
-  constexpr int esz = IN == 1 ? 2 : IN == 4 ? 1 : 4;
-  const bool vec = reinterpret_cast<uintptr_t>(in) % (4 * esz) == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  if (vec)
-    hipLaunchKernelGGL((k_convert<IN, OUT, true>), dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0, st, in, out, strategy, n);
+  constexpr int V = convert_width(IN, OUT);
+  constexpr int in_bytes = V * (IN == 1 ? 2 : IN == 4 ? 1 : IN == 3 ? 8 : 4), out_bytes = V * (OUT == 3 ? 8 : 4);
+  const bool wide = reinterpret_cast<uintptr_t>(in) % in_bytes == 0 && reinterpret_cast<uintptr_t>(out) % out_bytes == 0;
+  auto go = [&](auto g) {
+    constexpr int G = decltype(g)::value;
+    const long long per_block = 256 * (G == 0 ? 1 : V * G);
+    hipLaunchKernelGGL((k_convert<IN, OUT, G>), dim3((unsigned)((n + per_block - 1) / per_block)), dim3(256), 0, st, in, out, strategy, n);
+  };
+  // two groups per lane only where the halved grid still fills the chip: argument of 1 M CF32 3.2 us
+  // with one, 3.7 with two (and 4.1 with four); 8 M CF32 moduli 16.1 with one, 15.1 with two
+  if (!wide)
+    go(std::integral_constant<int, 0>{});
+  else if (n < (1 << 21))
+    go(std::integral_constant<int, 1>{});
   else
-    hipLaunchKernelGGL((k_convert<IN, OUT, false>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, out, strategy, n);
+    go(std::integral_constant<int, 2>{});
 }
 
 // min / max of n floats: per-block partials, then one block folds them (order-free ops)
@@ -385,7 +374,9 @@ __global__ __launch_bounds__(256) void k_scaled(const float *__restrict__ in, O 
 }
 
 template <typename O> static void launch_scaled(const float *in, O *out, long long n, const float2 *mm, hipStream_t st) {
-  if (reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(O)) == 0)
+  // (four per lane leave a small grid short of blocks: 65,536 elements 6.4 us for the whole conversion
+  // with one per lane, 6.8 with four; 2 M 10.1 and 8.4)
+  if (n >= (1 << 20) && reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(O)) == 0)
     hipLaunchKernelGGL((k_scaled<O, 4>), dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, in, out, n, mm);
   else
     hipLaunchKernelGGL((k_scaled<O, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, out, n, mm);

@@ -40,3 +40,45 @@ def test_mean_of_complex_planes(gpu, planes, npix, weighted):
     assert bool(torch.isfinite(got[fine]).all()) and int((~fine).sum()) == 2
     # each |x| within 2 ulp, the product and each of `planes` additions of positive terms within half
     assert bool(((got[fine] - ref[fine]).abs() <= (planes + 4) * 2.0**-23 * ref[fine]).all())
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 512, 513, 1023, 1025, 4095, (1 << 21) - 1, 1 << 21, (1 << 21) + 1027])
+@pytest.mark.parametrize("src", [torch.uint8, torch.uint16, torch.float32])
+def test_conversion_tails(gpu, n, src):
+    from holoflow_amd._lib import DTYPE_CF32, DTYPE_F32, DTYPE_U16, check, lib
+    import ctypes as C
+
+    host = torch.arange(n, dtype=torch.int64) * 7 % (255 if src == torch.uint8 else 65521)
+    x = host.to(torch.int32).to(src).cuda() if src != torch.float32 else (host - 9.5).float().cuda()
+    if src == torch.float32 and n > 2:
+        x[0], x[n // 2], x[n - 1] = float("nan"), -0.0, float("inf")
+    want = x.cpu().float() if src == torch.float32 else host.float()
+    for dt, out in ((DTYPE_F32, torch.full((n + 1,), -3.0, device="cuda")),
+                    (DTYPE_CF32, torch.full((n + 1,), -3.0, dtype=torch.complex64, device="cuda"))):
+        if src == torch.float32 and dt == DTYPE_F32:
+            continue
+        code = {torch.uint8: 4, torch.uint16: DTYPE_U16, torch.float32: DTYPE_F32}[src]
+        check(lib().hfx_convert(C.c_void_p(x.data_ptr()), code, C.c_void_p(out.data_ptr()), dt, 0, n, None,
+                                C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got = out.cpu()
+        re = got.real if got.is_complex() else got
+        assert torch.equal(re[:n].contiguous().view(torch.int32), want.view(torch.int32)) and float(re[n]) == -3.0
+        if got.is_complex():
+            assert not bool(got.imag.any())
+
+
+@pytest.mark.parametrize("n", [1, 3, 513, 4095, 1 << 21, (1 << 21) + 1025])
+@pytest.mark.parametrize("off", [0, 1])
+def test_modulus_and_argument_tails(gpu, n, off):
+    from holoflow_amd._lib import DTYPE_CF32, DTYPE_F32, check, lib
+    import ctypes as C
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n + off, dtype=torch.complex64, device="cuda", generator=g)[off:]
+    out = torch.empty(n, device="cuda")
+    d = x.to(torch.complex128)
+    for strategy, ref in ((2, d.abs()), (3, d.angle())):
+        check(lib().hfx_convert(C.c_void_p(x.data_ptr()), DTYPE_CF32, C.c_void_p(out.data_ptr()), DTYPE_F32, strategy, n,
+                                None, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        # hypotf and atan2f are within a few ulp
+        assert bool(((out - ref).abs() <= 8 * 2.0**-24 * ref.abs() + 1e-30).all())
