@@ -746,8 +746,57 @@ __global__ void k_dft_axis(DftAxisArgs a) {
   a.out[t] = make_float2(sr * a.scale, si * a.scale);
 }
 
+// Band DFT of up to DFT_SHORT points: a lane owns one column and sums directly over j, which leaves
+// little but the stream (the matrix form spends 16 bins and four pairs of samples on them).  All bins
+// of 1 M U16 columns at n = 1, 4 and 8: 5.4, 9.5 and 21 us, in the matrix form 20, 23.8 and 27.
+// At 12 points and 12 bins the sums cost more than the matrix form (65,536 columns: 11.1 against 5.8).
+constexpr int DFT_SHORT = 8;
+template <int DT> __global__ __launch_bounds__(256) void k_dft_axis_short(DftAxisArgs a, long long cols) {
+  __shared__ float2 tw[DFT_SHORT];
+  if (threadIdx.x < a.n) {
+    double s, c;
+    sincospi(2.0 * (double)threadIdx.x / (double)a.n, &s, &c);
+    tw[threadIdx.x] = make_float2((float)c, (float)(-s));
+  }
+  __syncthreads();
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (c >= cols) return;
+  const long long o = c / a.inner, i = c - o * a.inner;
+  float2 x[DFT_SHORT];
+#pragma unroll
+  for (int j = 0; j < DFT_SHORT; ++j) {
+    if (j >= a.n) break;
+    const long long src = (o * a.n + j) * a.inner + i;
+    if constexpr (DT == 1)
+      x[j] = make_float2((float)reinterpret_cast<const uint16_t *>(a.in)[src], 0.f);
+    else if constexpr (DT == 2)
+      x[j] = make_float2(reinterpret_cast<const float *>(a.in)[src], 0.f);
+    else
+      x[j] = reinterpret_cast<const float2 *>(a.in)[src];
+  }
+  for (int k = a.kb; k < a.ke; ++k) {
+    float2 acc = make_float2(0.f, 0.f);
+    int m = 0;
+#pragma unroll
+    for (int j = 0; j < DFT_SHORT; ++j) {
+      if (j >= a.n) break;
+      const float2 w = tw[m];
+      if constexpr (DT == 3) {
+        acc.x += x[j].x * w.x - x[j].y * w.y;
+        acc.y += x[j].x * w.y + x[j].y * w.x;
+      } else {
+        acc.x += x[j].x * w.x;
+        acc.y += x[j].x * w.y;
+      }
+      m += k;
+      m = m >= a.n ? m - a.n : m;
+    }
+    a.out[(o * (a.ke - a.kb) + (k - a.kb)) * a.inner + i] = make_float2(acc.x * a.scale, acc.y * a.scale);
+  }
+}
+
 // Band DFT along the middle axis on the matrix cores, n <= DFT_MAXN.  A wave owns 64 columns (an
-// outer and an inner index; four adjacent ones per lane), and the symmetry of the kernel is folded
+// outer and an inner index; four per lane, AxisColumns), and the symmetry of the kernel is folded
 // as in the fused path's time DFT: with s = x_p + x_{n-p}, d = x_p - x_{n-p},
 //   X_k = x_0 [+ (-1)^k x_{n/2}] + sum_{p=1}^{(n-1)/2} (s cos(2 pi k p / n) - i d sin(2 pi k p / n)),
 // so 16 bins and 16 columns take 2 ((n-1)/2)/4 + 1 FP32 MFMAs for real input, twice that for
@@ -770,10 +819,9 @@ template <int DT, bool VEC> struct DftColumns {
   static constexpr int NF = DT == 3 ? 8 : 4;  // floats of four samples
   const char *in;
   AxisColumns<DT == 1 ? 2 : DT == 2 ? 4 : 8, VEC> col;
-  // columns c0 .. c0 + 3 (of outer * inner)
-  __device__ __forceinline__ void init(const DftAxisArgs &a, long long c0, long long cols) {
+  __device__ __forceinline__ void init(const DftAxisArgs &a, long long tile, int rw, long long cols) {
     in = reinterpret_cast<const char *>(a.in);
-    col.init(c0, cols, a.n, a.inner);
+    col.init(tile, rw, cols, a.n, a.inner);
   }
   // the raw samples j of the four columns
   struct Raw {
@@ -845,9 +893,8 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
   const int lane = threadIdx.x & 63, g = lane >> 4, rw = lane & 15;
   const long long tiles = (cols + 63) / 64;
   for (long long it = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); it < tiles; it += (long long)gridDim.x * 4) {
-    const long long c0 = it * 64 + 4 * rw;
     X x;
-    x.init(a, c0, cols);
+    x.init(a, it, rw, cols);
     f4v re[NBF][4], im[NBF][4];
     int idx[NBF], inc[NBF];  // k p mod n of this lane's bin and pair, and its advance by four pairs
 #pragma unroll
@@ -930,7 +977,7 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
       }
     }
     // lane holds bins 16 f + 4 g + r of its four columns
-    const long long nk = a.ke - a.kb;
+    const long long nk = a.ke - a.kb, c0 = x.col.column(it, rw, 0);
     if (c0 >= cols) continue;
 #pragma unroll
     for (int f = 0; f < NBF; ++f) {
@@ -949,8 +996,9 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
         } else {
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            if (c0 + t < cols) {
-              const long long o = (c0 + t) / a.inner, i = c0 + t - o * a.inner;
+            const long long c = x.col.column(it, rw, t);
+            if (c < cols) {
+              const long long o = c / a.inner, i = c - o * a.inner;
               a.out[(o * nk + (k - a.kb)) * a.inner + i] = v[t];
             }
           }
@@ -991,8 +1039,15 @@ int launch_dft_axis(const void *in, int dtype, long long outer, int n, long long
   DftAxisArgs a{in, dtype, outer, inner, n, kb, ke, scale, out};
   long long total = outer * (long long)(ke - kb) * inner;
   if (total == 0) return 0;
-  if (n <= DFT_MAXN) {
-    const long long cols = outer * inner;
+  const long long cols = outer * inner;
+  if (n <= DFT_SHORT) {
+    const dim3 grid((unsigned)((cols + 255) / 256)), block(256);
+    switch (dtype) {
+      case 1: hipLaunchKernelGGL(k_dft_axis_short<1>, grid, block, 0, st, a, cols); break;
+      case 2: hipLaunchKernelGGL(k_dft_axis_short<2>, grid, block, 0, st, a, cols); break;
+      default: hipLaunchKernelGGL(k_dft_axis_short<3>, grid, block, 0, st, a, cols); break;
+    }
+  } else if (n <= DFT_MAXN) {
     const uintptr_t align = reinterpret_cast<uintptr_t>(in) % (dtype == 1 ? 8 : 16) + reinterpret_cast<uintptr_t>(out) % 16;
     const bool vec = inner % 4 == 0 && align == 0;  // four adjacent columns share an outer index
     switch (dtype) {

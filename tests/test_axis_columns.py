@@ -17,13 +17,12 @@ template <int ESZ, bool VEC> void walk(long long outer, int n, long long inner) 
   const long long width = VEC ? 4 * ESZ : ESZ;  // bytes of one access
   for (long long tile = 0; tile < (cols + 63) / 64; ++tile)
     for (int lane = 0; lane < 16; ++lane) {
-      const long long c0 = tile * 64 + 4 * lane;
       hfx::AxisColumns<ESZ, VEC> a;
-      a.init(c0, cols, n, inner);
+      a.init(tile, lane, cols, n, inner);
       for (int t = 0; t < a.N; ++t)
         for (int j = 0; j < n; ++j) {
           const long long at = a.off[t] + j * a.step;
-          const long long c = c0 + t, own = ((c / inner * n + j) * inner + c % inner) * ESZ;
+          const long long c = a.column(tile, lane, t), own = ((c / inner * n + j) * inner + c % inner) * ESZ;
           const bool bad = at < 0 || at + width > bytes || (VEC && at % (width < 16 ? width : 16) != 0) ||
                            (c < cols && at != own);
           if (bad) {

@@ -82,3 +82,26 @@ def test_modulus_and_argument_tails(gpu, n, off):
                                 None, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
         # hypotf and atan2f are within a few ulp
         assert bool(((out - ref).abs() <= 8 * 2.0**-24 * ref.abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("kind", ["u16", "f32", "cf32"])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 9, 12, 13])
+@pytest.mark.parametrize("outer,inner", [(1, 4099), (3, 64), (70, 1), (5, 33), (1, 300 * 3)])
+def test_dft_of_few_points_and_odd_columns(gpu, kind, n, outer, inner):
+    """The direct sums up to eight points and the matrix form beyond, with columns that are and are not
+    adjacent per lane."""
+    from holoflow_amd import hfx
+
+    g = torch.Generator().manual_seed(n + inner)
+    if kind == "u16":
+        x = torch.randint(0, 1 << 16, (outer, n, inner), generator=g, dtype=torch.int32)
+        wide, x = x.double(), x.to(torch.uint16)
+    else:
+        x = torch.randn((outer, n, inner), generator=g, dtype=torch.float32 if kind == "f32" else torch.complex64)
+        wide = x.to(torch.complex128)
+    for kb, ke in ((0, n), (n - 1, n), (0, n // 2 + 1)):
+        ref = torch.fft.fft(wide, dim=1)[:, kb:ke]
+        got = hfx.dft_axis(x.cuda(), 1, kb, ke).cpu()
+        # n products with twiddles rounded once, summed in FP32
+        bound = (n + 2) * 2.0**-23 * wide.abs().sum(1, keepdim=True) * 2**0.5
+        assert bool(((got - ref).abs() <= bound).all())
