@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
 // keep the accumulators in ordinary registers instead of splitting them off into accumulation
 // registers: up to two tiles fit in three waves per SIMD, three and four tiles in two.
 constexpr int fold_min_blocks(int nbf) { return nbf <= 2 ? 3 : 2; }
-template <int NBF>
+template <int NBF, bool CUT>
 __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs a) {
   extern __shared__ float4 lds_dyn[];
   float *lf = reinterpret_cast<float *>(lds_dyn);
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs 
     // tiles past the end load clamped pixels (dft_px) and store nothing
     const long long p0w = ((long long)(it - w * quads) * 4 + wave) * 64;
     f4 ac[NBF][4], as[NBF][4];
-    dft_fold_tile<NBF>(r, lf, p0w, lane, ac, as);
+    dft_fold_tile<NBF, CUT>(r, lf, p0w, lane, ac, as);
 
     const long long p0 = p0w + 4 * (lane & 15);
     if (p0 >= a.r.npix) continue;
@@ -674,11 +674,15 @@ template <int NBT> static int launch_plain_mode(const DftArgs &a, int mode, hipS
   return -2;
 }
 
-template <int NBF> static int launch_fold(const DftArgs &a, hipStream_t st) {
+template <int NBF, bool CUT> static int launch_fold_cut(const DftArgs &a, hipStream_t st) {
   const size_t lds = dft_fold_lds_bytes(NBF, a.r.T);
-  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF>), lds, dft_quads(a));
-  hipLaunchKernelGGL((k_dft_fold<NBF>), dim3(grid), dim3(256), lds, st, a);
+  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF, CUT>), lds, dft_quads(a));
+  hipLaunchKernelGGL((k_dft_fold<NBF, CUT>), dim3(grid), dim3(256), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <int NBF> static int launch_fold(const DftArgs &a, hipStream_t st) {
+  return a.r.T % 32 == 0 ? launch_fold_cut<NBF, false>(a, st) : launch_fold_cut<NBF, true>(a, st);
 }
 
 int launch_time_dft(const DftLaunch &L, hipStream_t st) {

@@ -441,12 +441,13 @@ template <int TPW, int T, int K> struct DftStreamFold {
 
 // Runtime-T form of the folded FP32 time DFT (see DftStreamFold) for NBF 16-bin tiles and one
 // 64-pixel tile per wave (stand-alone time DFT), T % 4 == 0: steps of four frame pairs in batches
-// of K, the last batch cut where the steps end.  Operand matrix from stage_fold_matrix_rt (NBF
-// tiles).
-template <int NBF, int K = 4>
+// of K.  CUT: T is no multiple of 8 K, so the last batch ends where the steps do (its own form, since
+// the branches make the last batch wait for all loads in flight: 52 bins of 1024^2, T = 128, 223 us
+// where 216 do).  Operand matrix from stage_fold_matrix_rt (NBF tiles).
+template <int NBF, bool CUT, int K = 4>
 __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds, long long p0w, int lane,
                                               f4 (&ac)[NBF][4], f4 (&as)[NBF][4]) {
-  const int T = r.T, steps = (T / 2 + 2) / 4, PC = fold_pitch(T);  // ceil((T/2 - 1) / 4) steps
+  const int T = r.T, steps = CUT ? (T / 2 + 2) / 4 : T / 8, PC = fold_pitch(T);  // ceil((T/2 - 1) / 4) steps
   const float *lc = lds, *ls = lds + 16 * NBF * PC, *lx = lds + 32 * NBF * PC;
   const int g = lane >> 4, rw = lane & 15;
   const long long p0 = dft_px(r, p0w, lane, 0);
@@ -460,7 +461,7 @@ __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds
   const uint2 xe = dft_load4(r, ring_frame(r, g == 0 ? 0 : T / 2), p0);  // x_0, x_{T/2}
   uint2 ring[K][2];
   auto load = [&](int st, int k) {
-    const int p = min(4 * st + g + 1, T / 2);  // pairs past the last one: any frame, zero weights or no step
+    const int p = CUT ? min(4 * st + g + 1, T / 2) : 4 * st + g + 1;  // pairs past the last one: any frame, zero weights or no step
     ring[k][0] = dft_load4(r, ring_frame(r, p), p0);
     ring[k][1] = dft_load4(r, ring_frame(r, T - p), p0);
   };
@@ -501,7 +502,7 @@ __device__ __forceinline__ void dft_fold_tile(const DftRing &r, const float *lds
   }
 #pragma unroll
   for (int k = 0; k < K; ++k)
-    if (s0 + k < steps) step(s0 + k, k, std::false_type{});
+    if (!CUT || s0 + k < steps) step(s0 + k, k, std::false_type{});
   float x[4];
   unpack4(xe, x);
 #pragma unroll
