@@ -19,6 +19,7 @@
 // Plane q of the output: q < nb -> bin kb+q; q >= nb (two-sided path) -> conj of computed
 // bin 2*nb - q, i.e. X[T - (kb + 2*nb - q)] of a real input (fft.cu:163-194 +
 // graph_builder.cc:270-287).
+#include <algorithm>
 #include <type_traits>
 
 #include "dft_core.hh"
@@ -29,21 +30,20 @@ namespace hfx {
 
 struct DftArgs {
   DftRing r;
-  int W;
-  int kb, nb, nbc, both;
-  const float2 *lx, *ly;   // k_dft, k_dft_row: Fresnel lens vectors or null
-  const void *wm_hi, *wm_lo;
-  // fused kernels only
-  int H, blk_c, n_planes;
-  const float2 *tw;        // W-point FFT twiddles
-  // the windows of one launch: one plan's consecutive windows (first frames, planes at a stride),
-  // or for k_front one window each of a group of plans of one shape (the group's tables).  The
-  // fields of the common case come first and the tables last: kernel arguments lie in host memory,
-  // and each further line of them that a kernel reads is another round trip (a table entry per
-  // pointer cost a 64 x 64 window's time DFT 0.7 us)
-  int nwin, grouped;
+  int kb, nb, nbc, both, W;
+  int nwin;                // windows of the launch
   float2 *planes;          // k_dft: natural [planes][npix]; the fused kernels: blocked
   long long planes_stride; // elements from one window's planes to the next
+  const void *wm_hi, *wm_lo;
+  const float2 *lx, *ly;   // k_dft, k_dft_row: Fresnel lens vectors or null
+  // fused kernels only
+  const float2 *tw;        // W-point FFT twiddles
+  int H, blk_c, n_planes, grouped;
+  // the windows of one launch: one plan's consecutive windows (first frames, planes at a stride),
+  // or for k_front one window each of a group of plans of one shape (the group's tables).  What a
+  // single window of the stand-alone kernels needs comes first, in two 64-byte lines, and the tables
+  // last: kernel arguments lie in host memory, and each further line of them that a kernel reads is
+  // another round trip (load_args)
   int firsts[HFX_MAX_WIN];
   const uint16_t *rings[HFX_MAX_GROUP];
   long long ring_frames_w[HFX_MAX_GROUP];
@@ -113,6 +113,15 @@ __device__ __forceinline__ void dft_store_bin(float2 *planes, long long npix, co
   }
 }
 
+// All arguments that a stand-alone kernel reads, asked for in one go at its start: kernel arguments lie
+// in host memory, and the compiler else loads each where it is first used, one round trip after the
+// other (time DFT of a 64 x 64 window, T = 32: 5.3 us so, 4.9 here).
+__device__ __forceinline__ void load_args(const DftArgs &a) {
+  asm volatile("" ::"s"(a.r.ring), "s"(a.r.ring_frames), "s"(a.r.first), "s"(a.r.npix), "s"(a.r.T), "s"(a.kb), "s"(a.nb),
+               "s"(a.nbc), "s"(a.both), "s"(a.W), "s"(a.planes), "s"(a.planes_stride), "s"(a.wm_hi), "s"(a.wm_lo), "s"(a.lx),
+               "s"(a.ly));
+}
+
 // Window of item i where each window has `per` items (no division in the first window, which is all
 // of a single-window launch: the integer division is some forty dependent instructions).
 __device__ __forceinline__ int window_of(unsigned i, unsigned per) {
@@ -132,26 +141,26 @@ template <bool GROUPS = false> __device__ __forceinline__ DftRing window_ring(co
 }
 
 // Persistent: a block stages the operand matrix once (tens of KB, and index arithmetic per
-// element) and then walks groups of four 64-pixel tiles blockIdx, blockIdx + grid, ... of all
-// windows of the launch, window-major.
+// element) and then walks groups of four 64-pixel tiles blockIdx.x, blockIdx.x + gridDim.x, ... of
+// window blockIdx.y.
 template <int NBT, int MODE>
 __global__ __launch_bounds__(256) void k_dft(DftArgs a) {
   extern __shared__ float4 lds_dyn[];
+  load_args(a);
   dft_stage_matrix<NBT, MODE>(lds_dyn, a.wm_hi, a.wm_lo, a.r.T, threadIdx.x, 256);
   __syncthreads();
   const Band b = pinned_band(a);
   const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
+  const DftRing r = window_ring(a, blockIdx.y);
+  float2 *planes = a.planes + blockIdx.y * a.planes_stride;
   const bool lens = a.lx != nullptr;
-  for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
-    const unsigned w = window_of(it, quads);
-    const DftRing r = window_ring(a, w);
-    float2 *planes = a.planes + w * a.planes_stride;
+  for (unsigned it = blockIdx.x; it < quads; it += gridDim.x) {
     // an opaque per-tile copy of the lane index keeps the lane-derived LDS and load addresses of
     // the MFMA loop from being hoisted out of the tile loop (where they would hold registers)
     int lane;
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(threadIdx.x & 63));
     // tiles past the end load clamped pixels (dft_px) and store nothing
-    const long long p0w = ((long long)(it - w * quads) * 4 + (threadIdx.x >> 6)) * 64;
+    const long long p0w = ((long long)it * 4 + (threadIdx.x >> 6)) * 64;
     uint2 pre[1][dft_pre_steps<MODE>()];
     dft_prefetch<MODE, 1>(r, p0w, lane, pre);
     f4 acc1[1][NBT][4];
@@ -193,20 +202,20 @@ template <int NBF, bool CUT>
 __global__ __launch_bounds__(256, fold_min_blocks(NBF)) void k_dft_fold(DftArgs a) {
   extern __shared__ float4 lds_dyn[];
   float *lf = reinterpret_cast<float *>(lds_dyn);
+  load_args(a);
   stage_fold_matrix_rt(lf, reinterpret_cast<const float *>(a.wm_hi), a.r.T, NBF, a.nbc, threadIdx.x, 256);
   __syncthreads();
   const Band b = pinned_band(a);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned quads = (unsigned)((a.r.npix + 255) / 256);  // groups of four tiles of a window
+  const DftRing r = window_ring(a, blockIdx.y);
+  float2 *planes = a.planes + blockIdx.y * a.planes_stride;
   const bool lens = a.lx != nullptr;
-  for (unsigned it = blockIdx.x; it < quads * a.nwin; it += gridDim.x) {
-    const unsigned w = window_of(it, quads);
-    const DftRing r = window_ring(a, w);
-    float2 *planes = a.planes + w * a.planes_stride;
+  for (unsigned it = blockIdx.x; it < quads; it += gridDim.x) {
     int lane;  // opaque per tile, as in k_dft
     asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(threadIdx.x & 63));
     // tiles past the end load clamped pixels (dft_px) and store nothing
-    const long long p0w = ((long long)(it - w * quads) * 4 + wave) * 64;
+    const long long p0w = ((long long)it * 4 + wave) * 64;
     f4 ac[NBF][4], as[NBF][4];
     dft_fold_tile<NBF, CUT>(r, lf, p0w, lane, ac, as);
 
@@ -643,24 +652,22 @@ static DftArgs make_args(const DftLaunch &L) {
   return a;
 }
 
-// Grid of a persistent stand-alone DFT kernel: as many blocks as are resident at once (the
-// occupancy calculator's count per CU times the CUs), at most one per work item.
-static unsigned persistent_grid(const void *kernel, size_t lds, long long items) {
+// Grid of a persistent stand-alone DFT kernel: x blocks per window, y windows, as many blocks in all
+// as are resident at once (the occupancy calculator's count per CU times the CUs), at most one per
+// group of four 64-pixel tiles.
+static dim3 persistent_grid(const void *kernel, size_t lds, const DftArgs &a) {
   int dev = 0, cus = 256, per_cu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, lds) != hipSuccess || per_cu < 1) per_cu = 1;
-  const long long g = (long long)cus * per_cu;
-  return (unsigned)(items < g ? (items > 0 ? items : 1) : g);
+  const long long quads = (a.r.npix + 255) / 256, most = std::max(1LL, (long long)cus * per_cu / a.nwin);
+  return dim3((unsigned)std::min(quads, most), (unsigned)a.nwin);
 }
-
-// groups of four 64-pixel tiles over all windows of a stand-alone launch
-static long long dft_quads(const DftArgs &a) { return (a.r.npix + 255) / 256 * a.nwin; }
 
 template <int NBT, int MODE> static int launch_plain(const DftArgs &a, hipStream_t st) {
   const size_t lds = dft_matrix_lds_bytes(NBT, MODE, a.r.T);
-  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft<NBT, MODE>), lds, dft_quads(a));
-  hipLaunchKernelGGL((k_dft<NBT, MODE>), dim3(grid), dim3(256), lds, st, a);
+  const dim3 grid = persistent_grid(reinterpret_cast<const void *>(&k_dft<NBT, MODE>), lds, a);
+  hipLaunchKernelGGL((k_dft<NBT, MODE>), grid, dim3(256), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -676,8 +683,8 @@ template <int NBT> static int launch_plain_mode(const DftArgs &a, int mode, hipS
 
 template <int NBF, bool CUT> static int launch_fold_cut(const DftArgs &a, hipStream_t st) {
   const size_t lds = dft_fold_lds_bytes(NBF, a.r.T);
-  const unsigned grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF, CUT>), lds, dft_quads(a));
-  hipLaunchKernelGGL((k_dft_fold<NBF, CUT>), dim3(grid), dim3(256), lds, st, a);
+  const dim3 grid = persistent_grid(reinterpret_cast<const void *>(&k_dft_fold<NBF, CUT>), lds, a);
+  hipLaunchKernelGGL((k_dft_fold<NBF, CUT>), grid, dim3(256), lds, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
