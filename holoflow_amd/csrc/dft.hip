@@ -600,8 +600,10 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last row's unused refills land first
   } else {
     // the row FFTs are the longer half of a row at 9..16 bins: their waves issue first (front alone
-    // 84.6 -> 75.5 us at 1024^2, 15 planes; at up to 8 bins it measured 3 % slower)
-    if constexpr (FOLD) __builtin_amdgcn_s_setprio(3);
+    // 84.6 -> 75.5 us at 1024^2, T = 64, 15 planes; at up to 8 bins it measured 3 % slower).  At T = 128
+    // the DFT is as long, and rows shorter than 1024 points lose: 2048 x 512, 15 planes 109 -> 115 us,
+    // 1024 x 768 90 -> 94 (1024^2 121 -> 104)
+    if constexpr (FOLD && (W == 1024 || T < 128)) __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       for (int g = 0; g < ng; ++g) {
