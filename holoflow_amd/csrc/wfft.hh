@@ -182,18 +182,31 @@ __host__ __device__ constexpr int fft_twiddle_index(int n, int i) {
 
 // One 8-byte LDS access.  Volatile, so that accesses at constant offsets are not paired into
 // ds_read2_b64 / ds_write2_b64: a pair keeps the LDS unit busy about a third longer than two single
-// accesses (2048-row column pass: 133 M against 100 M LDS cycles, waits on LDS twice as long).
+// accesses (2048-row column pass: 133 M against 100 M LDS cycles, waits on LDS twice as long).  PAIR
+// leaves the pairing to the compiler, for passes with one wave per SIMD, which wait for instructions
+// rather than for the LDS unit (k_wcol).
 typedef float lds_f2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) volatile lds_f2 lds_vf2;
-__device__ __forceinline__ float2 lds_get(const float2 *p) {
-  const lds_f2 v = *(const lds_vf2 *)p;
+typedef __attribute__((address_space(3))) lds_f2 lds_pf2;
+template <bool PAIR = false> __device__ __forceinline__ float2 lds_get(const float2 *p) {
+  lds_f2 v;
+  if constexpr (PAIR)
+    v = *(const lds_pf2 *)p;
+  else
+    v = *(const lds_vf2 *)p;
   return make_float2(v.x, v.y);
 }
-__device__ __forceinline__ void lds_put(float2 *p, float2 x) { *(lds_vf2 *)p = lds_f2{x.x, x.y}; }
+template <bool PAIR = false> __device__ __forceinline__ void lds_put(float2 *p, float2 x) {
+  if constexpr (PAIR)
+    *(lds_pf2 *)p = lds_f2{x.x, x.y};
+  else
+    *(lds_vf2 *)p = lds_f2{x.x, x.y};
+}
 typedef volatile __attribute__((address_space(3))) float lds_vf1;
 __device__ __forceinline__ void lds_put(float *p, float x) { *(lds_vf1 *)p = x; }
 
-template <int N> struct WaveFft {
+// PAIR: see lds_get.
+template <int N, bool PAIR = false> struct WaveFft {
   static constexpr int L = fft_lanes(N);
   static constexpr int P = 64 / L;  // transforms per wave
   static constexpr int E = N / L;
@@ -248,12 +261,12 @@ template <int N> struct WaveFft {
 #pragma unroll
       for (int q = 0; q < PER; ++q)
 #pragma unroll
-        for (int r = 0; r < R; ++r) u[q][r] = lds_get(src + padc(L * q + r * NB));
+        for (int r = 0; r < R; ++r) u[q][r] = lds_get<PAIR>(src + padc(L * q + r * NB));
     } else {
 #pragma unroll
       for (int q = 0; q < PER; ++q)
 #pragma unroll
-        for (int r = 0; r < R; ++r) u[q][r] = lds_get(scr + pad(ul + L * q + r * NB));
+        for (int r = 0; r < R; ++r) u[q][r] = lds_get<PAIR>(scr + pad(ul + L * q + r * NB));
     }
     // (ul + L q) mod NS, the division left to the cases where neither of L, NS divides the other
     auto mod_ns = [&](int q) { return L % NS == 0 ? ul % NS : NS % L == 0 ? ul + L * q % NS : (ul + L * q) % NS; };
@@ -263,7 +276,7 @@ template <int N> struct WaveFft {
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
-      for (int r = 1; r < R; ++r) w[q][r] = lds_get(tw + TOFF + (r - 1) * NS + mod_ns(q));
+      for (int r = 1; r < R; ++r) w[q][r] = lds_get<PAIR>(tw + TOFF + (r - 1) * NS + mod_ns(q));
 #pragma unroll
     for (int q = 0; q < PER; ++q)
 #pragma unroll
@@ -292,13 +305,13 @@ template <int N> struct WaveFft {
         for (int q = 0; q < PER; ++q)
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            lds_put(dst + padc((L % NS == 0 ? L * q * R : L * q / NS * (NS * R) + L * q % NS) + r * NS), u[q][r]);
+            lds_put<PAIR>(dst + padc((L % NS == 0 ? L * q * R : L * q / NS * (NS * R) + L * q % NS) + r * NS), u[q][r]);
       } else {
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
           const unsigned j = ul + L * q, base = j / NS * (NS * R) + j % NS;
 #pragma unroll
-          for (int r = 0; r < R; ++r) lds_put(scr + pad(base + r * NS), u[q][r]);
+          for (int r = 0; r < R; ++r) lds_put<PAIR>(scr + pad(base + r * NS), u[q][r]);
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -324,10 +337,10 @@ template <int N> struct WaveFft {
     if constexpr ((1 << PSH) % E == 0) {
       float2 *dst = scr + pad((unsigned)lane * E);
 #pragma unroll
-      for (int r = 0; r < E; ++r) lds_put(dst + r, v[r]);
+      for (int r = 0; r < E; ++r) lds_put<PAIR>(dst + r, v[r]);
     } else {
 #pragma unroll
-      for (int r = 0; r < E; ++r) lds_put(scr + pad((unsigned)lane * E + r), v[r]);
+      for (int r = 0; r < E; ++r) lds_put<PAIR>(scr + pad((unsigned)lane * E + r), v[r]);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -336,7 +349,7 @@ template <int N> struct WaveFft {
     __builtin_assume(lane >= 0 && lane < L);
     if constexpr (N == E) {  // one lane holds the whole transform: pass 1 was all of it
 #pragma unroll
-      for (int r = 0; r < E; ++r) o[r] = lds_get(scr + pad(r));
+      for (int r = 0; r < E; ++r) o[r] = lds_get<PAIR>(scr + pad(r));
     } else {
       pass<E, INV ? 1 : -1>(o, scr, tw, lane);
     }

@@ -416,9 +416,12 @@ constexpr int wcol_threads(int n, int kind) { return 64 * wcol_waves(n, kind) * 
 // it: 1677 -> 1596 us.  At 1024 rows and below, where blocks share a CU, one item per block is
 // faster (28 planes of 1024^2 with the moment pass: 169 against 176).
 // PADDED (BLK_MID): only the rows [row0, row1) of the input were written; the others are zero.
+// The 2048-row moment kinds, one wave per SIMD, let their LDS accesses be paired: 52 planes of 2048^2
+// 630 -> 541 us, of 2048 x 512 303 -> 254 (the 2048-row transfer-function kind, two waves per SIMD, is
+// 3 % slower with pairs, and the shorter lengths are even or slower).
 template <int N, int KIND, bool G = false, bool PADDED = false, bool LOOP = false>
 __global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
-  using F = WaveFft<N>;
+  using F = WaveFft<N, is_mom(KIND) && N >= 2048>;
   constexpr int E = F::E, L = F::L, P = F::P;
   constexpr int S = wcol_subsets(N, KIND), WC = wcol_waves(N, KIND);
   __shared__ __align__(16) float2 scr[WC * S * P * F::SCR];

@@ -1,0 +1,38 @@
+"""The launch rules of the column and row passes at the edges of their ranges: 1024-row columns with a
+transfer function in blocks of four waves and of eight, moment rows with the planes of a row over
+several waves and one wave per row, 2048-row moment columns."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(H, W, T, kb, ke, prop, frames=0, **kw):
+    from holoflow_amd import hfx
+
+    F = T + frames + 3
+    g = torch.Generator(device="cuda").manual_seed(H + W + ke)
+    ring = torch.randint(0, 4096, (F, H, W), dtype=torch.int16, device="cuda", generator=g)
+    p = O.PathParams(H, W, T, T // 4, kb, ke, prop, 852e-9, 12e-6, 12e-6, 0.4, fftshift=True, split_bin=kw.get("split_bin", 0))
+    plan = hfx.MomentPlan(hfx.MomentConfig(H, W, T, T // 4, kb, ke, prop, p.lambda_m, p.dx_m, p.dy_m, p.z_m, fftshift=True, **kw))
+    return ring, p, plan
+
+
+def _check(ring, p, plan, first):
+    out = plan.moments(ring, first)
+    win = ring.cpu().numpy().view(np.uint16)[(first + np.arange(p.window)) % ring.shape[0]]
+    ref = O.doppler_moments(win, p, "f64")
+    # the FP32 bar of the path: relative L2 against FP64
+    assert max(rel_l2(out[i].cpu().numpy(), ref[i]) for i in range(out.shape[0])) < 1e-5
+    return out
+
+
+@pytest.mark.parametrize("H,W,planes", [(2048, 16, 5), (2048, 24, 9)])
+@pytest.mark.parametrize("split", [0, 8])
+def test_moment_columns_of_2048_rows(gpu, H, W, planes, split):
+    ring, p, plan = _case(H, W, 64, 6, 6 + planes, "fresnel", split_bin=split)
+    assert _check(ring, p, plan, 4).shape[0] == (5 if split else 3)
