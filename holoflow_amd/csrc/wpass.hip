@@ -181,12 +181,17 @@ __device__ __forceinline__ void store_moment(const PassArgs &a, const PassWin &p
 // Launches of few rows split: one wave per row leaves most SIMDs empty there.  The more rows, the
 // more planes it takes to win back the rounds that S planes do not fill; from 1024 rows on the
 // chip is full without it.  Row pass, one wave per row -> split: 256 x 512 with 1, 4, 16 planes 5.0 ->
-// 4.5, 7.6 -> 5.1, 18.8 -> 10.0 us; 512 x 1024 with 1, 3, 5, 16 planes 7.6 -> 7.9, 12.3 -> 9.6, 16.7 ->
-// 13.7, 37.4 -> 24.7; 768 x 768 with 5, 8, 16 planes 15.4 -> 16.2, 20.5 -> 17.6, 34.4 -> 28.2; 512 x 2048
-// with 2, 5, 16 planes 20.1 -> 16.0, 34.4 -> 31.6, 79.1 -> 65.1; 1024 x 1024 with 5, 16 planes 18.5 ->
-// 21.9, 39.6 -> 39.9.
-constexpr bool wrow_splits(long long rows, int planes) {
-  return rows <= 256 || (rows <= 512 && planes >= 3) || (rows < 1024 && planes >= 8);
+// 4.5, 7.6 -> 5.1, 18.8 -> 10.0 us; 512 x 1024 with 1, 2, 5, 15 planes 7.9 -> 7.8, 9.8 -> 8.7, 15.7 ->
+// 13.5, 34.2 -> 24.3; 512 x 2048 with 2, 5, 15 20.1 -> 15.9, 34.3 -> 31.5, 74.3 -> 65.5; 768 x 768 with 3,
+// 4, 5, 6, 7, 8, 15 11.4 -> 10.9, 13.1 -> 11.6, 14.7 -> 15.9, 16.4 -> 16.4, 18.3 -> 16.8, 19.9 -> 17.8, 31.7
+// -> 27.8; 1024 x 1024 with 5, 16 planes 18.5 -> 21.9, 39.6 -> 39.9.  Above 512 rows one wave per row
+// stays better where the last-level cache does not hold the planes (768 x 1024 with 40, 44, 52
+// planes 80.3 -> 75.6, 92.2 -> 104, 115 -> 147) and for 2048-point rows with the band split, whose
+// block of eight waves holds two rows only (768 x 2048 with 9, 20 planes 55 -> 64, 101 -> 115).
+constexpr bool wrow_splits(long long rows, int planes, int n, bool band) {
+  if (rows <= 512) return rows <= 256 || planes >= 2;
+  return rows < 1024 && (planes >= 8 || planes % 4 == 3 || planes % 4 == 0) && rows * planes * n * 8 <= 256LL << 20 &&
+         !(n >= 2048 && band);
 }
 constexpr int wrow_subsets(int n, int kind, bool split) {
   if (!is_mom(kind)) return 1;
@@ -679,7 +684,7 @@ template <int N, int KIND> static int launch_wrow_n(const PassArgs &a, hipStream
   constexpr bool CAN_SPLIT = is_mom(KIND) && N >= 256;
   const int h = KIND == NAT_TO_BLK ? a.in_h : a.H;
   const unsigned nz = (unsigned)(a.nwin > 1 ? a.nwin : 1);
-  const bool split = CAN_SPLIT && wrow_splits((long long)a.H * nz, a.planes);
+  const bool split = CAN_SPLIT && wrow_splits((long long)a.H * nz, a.planes, N, KIND == BLK_TO_MOM5);
   const int rows = (split ? wrow_waves(N, KIND, CAN_SPLIT) : wrow_waves(N, KIND, false)) * WaveFft<N>::P;
   const dim3 grid((unsigned)((h + rows - 1) / rows), is_mom(KIND) ? 1u : (unsigned)a.planes, nz);
   const dim3 block(split ? wrow_threads(N, KIND, CAN_SPLIT) : wrow_threads(N, KIND, false));

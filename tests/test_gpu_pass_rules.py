@@ -36,3 +36,15 @@ def _check(ring, p, plan, first):
 def test_moment_columns_of_2048_rows(gpu, H, W, planes, split):
     ring, p, plan = _case(H, W, 64, 6, 6 + planes, "fresnel", split_bin=split)
     assert _check(ring, p, plan, 4).shape[0] == (5 if split else 3)
+
+
+# a batch of windows has rows enough for one wave each: the sums must be those of a single window
+@pytest.mark.parametrize("H,W", [(512, 256), (512, 768), (768, 512), (768, 768)])
+@pytest.mark.parametrize("planes", [1, 2, 3, 4, 5, 7, 8])
+def test_moment_rows_do_not_depend_on_the_launch(gpu, H, W, planes):
+    for split in (0, 7) if planes > 1 else (0,):
+        ring, p, plan = _case(H, W, 32, 6, 6 + planes, "asm", frames=16, split_bin=split)
+        F = ring.shape[0]
+        batch = plan.moments_batch(ring, 2, 3)
+        for w in range(3):
+            assert torch.equal(batch[w], plan.moments(ring, (2 + 8 * w) % F)), (split, w)
