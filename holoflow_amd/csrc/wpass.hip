@@ -404,14 +404,26 @@ __global__ __launch_bounds__(wrow_threads(N, KIND, SPLIT)) void k_wrow(PassArgs 
 // measured faster than two subsets with the next plane prefetched; the four-sum kind (band
 // split) takes two (8 waves, 256 registers each), and 2048-row columns leave room for one.
 // The plane-parallel kinds take one plane per block; at 2048 rows eight waves share one twiddle
-// table (155 KB of LDS, two waves per SIMD instead of one).  Short columns as in the row pass.
+// table (155 KB of LDS, two waves per SIMD instead of one).  At 1024 rows eight waves in the
+// plane-parallel kinds, or four (NARROW) where the grid is small (wcol_narrow).  Short columns as in
+// the row pass.
 constexpr int wcol_subsets(int n, int kind) {
   return !is_mom(kind) || n >= 2048 ? 1 : n >= 256 ? (kind == BLK_TO_MOM5 ? 2 : 3) : 8;
 }
-constexpr int wcol_waves(int n, int kind) {
-  return n < 256 ? 1 : kind == BLK_TO_NAT || (n >= 1024 && !is_mom(kind)) ? 8 : 4;
+constexpr int wcol_waves(int n, int kind, bool narrow = false) {
+  return n < 256 ? 1 : kind == BLK_TO_NAT || (n >= 1024 && !is_mom(kind) && !narrow) ? 8 : 4;
 }
-constexpr int wcol_threads(int n, int kind) { return 64 * wcol_waves(n, kind) * wcol_subsets(n, kind); }
+constexpr int wcol_threads(int n, int kind, bool narrow = false) {
+  return 64 * wcol_waves(n, kind, narrow) * wcol_subsets(n, kind);
+}
+// 1024-row columns with a transfer function in `blocks4` blocks of four waves: those, while they all
+// run at once (three per CU) and leave the busiest CU fewer waves than blocks of eight would.  Eight
+// -> four: 768 x 1024 planes (W x H) with 3 planes (576 blocks) 19.4 -> 16.2 us, 512 wide with 5 (640)
+// 19.2 -> 16.5, 128 wide with 7 (224) 13.1 -> 11.8; 512 wide with 3 (384) 12.7 -> 12.9, 768 wide with 7
+// (1,344) 29.9 -> 32.8.
+constexpr bool wcol_narrow(long long blocks4, int cus) {
+  return blocks4 <= 3LL * cus && 4 * ((blocks4 + cus - 1) / cus) < 8 * ((blocks4 + 2 * cus - 1) / (2 * cus));
+}
 
 // LOOP (BLK_MID): 2048-row columns, where a block fills the CU, so that nothing else runs while it
 // starts, loads its first columns and drains: 256 blocks stay and walk the (tile, plane) items, each
@@ -424,11 +436,11 @@ constexpr int wcol_threads(int n, int kind) { return 64 * wcol_waves(n, kind) * 
 // The 2048-row moment kinds, one wave per SIMD, let their LDS accesses be paired: 52 planes of 2048^2
 // 630 -> 541 us, of 2048 x 512 303 -> 254 (the 2048-row transfer-function kind, two waves per SIMD, is
 // 3 % slower with pairs, and the shorter lengths are even or slower).
-template <int N, int KIND, bool G = false, bool PADDED = false, bool LOOP = false>
-__global__ __launch_bounds__(wcol_threads(N, KIND)) void k_wcol(PassArgs a) {
+template <int N, int KIND, bool G = false, bool PADDED = false, bool LOOP = false, bool NARROW = false>
+__global__ __launch_bounds__(wcol_threads(N, KIND, NARROW)) void k_wcol(PassArgs a) {
   using F = WaveFft<N, is_mom(KIND) && N >= 2048>;
   constexpr int E = F::E, L = F::L, P = F::P;
-  constexpr int S = wcol_subsets(N, KIND), WC = wcol_waves(N, KIND);
+  constexpr int S = wcol_subsets(N, KIND), WC = wcol_waves(N, KIND, NARROW);
   __shared__ __align__(16) float2 scr[WC * S * P * F::SCR];
   __shared__ __align__(16) float2 twl[F::TWL];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -721,7 +733,7 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
   const dim3 grid(KIND == BLK_MID ? tiles * (unsigned)a.planes : tiles,
                   is_mom(KIND) || KIND == BLK_MID ? 1u : (unsigned)a.planes, (unsigned)(a.nwin > 1 ? a.nwin : 1));
   const dim3 block(wcol_threads(N, KIND));
-  constexpr bool CAN_LOOP = KIND == BLK_MID && N >= 2048;
+  constexpr bool CAN_LOOP = KIND == BLK_MID && N >= 2048, CAN_NARROW = KIND == BLK_MID && N == 1024;
   constexpr unsigned MID_BLOCKS = 256;  // one per CU
   const bool padded = a.row1 > a.row0 && (a.row0 > 0 || a.row1 < a.H);
   if (padded && KIND != BLK_MID) return -4;
@@ -731,6 +743,9 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
     hipLaunchKernelGGL((k_wcol<N, KIND, false, KIND == BLK_MID>), grid, block, 0, st, a);
   else if (CAN_LOOP && a.W % cols == 0 && a.nwin <= 1 && grid.x >= 4 * MID_BLOCKS)
     hipLaunchKernelGGL((k_wcol<N, KIND, false, false, CAN_LOOP>), dim3(MID_BLOCKS), block, 0, st, a);
+  else if (CAN_NARROW && wcol_narrow((long long)((a.W + 3) / 4) * a.planes, 256))
+    hipLaunchKernelGGL((k_wcol<N, KIND, false, false, false, CAN_NARROW>), dim3((unsigned)((a.W + 3) / 4) * (unsigned)a.planes),
+                       dim3(wcol_threads(N, KIND, CAN_NARROW)), 0, st, a);
   else
     hipLaunchKernelGGL((k_wcol<N, KIND>), grid, block, 0, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;

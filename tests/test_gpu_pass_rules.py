@@ -31,6 +31,12 @@ def _check(ring, p, plan, first):
     return out
 
 
+# blocks of four waves: W / 4 x planes
+@pytest.mark.parametrize("W,planes", [(4, 1), (8, 5), (128, 8), (128, 9), (512, 4), (512, 5), (768, 4), (256, 13)])
+def test_transfer_function_columns_of_1024_rows(gpu, W, planes):
+    _check(*_case(1024, W, 64, 6, 6 + planes, "asm"), 5)
+
+
 @pytest.mark.parametrize("H,W,planes", [(2048, 16, 5), (2048, 24, 9)])
 @pytest.mark.parametrize("split", [0, 8])
 def test_moment_columns_of_2048_rows(gpu, H, W, planes, split):
