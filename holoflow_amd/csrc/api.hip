@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/hfx.h"
+#include "dev_arena.hh"
 #include "hfx_kernels.hh"
 
 namespace {
@@ -43,41 +44,7 @@ hfx_status fail(hfx_status code, const std::string &msg) {
 
 inline hipStream_t S(hfx_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
-// Device allocation that records itself for release.  Small tables share blocks of kBlock bytes:
-// a plan has a dozen of them.
-struct DevArena {
-  static constexpr size_t kBlock = 128 << 10, kSmall = 32 << 10;
-  std::vector<void *> ptrs;
-  size_t bytes = 0;
-  char *block = nullptr;
-  size_t used = 0;
-  template <typename T> hfx_status alloc(T **p, size_t count) {
-    size_t b = count * sizeof(T);
-    if (b == 0) b = 16;
-    const bool small = b <= kSmall;
-    const size_t padded = (b + 255) & ~(size_t)255;
-    if (small && block && used + padded <= kBlock) {
-      *p = reinterpret_cast<T *>(block + used);
-      used += padded;
-      bytes += b;
-      return HFX_OK;
-    }
-    void *v = nullptr;
-    hipError_t e = hipMalloc(&v, small ? kBlock : b);
-    if (e != hipSuccess) return fail(HFX_E_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
-    ptrs.push_back(v);
-    bytes += b;
-    if (small) {
-      block = static_cast<char *>(v);
-      used = padded;
-    }
-    *p = static_cast<T *>(v);
-    return HFX_OK;
-  }
-  ~DevArena() {
-    for (void *p : ptrs) (void)hipFree(p);
-  }
-};
+using hfx::DevArena;
 
 #define HFX_TRY(expr)              \
   do {                             \
