@@ -193,7 +193,7 @@ static hfx_status gen_prop_tables(hfx_plan *p, hipStream_t st) {
   return HFX_OK;
 }
 
-static hfx_status plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_plan **out, bool one_window) {
+hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_plan **out) {
   if (!dp || !out) return fail(HFX_E_INVALID, "null argument");
   *out = nullptr;
   const hfx_plan_desc &d = *dp;
@@ -260,21 +260,22 @@ static hfx_status plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_
   DevArena &A = p->arena;
   p->filter2d = d.prop == HFX_PROP_FRESNEL && d.filter_enabled;
   p->fused_row = p->OH == p->H && p->OW == p->W && hfx::dft_row_supported(p->W, p->nbc, d.window);
-  if (d.batch_windows > 1 && p->fused_row && !p->filter2d &&
-      hfx::dft_front_pipelined(p->W, p->nbc, d.window, p->n_planes, d.precision))
-    p->nwin = std::min<int>(d.batch_windows, 4);
-  // Windows per launch the library chooses: as many as keep the group's planes within
-  // kBatchPlaneBytes.
+  // Windows per launch the library would choose: as many as keep the group's planes within
+  // kBatchPlaneBytes.  A caller's own count above it is for the pipelined front, which runs on across
+  // the windows' rows.
   const long long window_bytes = (long long)p->n_planes * std::max(p->npix, p->onpix) * (long long)sizeof(float2);
-  if (one_window)
-    p->nwin = 1;
+  const int fit = (int)std::clamp<long long>(kBatchPlaneBytes / window_bytes, 1, hfx::HFX_MAX_WIN);
+  const bool pipelined = p->fused_row && !p->filter2d &&
+                         hfx::dft_front_pipelined(p->W, p->nbc, d.window, p->n_planes, d.precision);
+  if (d.batch_windows == 0)
+    p->nwin = fit;
   else
-    p->nwin = std::max(p->nwin, (int)std::min<long long>(kBatchPlaneBytes / window_bytes, hfx::HFX_MAX_WIN));
+    p->nwin = std::min(std::clamp(d.batch_windows, 1, 4), pipelined ? 4 : fit);
   // batch lanes: a second stream (and plane workspaces) lets one window's kernels overlap the
   // neighbouring window's (measured +15 % at 1024^2, T = 64, in FP32 and the 16-bit modes);
   // the Flatfield's scratch images and Filter2D's tables are shared, so those keep one lane.
   if (d.batch_lanes < 0 || d.batch_lanes > 2) return fail(HFX_E_INVALID, "batch_lanes must be 0, 1 or 2");
-  p->lanes = d.batch_lanes != 1 && !one_window && !p->filter2d && !d.flatfield_enabled ? 2 : 1;
+  p->lanes = d.batch_lanes != 1 && !p->filter2d && !d.flatfield_enabled ? 2 : 1;
   // natural-layout planes per window of a launch and lane: only the stand-alone time DFT needs them
   HFX_TRY(A.alloc(&p->planes_nat, p->fused_row ? 1 : (size_t)p->lanes * p->nwin * p->n_planes * p->npix));
   if (p->lanes == 2) {
@@ -323,18 +324,6 @@ static hfx_status plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_
   *out = guard.release();
   return HFX_OK;
 }
-
-hfx_status hfx_plan_create(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out) {
-  return plan_create(d, stream, out, false);
-}
-
-}  // extern "C"
-namespace hfx {
-hfx_status plan_create_one_window(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out) {
-  return plan_create(d, stream, out, true);
-}
-}  // namespace hfx
-extern "C" {
 
 hfx_status hfx_plan_destroy(hfx_plan *p) {
   delete p;

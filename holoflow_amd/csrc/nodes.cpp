@@ -38,8 +38,6 @@
 #include "holoflow/core/registry.hh"
 
 namespace hfx {
-// hfx_plan_create without the batch workspaces (api.hip): for plans that only run hfx_moments
-hfx_status plan_create_one_window(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out);
 void set_last_error(const std::string &msg);  // libhfx's thread-local last error (api.hip)
 }
 
@@ -1121,7 +1119,8 @@ hfx_plan_desc moments_desc(const Json &j, const TDesc &d) {
   p.height = (int32_t)d.shape[r - 2];
   p.width = (int32_t)d.shape[r - 1];
   p.stride = (int32_t)j.get_int("stride", p.window);
-  p.batch_lanes = 1;  // one window per execute: no second lane
+  p.batch_lanes = 1;  // one window per execute: no second lane, no multi-window workspace
+  p.batch_windows = 1;
   p.fs_hz = j.get("fs", 37e3);
   p.weight_fs_hz = j.get("weight_fs", 37e3);
   p.lambda_m = f32(j, "lambda");
@@ -1233,7 +1232,7 @@ class DopplerMomentsFactory : public ISyncTaskFactory {
     t->settings = j;
     t->idesc = in[0];
     const auto p = moments_desc(j, in[0]);
-    HFX_CHECK(hfx::plan_create_one_window(&p, hs(ctx.stream), &t->plan));
+    HFX_CHECK(hfx_plan_create(&p, hs(ctx.stream), &t->plan));
     return t;
   }
   std::unique_ptr<ISyncTask> update(std::unique_ptr<ISyncTask> old, std::span<const TDesc> in, const Json &j,

@@ -40,8 +40,6 @@
 
 namespace hfx {
 void set_last_error(const std::string &msg);  // libhfx's thread-local last error (api.hip)
-// hfx_plan_create without the batch workspaces (api.hip): hfx_moments and hfx_moments_group only
-hfx_status plan_create_one_window(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out);
 }
 
 namespace {
@@ -204,7 +202,9 @@ hfx_status build_stream(hfx_server *s, Stream &st) {
   hipStream_t cs = s->capture;
   hfx_plan_desc pd = st.d.plan;
   // windows run one at a time through hfx_moments: no second lane, no multi-window workspace
-  SRV_TRY(hfx::plan_create_one_window(&pd, cs, &st.plan));
+  pd.batch_lanes = 1;
+  pd.batch_windows = 1;
+  SRV_TRY(hfx_plan_create(&pd, cs, &st.plan));
   hfx_plan_info info{};
   SRV_TRY(hfx_plan_get_info(st.plan, &info));
   st.groupable = info.groupable != 0;

@@ -95,7 +95,7 @@ class MomentConfig:
     filt: Optional[tuple] = None           # (r_inner, r_outer, s_inner, s_outer)
     split_bin: int = 0
     flatfield: Optional[tuple] = None      # (sigma_y, sigma_x)
-    batch_windows: int = 1                 # windows per launch in moments_batch (1 = library's choice)
+    batch_windows: int = 0                 # windows per launch in moments_batch (0 = library's choice, 1 = one)
     batch_lanes: int = 0                   # streams moments_batch alternates over (0 = library default)
 
     def to_desc(self) -> _lib.PlanDesc:

@@ -80,12 +80,14 @@ typedef struct hfx_plan_desc {
   int32_t flatfield_enabled; /* Flatfield on every moment image after the fftshift
                                 (graph_builder.cc:637-641) */
   float flatfield_sigma_y, flatfield_sigma_x;
-  int32_t batch_windows;     /* hfx_moments_batch: windows per launch, at least.  0 or 1: the
+  int32_t batch_windows;     /* hfx_moments_batch: windows per launch; each takes a plane
+                                workspace per lane, held from hfx_plan_create on.  0: the
                                 library's choice (up to 32 small windows, as long as their
-                                planes stay within 64 MiB per lane; one for large frames);
-                                2..4: that many also for large frames, at the cost of one plane
-                                workspace each (FP32 Fresnel/ASM on the pipelined front, without
-                                padding or Filter2D) */
+                                planes stay within 64 MiB per lane; one for large frames).
+                                1: one, for plans whose memory counts or that never run
+                                batches.  2..4: that many, also for large frames on the
+                                pipelined front (FP32 Fresnel/ASM without padding or Filter2D),
+                                elsewhere at most the library's choice */
   int32_t batch_lanes;       /* hfx_moments_batch: HIP streams the windows alternate over, so
                                 that one window's kernels overlap the neighbouring window's
                                 (0 or 2 = two unless a Flatfield or a Fresnel Filter2D stage
