@@ -75,3 +75,33 @@ def test_reported_bytes_are_the_bytes_held(tmp_path):
     CHECK(a.alloc(&big, 1 << 20) == HFX_E_NOMEM && a.bytes == g_total && !hfx::g_err.empty());
   }
   CHECK(g_total == 0 && g_held.empty());""")
+
+
+def test_a_full_device_gets_one_window(tmp_path):
+    """The workspaces of several windows, allocated in two parts; the second does not fit: what was got
+    goes back, shared blocks among it, one window is allocated, and tables after it are sound."""
+    _run(tmp_path, r"""
+  {
+    hfx::DevArena a;
+    char *first, *tiny, *planes, *table;
+    CHECK(a.alloc(&first, 100000) == HFX_OK);
+    const size_t before = a.bytes;
+    int n = 32, calls = 0;
+    auto alloc = [&](int k) {
+      ++calls;
+      if (a.alloc(&tiny, 16) != HFX_OK) return HFX_E_NOMEM;
+      return a.alloc(&planes, (size_t)k << 20);
+    };
+    g_limit = g_total + (8 << 20);
+    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_OK && n == 1 && calls == 2);
+    CHECK(a.bytes == g_total && a.bytes == before + a.kBlock + (1 << 20) && g_last == hipSuccess);
+    CHECK(tiny == a.block && a.alloc(&table, 1000) == HFX_OK && table == a.block + 256);
+    n = 4;
+    calls = 0;
+    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_OK && n == 4 && calls == 1);  // fits
+    g_limit = g_total;
+    n = 3;
+    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_E_NOMEM && n == 1);  // not even one
+    CHECK(a.bytes == g_total);
+  }
+  CHECK(g_total == 0 && g_held.empty());""")
