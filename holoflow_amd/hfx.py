@@ -17,8 +17,12 @@ from ._lib import check, lib
 def _stream(stream) -> C.c_void_p:
     if stream is None:
         # the current stream's handle without a torch.cuda.Stream object around it: 0.5 us instead of
-        # 2.7, of the 10 to 15 that a call of this module takes on the host
-        return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        # 2.7, of the 10 to 15 that a call of this module takes on the host (not a public name: a torch
+        # without it takes the object)
+        try:
+            return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        except AttributeError:
+            stream = torch.cuda.current_stream()
     if isinstance(stream, torch.cuda.Stream):
         return C.c_void_p(stream.cuda_stream)
     return C.c_void_p(int(stream))
