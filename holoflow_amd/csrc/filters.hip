@@ -202,6 +202,7 @@ __global__ __launch_bounds__(FF_NT) void k_flatfield_spatial(const float *__rest
       ff_tap(s, v0.y, v0.z, v0.w, v1.x, w.y);
       ff_tap(s, v0.z, v0.w, v1.x, v1.y, w.z);
     }
+    __builtin_amdgcn_wave_barrier();  // in place: no lane of the row writes before all have read
     row[0] = make_float4(s[0], s[1], s[2], s[3]);
   }
   __syncthreads();
