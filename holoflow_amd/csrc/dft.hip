@@ -762,7 +762,7 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
       go(std::integral_constant<int, 128>{});
   } else if (a.n_planes <= row_group<W>()) {
     hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, false>), dim3(grid), dim3(row_threads<W>()), lds, st, a);
-  } else {
+  } else if constexpr (CAN_MULTI) {
     for (int w = 0; w < a.nwin; ++w) {  // one window per launch
       DftArgs one = a;
       one.r.first = a.firsts[w];
@@ -770,6 +770,8 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
       hipLaunchKernelGGL((k_dft_row<W, NBT, MODE, true>), dim3((unsigned)(a.H < cus ? a.H : cus)), dim3(row_threads<W>()),
                          lds, st, one);
     }
+  } else {
+    return -2;
   }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -7,10 +7,6 @@
 
 namespace hfx {
 
-struct __align__(8) c32 {
-  float x, y;
-};
-
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }

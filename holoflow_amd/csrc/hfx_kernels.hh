@@ -112,8 +112,8 @@ struct PassArgs {
   MomentArgs mom;
   const float2 *tw;         // pass-major FFT twiddles for the transform length
   int nwin;                 // windows of the launch (blockIdx.z; 0 and 1: one)
-  // windows of one plan: byte strides of in and out, element stride of the moment images
-  long long win_in, win_out, win_mom;
+  // windows of one plan (moment kinds): byte stride of the input, element stride of the images
+  long long win_in, win_mom;
   int grouped;              // windows of several plans: window blockIdx.z takes win[blockIdx.z]
   PassWin win[HFX_MAX_GROUP];
 };

@@ -122,7 +122,7 @@ template <bool G> __device__ __forceinline__ PassWin pass_window(const PassArgs 
     const long long z = blockIdx.z;
     PassWin w;
     w.in = reinterpret_cast<const char *>(a.in) + z * a.win_in;
-    w.out = reinterpret_cast<char *>(a.out) + z * a.win_out;
+    w.out = a.out;
     w.mid_tf = a.mid_tf;
 #pragma unroll
     for (int k = 0; k < 5; ++k) w.mom_out[k] = a.mom.out[k] + z * a.win_mom;
@@ -700,11 +700,13 @@ template <int N, int KIND> static int launch_wrow_n(const PassArgs &a, hipStream
   const int rows = (split ? wrow_waves(N, KIND, CAN_SPLIT) : wrow_waves(N, KIND, false)) * WaveFft<N>::P;
   const dim3 grid((unsigned)((h + rows - 1) / rows), is_mom(KIND) ? 1u : (unsigned)a.planes, nz);
   const dim3 block(split ? wrow_threads(N, KIND, CAN_SPLIT) : wrow_threads(N, KIND, false));
+  constexpr bool CAN_GROUP = is_mom(KIND) && N >= 256;  // (wave_pass_supported)
+  if (a.grouped && !CAN_GROUP) return -4;
   if constexpr (is_mom(KIND)) {
     if (a.grouped && split)
-      hipLaunchKernelGGL((k_wrow<N, KIND, true, 0, CAN_SPLIT>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((k_wrow<N, KIND, CAN_GROUP, 0, CAN_SPLIT>), grid, block, 0, st, a);
     else if (a.grouped)
-      hipLaunchKernelGGL((k_wrow<N, KIND, true>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((k_wrow<N, KIND, CAN_GROUP>), grid, block, 0, st, a);
     else if (split)
       hipLaunchKernelGGL((k_wrow<N, KIND, false, 0, CAN_SPLIT>), grid, block, 0, st, a);
     else
@@ -736,9 +738,10 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
   constexpr bool CAN_LOOP = KIND == BLK_MID && N >= 2048, CAN_NARROW = KIND == BLK_MID && N == 1024;
   constexpr unsigned MID_BLOCKS = 256;  // one per CU
   const bool padded = a.row1 > a.row0 && (a.row0 > 0 || a.row1 < a.H);
-  if (padded && KIND != BLK_MID) return -4;
+  constexpr bool CAN_GROUP = KIND != BLK_TO_NAT && N >= 256;  // (wave_pass_supported)
+  if ((padded && KIND != BLK_MID) || (a.grouped && !CAN_GROUP)) return -4;
   if (a.grouped)
-    hipLaunchKernelGGL((k_wcol<N, KIND, KIND != BLK_TO_NAT>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((k_wcol<N, KIND, CAN_GROUP>), grid, block, 0, st, a);
   else if (padded)
     hipLaunchKernelGGL((k_wcol<N, KIND, false, KIND == BLK_MID>), grid, block, 0, st, a);
   else if (CAN_LOOP && a.W % cols == 0 && a.nwin <= 1 && grid.x >= 4 * MID_BLOCKS)
