@@ -658,9 +658,8 @@ static DftArgs make_args(const DftLaunch &L) {
 // as are resident at once (the occupancy calculator's count per CU times the CUs), at most one per
 // group of four 64-pixel tiles.
 static dim3 persistent_grid(const void *kernel, size_t lds, const DftArgs &a) {
-  int dev = 0, cus = 256, per_cu = 0;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
+  int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, lds) != hipSuccess || per_cu < 1) per_cu = 1;
   const long long quads = (a.r.npix + 255) / 256, most = std::max(1LL, (long long)cus * per_cu / a.nwin);
   return dim3((unsigned)std::min(quads, most), (unsigned)a.nwin);
@@ -736,9 +735,7 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
   const size_t lds = dft_matrix_lds_bytes(NBT, MODE, a.r.T);
   // persistent grid: one workgroup per CU (the LDS footprint allows no more), each walking rows
   // blockIdx, blockIdx + grid, ... of the launch's windows
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
   const long long rows = (long long)a.H * a.nwin;
   const unsigned grid = (unsigned)(rows < cus ? rows : cus);
   const int T = a.r.T;

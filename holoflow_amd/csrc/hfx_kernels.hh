@@ -31,6 +31,14 @@ bool flatfield_spatial_fused(int rx, int ry);
 int launch_flatfield_spatial(const float *in, float *out, float *tmp, long long planes, int H, int W,
                              const float *kx, int rx, const float *ky, int ry, hipStream_t st);
 
+// compute units of the current device (256 if that cannot be told): persistent grids are sized by it
+inline int device_cus() {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return cus;
+}
+
 // ---- time DFT (dft.hip)
 constexpr int HFX_MAX_WIN = 32;   // windows of one plan per launch
 constexpr int HFX_MAX_GROUP = 4;  // windows of several plans per launch

@@ -571,9 +571,7 @@ static int launch_probe_mode(int unroll, int nt, unsigned blocks, const uint4 *i
 
 int launch_hbm_probe(int mode, const void *in, void *out, long long bytes, int blocks_per_cu, int unroll,
                      int nontemporal, unsigned *sink, hipStream_t st) {
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
   const long long n16 = bytes / 16;
   if (n16 <= 0) return 0;
   long long blocks = (long long)blocks_per_cu * cus;
@@ -591,9 +589,7 @@ int launch_hbm_probe(int mode, const void *in, void *out, long long bytes, int b
 }
 
 static int launch_copy_bytes(const uint8_t *in, uint8_t *out, long long bytes, hipStream_t st) {
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
   const long long n16 = bytes / 16;
   if (n16 > 0) {
     long long blocks = (n16 + 255) / 256;
@@ -1009,9 +1005,7 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
 }
 
 template <int DT, bool VEC, int NBF> static void launch_axis_nbf(const DftAxisArgs &a, int k0, long long cols, hipStream_t st) {
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
   // persistent: the blocks that are resident at once (their registers allow four, three and two per
   // CU for one, two and three 16-bin tiles) walk the tiles
   const long long quads = (cols + 255) / 256, most = (long long)cus * (NBF == 1 ? 4 : NBF == 2 ? 3 : 2);

@@ -25,6 +25,7 @@
 //   M2 = sum_k (f_k^2 a_k) / n, summed in ascending k within a subset with the products rounded
 //   before the sum as the reference's multiply-then-mean does; stored with the optional
 //   fftshift out[i] = in[(i + n/2) mod n] (fftshift.cu:110-145).
+#include <algorithm>
 #include <type_traits>
 
 #include "hfx_kernels.hh"
@@ -426,7 +427,7 @@ constexpr bool wcol_narrow(long long blocks4, int cus) {
 }
 
 // LOOP (BLK_MID): 2048-row columns, where a block fills the CU, so that nothing else runs while it
-// starts, loads its first columns and drains: 256 blocks stay and walk the (tile, plane) items, each
+// starts, loads its first columns and drains: one block per CU stays and walks the (tile, plane) items, each
 // loading its next column behind the inverse transform and the stores of this one.  The waves load
 // in step, since four columns share every cache line (without the barrier they drift apart and the
 // pass is slower than one item per block: 1.9 ms).  52 planes of 2048^2 with the moment pass behind
@@ -736,7 +737,11 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
                   is_mom(KIND) || KIND == BLK_MID ? 1u : (unsigned)a.planes, (unsigned)(a.nwin > 1 ? a.nwin : 1));
   const dim3 block(wcol_threads(N, KIND));
   constexpr bool CAN_LOOP = KIND == BLK_MID && N >= 2048, CAN_NARROW = KIND == BLK_MID && N == 1024;
-  constexpr unsigned MID_BLOCKS = 256;  // one per CU
+  // LOOP from five items per block on.  One item per block -> LOOP: 512 wide with 8, 16 (four per block),
+  // 20, 52 planes 49.2 -> 51.5, 98.8 -> 101, 110.2 -> 108.7, 288 -> 272 us; 2048 wide with 4 (four), 5, 12,
+  // 52 97.5 -> 98.4, 115.4 -> 113.9, 276 -> 246, 1174 -> 1045.  A multiple of eight blocks: the items are
+  // split over the XCDs.
+  const unsigned cus = CAN_LOOP || CAN_NARROW ? (unsigned)device_cus() : 0, loop_blocks = std::max(8u, cus & ~7u);
   const bool padded = a.row1 > a.row0 && (a.row0 > 0 || a.row1 < a.H);
   constexpr bool CAN_GROUP = KIND != BLK_TO_NAT && N >= 256;  // (wave_pass_supported)
   if ((padded && KIND != BLK_MID) || (a.grouped && !CAN_GROUP)) return -4;
@@ -744,9 +749,9 @@ template <int N, int KIND> static int launch_wcol_n(const PassArgs &a, hipStream
     hipLaunchKernelGGL((k_wcol<N, KIND, CAN_GROUP>), grid, block, 0, st, a);
   else if (padded)
     hipLaunchKernelGGL((k_wcol<N, KIND, false, KIND == BLK_MID>), grid, block, 0, st, a);
-  else if (CAN_LOOP && a.W % cols == 0 && a.nwin <= 1 && grid.x >= 4 * MID_BLOCKS)
-    hipLaunchKernelGGL((k_wcol<N, KIND, false, false, CAN_LOOP>), dim3(MID_BLOCKS), block, 0, st, a);
-  else if (CAN_NARROW && wcol_narrow((long long)((a.W + 3) / 4) * a.planes, 256))
+  else if (CAN_LOOP && a.W % cols == 0 && a.nwin <= 1 && grid.x >= 5 * loop_blocks)
+    hipLaunchKernelGGL((k_wcol<N, KIND, false, false, CAN_LOOP>), dim3(loop_blocks), block, 0, st, a);
+  else if (CAN_NARROW && wcol_narrow((long long)((a.W + 3) / 4) * a.planes, (int)cus))
     hipLaunchKernelGGL((k_wcol<N, KIND, false, false, false, CAN_NARROW>), dim3((unsigned)((a.W + 3) / 4) * (unsigned)a.planes),
                        dim3(wcol_threads(N, KIND, CAN_NARROW)), 0, st, a);
   else

@@ -44,6 +44,14 @@ def test_moment_columns_of_2048_rows(gpu, H, W, planes, split):
     assert _check(ring, p, plan, 4).shape[0] == (5 if split else 3)
 
 
+# items (W / 8 x planes) around five per CU, where the blocks start to stay
+@pytest.mark.parametrize("W,planes", [(1024, 9), (1024, 10), (1024, 11), (512, 21)])
+def test_transfer_function_columns_of_2048_rows(gpu, W, planes):
+    ring, p, plan = _case(2048, W, 64, 1, 1 + planes, "asm", frames=16)
+    out = _check(ring, p, plan, 2)
+    assert torch.equal(plan.moments_batch(ring, 2, 2)[0], out)
+
+
 # a batch of windows has rows enough for one wave each: the sums must be those of a single window
 @pytest.mark.parametrize("H,W", [(512, 256), (512, 768), (768, 512), (768, 768)])
 @pytest.mark.parametrize("planes", [1, 2, 3, 4, 5, 7, 8])
