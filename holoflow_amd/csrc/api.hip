@@ -193,10 +193,7 @@ static hfx_status gen_prop_tables(hfx_plan *p, hipStream_t st) {
   return HFX_OK;
 }
 
-hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_plan **out) {
-  if (!dp || !out) return fail(HFX_E_INVALID, "null argument");
-  *out = nullptr;
-  const hfx_plan_desc &d = *dp;
+static hfx_status plan_create(const hfx_plan_desc &d, hfx_stream_t stream, hfx_plan **out) {
   if (d.height <= 0 || d.width <= 0) return fail(HFX_E_INVALID, "frame size must be positive");
   if (d.window <= 0 || d.stride <= 0) return fail(HFX_E_INVALID, "window and stride must be positive");
   if (d.window % 4 != 0) return fail(HFX_E_UNSUPPORTED, "window must be a multiple of 4");
@@ -276,11 +273,16 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
   // the Flatfield's scratch images and Filter2D's tables are shared, so those keep one lane.
   if (d.batch_lanes < 0 || d.batch_lanes > 2) return fail(HFX_E_INVALID, "batch_lanes must be 0, 1 or 2");
   p->lanes = d.batch_lanes != 1 && !p->filter2d && !d.flatfield_enabled ? 2 : 1;
+  // natural-layout planes per window of a launch and lane: only the stand-alone time DFT needs them
+  const size_t sets = (size_t)p->lanes * p->nwin * p->n_planes;
+  HFX_TRY(A.alloc(&p->planes_nat, p->fused_row ? 1 : sets * p->npix));
   if (p->lanes == 2) {
     HFX_TRY_HIP(hipStreamCreateWithFlags(&p->aux, hipStreamNonBlocking));
     HFX_TRY_HIP(hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming));
     HFX_TRY_HIP(hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming));
   }
+  // one blocked plane workspace per window of a launch, per lane
+  HFX_TRY(A.alloc(&p->planes_blk, sets * p->onpix));
   HFX_TRY(A.alloc(&p->tw_w, p->OW));
   HFX_TRY(A.alloc(&p->tw_h, p->OH));
   HFX_TRY(A.alloc(&p->wm32, (size_t)p->wm_rows * d.window));
@@ -307,21 +309,10 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
                                (int)d.s_outer, 1, p->blk_c, st);
   }
   if (d.flatfield_enabled) {
+    HFX_TRY(A.alloc(&p->mom_tmp, (size_t)p->nwin * p->n_out * p->onpix));
     HFX_TRY(hfx_flatfield_create(p->n_out, p->OH, p->OW, d.flatfield_sigma_y, d.flatfield_sigma_x, stream, &p->ff,
                                  nullptr));
   }
-  // Workspaces per window of a launch: the blocked planes and, for the stand-alone time DFT, the
-  // natural ones (both per lane), and the images that the Flatfield reads.
-  auto workspaces = [&](int nwin) -> hfx_status {
-    const size_t sets = (size_t)p->lanes * nwin * p->n_planes;
-    HFX_TRY(A.alloc(&p->planes_nat, p->fused_row ? 1 : sets * p->npix));
-    HFX_TRY(A.alloc(&p->planes_blk, sets * p->onpix));
-    if (d.flatfield_enabled) HFX_TRY(A.alloc(&p->mom_tmp, (size_t)nwin * p->n_out * p->onpix));
-    return HFX_OK;
-  };
-  // (last, so that the tables have their room: a device too full for the windows that the library
-  // chose holds one, and the plan is made all the same)
-  HFX_TRY(d.batch_windows == 0 ? hfx::alloc_or_one(A, p->nwin, workspaces) : workspaces(p->nwin));
   std::vector<float> f, f2;
   double fs_w = d.weight_fs_hz > 0 ? d.weight_fs_hz : d.fs_hz;
   build_weights(d.bin_begin, d.bin_end, d.window, fs_w, both, f, f2);
@@ -330,6 +321,12 @@ hfx_status hfx_plan_create(const hfx_plan_desc *dp, hfx_stream_t stream, hfx_pla
   HFX_TRY_HIP(hipStreamSynchronize(st));
   *out = guard.release();
   return HFX_OK;
+}
+
+hfx_status hfx_plan_create(const hfx_plan_desc *d, hfx_stream_t stream, hfx_plan **out) {
+  if (!d || !out) return fail(HFX_E_INVALID, "null argument");
+  *out = nullptr;
+  return hfx::create_or_one_window(*d, [&](const hfx_plan_desc &x) { return plan_create(x, stream, out); });
 }
 
 hfx_status hfx_plan_destroy(hfx_plan *p) {

@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
-#include <utility>
 #include <vector>
 
 #include "../../include/hfx.h"
@@ -16,7 +15,7 @@ void set_last_error(const std::string &msg);
 // Small tables share blocks of kBlock bytes: a plan has a dozen of them.
 struct DevArena {
   static constexpr size_t kBlock = 128 << 10, kSmall = 32 << 10;
-  std::vector<std::pair<void *, size_t>> ptrs;  // with their sizes
+  std::vector<void *> ptrs;
   size_t bytes = 0;  // device memory held: whole blocks, whatever is used of them
   char *block = nullptr;
   size_t used = 0;
@@ -25,7 +24,7 @@ struct DevArena {
   DevArena(const DevArena &) = delete;
   DevArena &operator=(const DevArena &) = delete;
   ~DevArena() {
-    release_to(0);
+    for (void *p : ptrs) (void)hipFree(p);
   }
 
   template <typename T> hfx_status alloc(T **p, size_t count) {
@@ -44,7 +43,7 @@ struct DevArena {
       set_last_error("hipMalloc of " + std::to_string(held) + " bytes failed");
       return HFX_E_NOMEM;
     }
-    ptrs.emplace_back(v, held);
+    ptrs.push_back(v);
     bytes += held;
     if (small) {
       block = static_cast<char *>(v);
@@ -53,28 +52,16 @@ struct DevArena {
     *p = static_cast<T *>(v);
     return HFX_OK;
   }
-
-  // Gives back all but the first n allocations.
-  void release_to(size_t n) {
-    for (; ptrs.size() > n; ptrs.pop_back()) {
-      if (ptrs.back().first == block) block = nullptr;
-      bytes -= ptrs.back().second;
-      (void)hipFree(ptrs.back().first);
-    }
-  }
 };
 
-// Runs alloc(n) (allocations from `a`); where the device has no room for them, gives back what it got
-// and runs alloc(1), with n = 1 from then on.
-template <typename F> hfx_status alloc_or_one(DevArena &a, int &n, F alloc) {
-  const size_t mark = a.ptrs.size();
-  hfx_status rc = alloc(n);
-  if (rc == HFX_E_NOMEM && n > 1) {
-    a.release_to(mark);
-    n = 1;
-    rc = alloc(n);
-  }
-  return rc;
+// Makes a plan by create(d); where the device has no room for the windows per launch that the library
+// would choose (batch_windows 0), for one.
+template <typename F> hfx_status create_or_one_window(const hfx_plan_desc &d, F create) {
+  const hfx_status rc = create(d);
+  if (rc != HFX_E_NOMEM || d.batch_windows != 0) return rc;
+  hfx_plan_desc one = d;
+  one.batch_windows = 1;
+  return create(one);
 }
 
 }  // namespace hfx

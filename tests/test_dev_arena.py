@@ -78,30 +78,29 @@ def test_reported_bytes_are_the_bytes_held(tmp_path):
 
 
 def test_a_full_device_gets_one_window(tmp_path):
-    """The workspaces of several windows, allocated in two parts; the second does not fit: what was got
-    goes back, shared blocks among it, one window is allocated, and tables after it are sound."""
+    """Creation where the library's windows do not fit, and where not even one does; a caller's own
+    count and other failures stand."""
     _run(tmp_path, r"""
-  {
+  int calls = 0;
+  auto create = [&](const hfx_plan_desc &d) -> hfx_status {
+    ++calls;
     hfx::DevArena a;
-    char *first, *tiny, *planes, *table;
-    CHECK(a.alloc(&first, 100000) == HFX_OK);
-    const size_t before = a.bytes;
-    int n = 32, calls = 0;
-    auto alloc = [&](int k) {
-      ++calls;
-      if (a.alloc(&tiny, 16) != HFX_OK) return HFX_E_NOMEM;
-      return a.alloc(&planes, (size_t)k << 20);
-    };
-    g_limit = g_total + (8 << 20);
-    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_OK && n == 1 && calls == 2);
-    CHECK(a.bytes == g_total && a.bytes == before + a.kBlock + (1 << 20) && g_last == hipSuccess);
-    CHECK(tiny == a.block && a.alloc(&table, 1000) == HFX_OK && table == a.block + 256);
-    n = 4;
-    calls = 0;
-    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_OK && n == 4 && calls == 1);  // fits
-    g_limit = g_total;
-    n = 3;
-    CHECK(hfx::alloc_or_one(a, n, alloc) == HFX_E_NOMEM && n == 1);  // not even one
-    CHECK(a.bytes == g_total);
-  }
+    char *tiny, *planes;
+    hfx_status rc = a.alloc(&tiny, 16);
+    if (rc == HFX_OK) rc = a.alloc(&planes, (size_t)(d.batch_windows ? d.batch_windows : 32) << 20);
+    return rc != HFX_OK ? rc : d.height > 0 ? HFX_OK : HFX_E_INVALID;
+  };
+  hfx_plan_desc d{};
+  d.height = 8;
+  g_limit = 8 << 20;
+  CHECK(hfx::create_or_one_window(d, create) == HFX_OK && calls == 2 && g_last == hipSuccess);
+  d.batch_windows = 9;
+  CHECK(hfx::create_or_one_window(d, create) == HFX_E_NOMEM && calls == 3);
+  d.batch_windows = 0;
+  g_limit = 1 << 20;
+  CHECK(hfx::create_or_one_window(d, create) == HFX_E_NOMEM && calls == 5);
+  g_limit = 1 << 30;
+  CHECK(hfx::create_or_one_window(d, create) == HFX_OK && calls == 6);
+  d.height = 0;
+  CHECK(hfx::create_or_one_window(d, create) == HFX_E_INVALID && calls == 7);
   CHECK(g_total == 0 && g_held.empty());""")
