@@ -805,7 +805,8 @@ template <int DT> __global__ __launch_bounds__(256) void k_dft_axis_short(DftAxi
 // replaces (direct sums on the VALU, 16 bins per pass over the input) took 570 us there.
 //
 // Lanes whose pair or column does not exist get zero samples, not zero weights, so that an
-// infinity elsewhere in the column is not turned into a NaN.
+// infinity elsewhere in the column is not turned into a NaN.  The sums and differences of pairs overflow for
+// samples beyond half the float range, as the first butterflies of an FFT do.
 //
 // DT: 1 U16, 2 F32, 3 CF32.  VEC: the four columns of a lane are adjacent in memory and aligned.
 constexpr int DFT_MAXN = 4096;
