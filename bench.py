@@ -553,11 +553,11 @@ def main():
         # The bound on any time-DFT speedup: the same batch with the time DFT (its frame loads and
         # MFMAs) taken out of the fused front kernels, measured with a timing-only build of the
         # current kernels (means of two runs, same GPU and workload): FP32 pipelined front
-        # 9,080 -> 12,724, the 16-bit fused fronts 10,015 -> 14,442 moment frames/s.  A 16-bit DFT
-        # that cost nothing at all, frame loads included, would reach 14,442 / 9,080 = 1.59x the
+        # 9,863 -> 14,859, the 16-bit fused fronts 10,989 -> 15,784 moment frames/s.  A 16-bit DFT
+        # that cost nothing at all, frame loads included, would reach 15,784 / 9,863 = 1.60x the
         # FP32 path.
-        mixed["ceiling_if_time_dft_free"] = {"fp32_batch_without_dft": 12724, "16bit_batch_without_dft": 14442,
-                                             "fp32_batch_same_run": 9080, "max_speedup_vs_fp32": 1.59,
+        mixed["ceiling_if_time_dft_free"] = {"fp32_batch_without_dft": 14859, "16bit_batch_without_dft": 15784,
+                                             "fp32_batch_same_run": 9863, "max_speedup_vs_fp32": 1.60,
                                              "source": "design measurement (fused fronts built without the time DFT)"}
 
     del out
