@@ -805,8 +805,9 @@ template <int DT> __global__ __launch_bounds__(256) void k_dft_axis_short(DftAxi
 // replaces (direct sums on the VALU, 16 bins per pass over the input) took 570 us there.
 //
 // Lanes whose pair or column does not exist get zero samples, not zero weights, so that an
-// infinity elsewhere in the column is not turned into a NaN.  The sums and differences of pairs overflow for
-// samples beyond half the float range, as the first butterflies of an FFT do.
+// infinity elsewhere in the column is not turned into a NaN.  Floating samples are halved on the way into
+// the pairs and the results scaled by two more (exact), so that the pairs of samples beyond half the
+// float range stay finite.
 //
 // DT: 1 U16, 2 F32, 3 CF32.  VEC: the four columns of a lane are adjacent in memory and aligned.
 constexpr int DFT_MAXN = 4096;
@@ -886,6 +887,8 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
   using X = DftColumns<DT, VEC>;
   constexpr int NF = X::NF;
   constexpr int K = DT == 3 ? 2 : 4;  // pair steps in flight
+  constexpr float HALF = DT == 1 ? 1.f : 0.5f;
+  const float scale = a.scale * (1.f / HALF);
   const int n = a.n, pairs = (n - 1) / 2, steps = (pairs + 3) / 4;
   const int lane = threadIdx.x & 63, g = lane >> 4, rw = lane & 15;
   const long long tiles = (cols + 63) / 64;
@@ -920,8 +923,9 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
       float sm[NF], df[NF];
 #pragma unroll
       for (int t = 0; t < NF; ++t) {
-        sm[t] = in ? x1[t] + x2[t] : 0.f;
-        df[t] = in ? x1[t] - x2[t] : 0.f;
+        const float h = HALF * x1[t];
+        sm[t] = in ? fmaf(HALF, x2[t], h) : 0.f;
+        df[t] = in ? fmaf(-HALF, x2[t], h) : 0.f;
       }
 #pragma unroll
       for (int f = 0; f < NBF; ++f) {
@@ -959,7 +963,7 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
     X::unpack(xe, xv);
     const bool in = g == 0 || (g == 1 && n % 2 == 0);
 #pragma unroll
-    for (int t = 0; t < NF; ++t) xv[t] = in ? xv[t] : 0.f;
+    for (int t = 0; t < NF; ++t) xv[t] = in ? HALF * xv[t] : 0.f;
 #pragma unroll
     for (int f = 0; f < NBF; ++f) {
       const float w = g == 1 && ((k0 + 16 * f + rw) & 1) ? -1.f : 1.f;
@@ -984,7 +988,7 @@ __global__ __launch_bounds__(256, 2) void k_dft_axis_mfma(DftAxisArgs a, int k0,
         if (k >= a.ke) continue;
         float2 v[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = make_float2(re[f][t][q] * a.scale, im[f][t][q] * a.scale);
+        for (int t = 0; t < 4; ++t) v[t] = make_float2(re[f][t][q] * scale, im[f][t][q] * scale);
         if constexpr (VEC) {
           const long long o = c0 / a.inner, i = c0 - o * a.inner;
           float4 *dst = reinterpret_cast<float4 *>(a.out + (o * nk + (k - a.kb)) * a.inner + i);

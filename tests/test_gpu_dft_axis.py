@@ -60,3 +60,23 @@ def test_dft_axis_infinite_sample_stays_in_its_column(gpu, kind, n, j):
     keep = torch.arange(70) != 17
     assert torch.equal(torch.view_as_real(got[:, keep]), torch.view_as_real(ref[:, keep]))
     assert not torch.isfinite(torch.view_as_real(got[:, 17])).all(dim=-1).any()
+
+
+@pytest.mark.parametrize("kind", ["f32", "cf32"])
+@pytest.mark.parametrize("n", [9, 12, 13, 33, 64, 127])
+def test_dft_axis_samples_near_the_largest_float(gpu, kind, n):
+    """Two samples of a folded pair whose sum or difference is beyond the float range, in results that
+    are not: each product and sum rounds by half an ulp of at most sqrt(2) |x|, as does each twiddle."""
+    from holoflow_amd import hfx
+
+    big = 3.0e38
+    x = torch.zeros((n, 6), dtype=torch.complex64 if kind == "cf32" else torch.float32)
+    for c, (p, q, a, b) in enumerate([(1, n - 1, 1, 1), (1, n - 1, 1, -1), (2, n - 2, -1, -1), (n // 2, n - n // 2, 1, 1),
+                                      (4, n - 4, 1, 1), (4, n - 4, -1, 1)]):
+        x[p, c], x[q, c] = a * big, b * big
+        if kind == "cf32":
+            x[p, c] *= 1j
+    got = hfx.dft_axis(x.cuda(), 0, scale=0.25).cpu().to(torch.complex128)
+    ref = torch.fft.fft(x.to(torch.complex128), dim=0) * 0.25
+    assert bool(torch.isfinite(torch.view_as_real(got)).all())
+    assert bool(((got - ref).abs() <= 6 * 2.0**-23 * 0.25 * 2 * big).all())
