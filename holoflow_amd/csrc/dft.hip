@@ -420,20 +420,45 @@ __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
 // and eight at 1024, 768 and 512; up to 8 bins, eight at 512 (four windows of 512^2, T = 32: 92 ->
 // 87 us) and four beyond, where eight measured 3-5 % slower.
 template <int W> constexpr int front_pw() { return W / 128; }
-template <int W, bool FOLD> constexpr int front_cw() { return W == 512 ? 8 : FOLD ? 12 - front_pw<W>() : 4; }
-template <int W, int NBT> constexpr int front_threads() { return (front_pw<W>() + front_cw<W, NBT == 2>()) * 64; }
+template <int W, bool FOLD, bool FEW> constexpr int front_cw() {
+  return FEW ? 4 : W == 512 ? 8 : FOLD ? 12 - front_pw<W>() : 4;
+}
+template <int W, int NBT, bool FEW> constexpr int front_threads() { return (front_pw<W>() + front_cw<W, NBT == 2, FEW>()) * 64; }
+// k_front: whether the row FFTs' waves issue first.  They are the longer half of a row at 9..16 bins
+// (front alone 84.6 -> 75.5 us at 1024^2, T = 64, 15 planes; at up to 8 bins 3 % slower), but a cache
+// line of the planes holds four rows, and blocks that run ahead leave it before their neighbours have
+// filled it: with T = 32, where the DFT holds them back least, tall frames lose (rows x width, 15
+// planes, without -> with: 1024 x 512 33.5 -> 39.7, 1024 x 768 49.1 -> 70.5, 1024^2 54.4 -> 79.8) and only
+// short ones gain (512 x 768, 9 planes 24.3 -> 23.0).  Several groups of planes per row hold them back
+// too: 1024^2, T = 32, 24 planes 113 -> 92.  With T = 128 the DFT is as long as the FFTs and rows shorter
+// than 1024 points lose: 2048 x 512, 15 planes 109 -> 115, 1024 x 768 90 -> 94 (1024^2 121 -> 104).
+constexpr bool front_fft_first(int W, bool fold, int T, bool multi, bool tall) {
+  if (!fold) return false;
+  if (W == 1024) return T > 32 || multi || !tall;
+  if (W == 768) return T == 64 || (T == 32 && !multi && !tall);
+  return T == 64 && !tall;
+}
+// 512-point rows of tall frames at T = 64: four consumer waves keep the blocks together (1024 rows,
+// windows with 15 planes 70.3 -> 68.0 us, 30 planes 112.5 -> 108.0; batches of 2048 rows with 30 planes 2,035 ->
+// 1,873; frames of 512 rows with an angular spectrum 51.0 with eight and priority, 54.1 with four).
+constexpr bool front_few(int W, bool fold, int T, bool tall) { return W == 512 && fold && T == 64 && tall; }
+// where frames of 1024 rows and more take a form of their own
+constexpr bool front_has_tall(int W, bool fold, int T) {
+  return front_few(W, fold, T, true) || front_fft_first(W, fold, T, false, true) != front_fft_first(W, fold, T, false, false);
+}
 constexpr int front_ring(int T) { return T / 4 < 8 ? T / 4 : 8; }
 
 // MULTI: the planes take several LDS groups (two-sided bands).  The producers keep a row's spectra
 // and scatter one group after the other, each as soon as the consumers are done with the previous
 // one; the next row's DFT overlaps the last group's row FFTs.
-template <int W, int NBT, int MODE, int T, bool MULTI = false>
-__global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) {
+template <int W, int NBT, int MODE, int T, bool MULTI = false, bool TALL = false>
+__global__ __launch_bounds__((front_threads<W, NBT, front_few(W, NBT == 2, T, TALL)>())) void k_front(DftArgs a) {
+  constexpr bool FEW = front_few(W, NBT == 2, T, TALL);
   static_assert(MODE == 0, "the pipelined front kernel runs the FP32 time DFT");
   using F = WaveFft<W>;
   constexpr int TPW = 2;
   constexpr int NPW = front_pw<W>();
-  constexpr int NT = (front_threads<W, NBT>());
+  constexpr int NT = (front_threads<W, NBT, FEW>());
   constexpr int E = F::E;
   constexpr int GB = row_group<W>();
   __shared__ float2 scr[GB * F::SCR];  // one padded row per plane
@@ -562,7 +587,7 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
     float2 *planes = a.grouped ? a.planes_w[win_of(i)] : a.planes + win_of(i) * a.planes_stride;
     const long long row_off = blk_lane_offset(lane, a.H, a.blk_c) + (long long)y * a.blk_c;
     const int q1 = MULTI ? min(q0 + gp, a.n_planes) : a.n_planes;
-    for (int q = q0 + rw; q < q1; q += front_cw<W, FOLD>()) {
+    for (int q = q0 + rw; q < q1; q += front_cw<W, FOLD, FEW>()) {
       float2 *ws = scr + (q - q0) * F::SCR;
       float2 v[E];
 #pragma unroll
@@ -602,11 +627,7 @@ __global__ __launch_bounds__((front_threads<W, NBT>())) void k_front(DftArgs a) 
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last row's unused refills land first
   } else {
-    // the row FFTs are the longer half of a row at 9..16 bins: their waves issue first (front alone
-    // 84.6 -> 75.5 us at 1024^2, T = 64, 15 planes; at up to 8 bins it measured 3 % slower).  At T = 128
-    // the DFT is as long, and rows shorter than 1024 points lose: 2048 x 512, 15 planes 109 -> 115 us,
-    // 1024 x 768 90 -> 94 (1024^2 121 -> 104)
-    if constexpr (FOLD && (W == 1024 || T < 128)) __builtin_amdgcn_s_setprio(3);
+    if constexpr (front_fft_first(W, FOLD, T, MULTI, TALL)) __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       for (int g = 0; g < ng; ++g) {
@@ -743,13 +764,16 @@ template <int W, int NBT, int MODE> static int launch_row(const DftArgs &a, hipS
   constexpr bool CAN_MULTI = NBT == 2 && W > 512;
   const bool multi = a.n_planes > row_group<W>();
   if (MODE == 0 && (CAN_MULTI || !multi) && (T == 32 || T == 64 || T == 128)) {
-    const dim3 g(grid), b((front_threads<W, NBT>()));
+    const dim3 g(grid);
     auto go = [&](auto t) {
       constexpr int TT = decltype(t)::value;
+      constexpr bool CAN_TALL = front_has_tall(W, NBT == 2, TT), FEW = front_few(W, NBT == 2, TT, CAN_TALL);
       if (multi)
-        hipLaunchKernelGGL((k_front<W, NBT, 0, TT, CAN_MULTI>), g, b, lds, st, a);
+        hipLaunchKernelGGL((k_front<W, NBT, 0, TT, CAN_MULTI>), g, dim3(front_threads<W, NBT, false>()), lds, st, a);
+      else if (CAN_TALL && a.H >= 1024)
+        hipLaunchKernelGGL((k_front<W, NBT, 0, TT, false, CAN_TALL>), g, dim3(front_threads<W, NBT, FEW>()), lds, st, a);
       else
-        hipLaunchKernelGGL((k_front<W, NBT, 0, TT>), g, b, lds, st, a);
+        hipLaunchKernelGGL((k_front<W, NBT, 0, TT>), g, dim3(front_threads<W, NBT, false>()), lds, st, a);
     };
     if (T == 32)
       go(std::integral_constant<int, 32>{});

@@ -62,3 +62,20 @@ def test_moment_rows_do_not_depend_on_the_launch(gpu, H, W, planes):
         batch = plan.moments_batch(ring, 2, 3)
         for w in range(3):
             assert torch.equal(batch[w], plan.moments(ring, (2 + 8 * w) % F)), (split, w)
+
+
+# 512-point rows at T = 64: four consumer waves from 1024 rows on, eight below; the folded and the
+# interleaved DFT, one band and two
+@pytest.mark.parametrize("H", [768, 1024, 2048])
+@pytest.mark.parametrize("kb,ke,both", [(8, 15, False), (8, 17, False), (8, 24, False), (8, 23, True)])
+def test_front_of_512_point_rows(gpu, H, kb, ke, both):
+    from holoflow_amd import hfx
+
+    g = torch.Generator(device="cuda").manual_seed(H + ke)
+    ring = torch.randint(0, 4096, (64 + 35, H, 512), dtype=torch.int16, device="cuda", generator=g)
+    p = O.PathParams(H, 512, 64, 16, kb, ke, "fresnel", 852e-9, 12e-6, 12e-6, 0.4, fftshift=True, both_sidebands=both)
+    plan = hfx.MomentPlan(hfx.MomentConfig(H, 512, 64, 16, kb, ke, "fresnel", p.lambda_m, p.dx_m, p.dy_m, p.z_m, fftshift=True,
+                                           both_sidebands=both, batch_windows=2))
+    out = _check(ring, p, plan, 5)
+    batch = plan.moments_batch(ring, 5, 2)
+    assert torch.equal(batch[0], out) and torch.equal(batch[1], plan.moments(ring, 21))
