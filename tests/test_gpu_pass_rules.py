@@ -79,3 +79,14 @@ def test_front_of_512_point_rows(gpu, H, kb, ke, both):
     out = _check(ring, p, plan, 5)
     batch = plan.moments_batch(ring, 5, 2)
     assert torch.equal(batch[0], out) and torch.equal(batch[1], plan.moments(ring, 21))
+
+
+# 768- and 1024-point rows at T = 32: frames of 1024 rows and more take a form of their own
+@pytest.mark.parametrize("H", [768, 1024, 2048])
+@pytest.mark.parametrize("W", [768, 1024])
+@pytest.mark.parametrize("kb,ke", [(1, 10), (1, 17)])
+def test_front_of_short_windows(gpu, H, W, kb, ke):
+    ring, p, plan = _case(H, W, 32, kb, ke, "fresnel", frames=8, batch_windows=2)
+    out = _check(ring, p, plan, 5)
+    batch = plan.moments_batch(ring, 5, 2)
+    assert torch.equal(batch[0], out) and torch.equal(batch[1], plan.moments(ring, 13))
