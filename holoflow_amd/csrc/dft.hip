@@ -113,13 +113,15 @@ __device__ __forceinline__ void dft_store_bin(float2 *planes, long long npix, co
   }
 }
 
-// All arguments that a stand-alone kernel reads, asked for in one go at its start: kernel arguments lie
-// in host memory, and the compiler else loads each where it is first used, one round trip after the
-// other (time DFT of a 64 x 64 window, T = 32: 5.3 us so, 4.9 here).
-__device__ __forceinline__ void load_args(const DftArgs &a) {
+// All arguments that a kernel reads, asked for in one go at its start: kernel arguments lie in host
+// memory, and the compiler else loads each where it is first used, one round trip after the other
+// (time DFT of a 64 x 64 window, T = 32: 5.3 us so, 4.9 here; front of 256 x 512, T = 32, 7 planes 9.0 and 8.5).
+template <bool FUSED = false> __device__ __forceinline__ void load_args(const DftArgs &a) {
   asm volatile("" ::"s"(a.r.ring), "s"(a.r.ring_frames), "s"(a.r.first), "s"(a.r.npix), "s"(a.r.T), "s"(a.kb), "s"(a.nb),
                "s"(a.nbc), "s"(a.both), "s"(a.W), "s"(a.nwin), "s"(a.planes), "s"(a.planes_stride), "s"(a.wm_hi),
                "s"(a.wm_lo), "s"(a.lx), "s"(a.ly));
+  if constexpr (FUSED)
+    asm volatile("" ::"s"(a.tw), "s"(a.H), "s"(a.blk_c), "s"(a.n_planes), "s"(a.grouped), "s"(gridDim.x));
 }
 
 // Window of item i where each window has `per` items (no division in the first window, which is all
@@ -261,6 +263,7 @@ template <int W> constexpr int row_threads() { return W / row_tpw<W>(); }
 // separate instantiation so the common single-group kernel carries no spill code.
 template <int W, int NBT, int MODE, bool MULTI>
 __global__ __launch_bounds__(row_threads<W>()) void k_dft_row(DftArgs a) {
+  load_args<true>(a);
   using F = WaveFft<W>;
   constexpr int TPW = row_tpw<W>();
   constexpr int NT = row_threads<W>();
@@ -455,6 +458,7 @@ template <int W, int NBT, int MODE, int T, bool MULTI = false, bool TALL = false
 __global__ __launch_bounds__((front_threads<W, NBT, front_few(W, NBT == 2, T, TALL)>())) void k_front(DftArgs a) {
   constexpr bool FEW = front_few(W, NBT == 2, T, TALL);
   static_assert(MODE == 0, "the pipelined front kernel runs the FP32 time DFT");
+  load_args<true>(a);
   using F = WaveFft<W>;
   constexpr int TPW = 2;
   constexpr int NPW = front_pw<W>();
@@ -631,6 +635,11 @@ __global__ __launch_bounds__((front_threads<W, NBT, front_few(W, NBT == 2, T, TA
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       for (int g = 0; g < ng; ++g) {
+        // The row FFTs are 4- and 8-byte instructions without a loop among them, and how they fall on
+        // the instruction fetch counts: from 4 bytes past a 64-byte line on, 1024^2, T = 64, 15 planes
+        // take 75 us; with the whole kernel moved by 0 to 16 dwords, 75 wherever this lands on an odd
+        // one and 79-84 on an even one.  The place is pinned, so that nothing ahead of it moves it.
+        asm volatile(".p2align 6\n\ts_nop 0");
         // opaque lane index: keeps loop-invariant LDS addresses out of registers
         int lane;
         asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
