@@ -449,6 +449,13 @@ constexpr bool front_few(int W, bool fold, int T, bool tall) { return W == 512 &
 constexpr bool front_has_tall(int W, bool fold, int T) {
   return front_few(W, fold, T, true) || front_fft_first(W, fold, T, false, true) != front_fft_first(W, fold, T, false, false);
 }
+// Whether the row FFTs' code of k_front starts on an odd dword.  It is 4- and 8-byte instructions without a
+// loop among them, and how they fall on the instruction fetch counts: 1024^2, T = 64, 15 planes take 75 us
+// wherever it lands on an odd dword and 79-86 on an even one (the whole kernel moved by 0 to 16 dwords);
+// 512-point rows with T = 128 are better on an even one (1024 rows, 30 planes 85 against 89 us), several
+// groups of planes with T = 32 too (1024^2, 30 planes 112 against 118), the others differ by less than
+// 2 %.  The place is pinned against a 64-byte line, so that nothing ahead of it in the kernel moves it.
+constexpr bool front_odd(int W, int T, bool multi) { return !(W == 512 && T == 128) && !(multi && T == 32); }
 constexpr int front_ring(int T) { return T / 4 < 8 ? T / 4 : 8; }
 
 // MULTI: the planes take several LDS groups (two-sided bands).  The producers keep a row's spectra
@@ -635,11 +642,11 @@ __global__ __launch_bounds__((front_threads<W, NBT, front_few(W, NBT == 2, T, TA
     __syncthreads();
     for (int i = 0; i < nr; ++i) {
       for (int g = 0; g < ng; ++g) {
-        // The row FFTs are 4- and 8-byte instructions without a loop among them, and how they fall on
-        // the instruction fetch counts: from 4 bytes past a 64-byte line on, 1024^2, T = 64, 15 planes
-        // take 75 us; with the whole kernel moved by 0 to 16 dwords, 75 wherever this lands on an odd
-        // one and 79-84 on an even one.  The place is pinned, so that nothing ahead of it moves it.
-        asm volatile(".p2align 6\n\ts_nop 0");
+        // the place of the row FFTs' code, pinned (front_odd)
+        if constexpr (front_odd(W, T, MULTI))
+          asm volatile(".p2align 6\n\ts_nop 0");
+        else
+          asm volatile(".p2align 6");
         // opaque lane index: keeps loop-invariant LDS addresses out of registers
         int lane;
         asm volatile("v_mov_b32 %0, %1" : "=v"(lane) : "v"(tid & 63));
